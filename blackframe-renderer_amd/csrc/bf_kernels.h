@@ -119,6 +119,16 @@ hipError_t bfk_shade(const bf_transport_params* P, const uint32_t* queue, const 
                      uint8_t* route, uint32_t* sample_counts, bool batch, uint32_t mode, hipStream_t s);
 hipError_t bfk_trace_shadow(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr,
                             uint32_t max_count, uint8_t* route, unsigned long long* counters, bool batch, hipStream_t s);
+/* Work orders: `order` becomes a permutation of the queue's items grouped by key (closure kind of the
+ * hit material, or direction octant of the ray or shadow ray), stable within a group; `keys` holds one
+ * byte per item. */
+#define BF_KEY_SHADE 0u
+#define BF_KEY_RAY 1u
+#define BF_KEY_SHADOW 2u
+void bfk_work_order(const bf_transport_params* P, uint32_t key, const uint32_t* queue, const uint32_t* count_ptr,
+                    uint32_t max_count, uint8_t* keys, uint32_t* order, bool batch, hipStream_t s);
+/* Workgroups of `block` lanes the device holds at once: the most over `count` kernels, 0 on error. */
+int bfk_max_resident(const void* const* kernels, int count, uint32_t block, int device);
 /* 256-item tiles the compaction of max_count items uses (size of the tile count / offset arrays / 2). */
 uint32_t bfk_compact_tiles(uint32_t max_count);
 hipError_t bfk_compact(const uint8_t* route, const uint32_t* count_ptr, uint32_t max_count, const uint32_t* src,

@@ -1,0 +1,939 @@
+/*
+ * Traversal kernels: the closest-hit and shadow stages of a bounce, and the stand-alone ray queries
+ * over prepared scenes and over the reference's device blobs.
+ */
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "bf_paths.h"
+#include "bf_scene_soa.h"
+#include "bf_traversal.h"
+
+/* ---- closest-hit stage: gather + traversal + classify + miss ---------------------------------- */
+/* The traversal kernels are persistent: a grid sized to the device's resident capacity, each wave
+ * taking 64 consecutive queue items at a time with a static stride, so that the per-lane stack
+ * spill area is bounded by the grid and empty tail workgroups cost nothing. */
+
+/* One lane's ray between traversal steps. */
+struct lane_ray {
+    uint32_t item, slot;
+    float t_min, t_max;
+    trav_state ts;
+    trav_hit best;
+    bool occluded;
+};
+
+/* World-space ray of a slot, re-read from the path columns (closest-hit rays). `inv` (optional)
+ * holds the lane's world-space reciprocals, entry k at inv[k * stride]. */
+struct closest_world {
+    const bf_dev_paths* paths;
+    uint32_t slot;
+    double* inv;
+    uint32_t stride;
+    BF_D void operator()(v3f& o, v3f& d) const {
+        const float4 a = paths->ray_origin[slot];
+        const float4 b = paths->ray_direction[slot];
+        o = mk(a.x, a.y, a.z);
+        d = mk(b.x, b.y, b.z);
+    }
+};
+
+BF_D void world_space(const closest_world& world, trav_space& s) {
+    world(s.o, s.d);
+    if (world.inv) {
+        s.inv[0] = world.inv[0];
+        s.inv[1] = world.inv[world.stride];
+        s.inv[2] = world.inv[2u * world.stride];
+        finish_space(s);
+    } else {
+        make_space(s.o, s.d, s);
+    }
+}
+
+/* Starts queue item i; returns the traversal status of the root test. */
+template <bool COUNT, bool BATCH, uint32_t BLOCK>
+BF_D uint32_t closest_start(const bf_transport_params& P, const uint32_t* queue, uint32_t i,
+                            trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L, trav_counters& ctr) {
+    L.item = i;
+    L.slot = queue[i];
+    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
+    const float4 ro = P.paths.ray_origin[L.slot];
+    const float4 rd = P.paths.ray_direction[L.slot];
+    trav_ray ray;
+    ray.o = mk(ro.x, ro.y, ro.z);
+    ray.d = mk(rd.x, rd.y, rd.z);
+    ray.t_min = rd.w;
+    ray.t_max = (P.paths.depth[L.slot].z & BF_FIRST_RAY) == 0u
+                    ? BF_INFINITY_F
+                    : (J.in_rays ? J.in_rays[path_of(J, L.slot)].t_max : J.camera.t_max);
+    ray.mask = P.paths.visibility[L.slot];
+    L.t_min = ray.t_min;
+    L.t_max = ray.t_max;
+    bool occluded;
+    return traverse_begin<COUNT>(J.scene, ray, stack, L.ts, L.best, occluded, ctr);
+}
+
+template <bool COUNT, bool BATCH, uint32_t BLOCK>
+BF_D uint32_t closest_step(const bf_transport_params& P, trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L,
+                           trav_counters& ctr, double* inv) {
+    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
+    bool occluded;
+    return traverse_step<false, COUNT>(J.scene, closest_world{&P.paths, L.slot, inv, BLOCK}, stack, L.ts, L.best,
+                                       occluded, ctr);
+}
+
+/* Classifies a finished closest-hit query: hit (route 1, barycentrics re-derived for the winner),
+ * miss (environment radiance, path escapes) or traversal failure. */
+template <bool BATCH>
+BF_D void closest_finish(const bf_transport_params& P, uint8_t* route, lane_ray& L, uint32_t st) {
+    const uint32_t slot = L.slot;
+    const bf_dev_job& J = job_at<BATCH>(P, slot);
+    trav_hit& best = L.best;
+    if (st == BF_HIT_MISS && best.present) {
+        v3f o, d;
+        closest_world{&P.paths, slot, nullptr, 0u}(o, d);
+        st = closest_hit_barycentrics(J.scene, o, d, L.t_min, L.t_max, best);
+    }
+    uint8_t r = 0;
+    if (st != BF_HIT_MISS) {
+        fail_path(P, J, slot, 60u + st);
+    } else if (best.present) {
+        P.paths.hit[slot] = make_float4(best.t, best.b0, best.b1, best.b2);
+        P.paths.hit_ids[slot] = make_uint2(best.scene_instance, best.primitive);
+        r = 1;
+    } else {
+        /* miss stage: CudaWavefrontStages.cu:3962-4040 */
+        if (J.scene.has_environment) {
+            const float4 wl = P.paths.wavelengths[slot];
+            const float4 beta = P.paths.beta[slot];
+            float4 Lr = P.paths.radiance[slot];
+            const float w4[4] = {wl.x, wl.y, wl.z, wl.w};
+            const float b4[4] = {beta.x, beta.y, beta.z, beta.w};
+            float l4[4] = {Lr.x, Lr.y, Lr.z, Lr.w};
+            bool ok = true;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float product;
+                const float radiance = spectrum_at(J.scene, J.scene.environment_spectrum, w4[k]);
+                if (!checked_product(b4[k], radiance, product)) ok = false;
+                else {
+                    l4[k] += product;
+                    if (!bf_isfinite(l4[k]) || l4[k] < 0.0f) ok = false;
+                }
+            }
+            if (!ok) {
+                fail_path(P, J, slot, 50);
+            } else {
+                P.paths.radiance[slot] = make_float4(l4[0], l4[1], l4[2], l4[3]);
+                P.paths.status[slot] = BF_TERM_ESCAPED;
+            }
+        } else {
+            P.paths.status[slot] = BF_TERM_ESCAPED;
+        }
+    }
+    route[L.item] = r;
+}
+
+/*
+ * The persistent lane loop shared by both traversal stages. Every lane holds one ray; a lane whose
+ * ray is done stays idle until REFILL lanes of its wave are (or all are), and then the
+ * wave claims that many queue items with one atomic on the launch's fetch counter. A wave
+ * therefore keeps working while any ray of the queue is unclaimed instead of waiting for its
+ * slowest ray before it moves on. Within a wave, an iteration steps either the lanes whose next
+ * entry is an interior node or those whose next entry is a leaf (LEAF lanes), so the wave issues
+ * one kind of step code at a time instead of every kind under partial masks. Every ray's
+ * traversal is the same sequence of steps in any schedule, so results do not depend on it; the
+ * loop ends when the counter has passed the item count and every lane of the wave is idle.
+ */
+template <uint32_t REFILL, uint32_t LEAF, typename Start, typename Step, typename Finish>
+BF_D void lane_loop(uint32_t n, uint32_t* fetch, Start start, Step step, Finish finish) {
+    const uint32_t lane = threadIdx.x & 63u;
+    bool active = false, exhausted = false;
+    for (;;) {
+        const uint64_t idle = __ballot(!active);
+        const uint32_t want = (uint32_t)__popcll(idle);
+        if (!exhausted && (want >= REFILL || want == 64u)) {
+            uint32_t base = 0u;
+            if (lane == 0u) base = atomicAdd(fetch, want);
+            base = __shfl(base, 0, 64);
+            exhausted = base >= n || n - base <= want;
+            if (!active) {
+                const uint32_t i = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                if (i < n && base < n) {
+                    const uint32_t st = start(i);
+                    if (st != BF_HIT_MISS || !step.pending()) finish(st);
+                    else active = true;
+                }
+            }
+        }
+        if (__ballot(active) == 0ull) {
+            if (exhausted) break;
+            continue;
+        }
+        bool go = active;
+        if (LEAF != 0u) {
+            /* one kind of step per iteration: interior nodes, unless LEAF lanes (or all
+             * active ones) have a leaf next */
+            const bool leaf = active && step.leaf_next();
+            const uint64_t leaves = __ballot(leaf);
+            const bool leaf_phase = (uint32_t)__popcll(leaves) >= LEAF || leaves == __ballot(active);
+            go = active && leaf == leaf_phase;
+        }
+        if (go) {
+            const uint32_t st = step();
+            if (st != BF_HIT_MISS || !step.pending()) {
+                finish(st);
+                active = false;
+            }
+        }
+    }
+}
+
+BF_D void reduce_counters(const trav_counters& c, unsigned long long* counters) {
+    trav_counters ctr = c;
+    for (int off = 32; off > 0; off >>= 1) {
+        ctr.nodes += __shfl_down(ctr.nodes, off, 64);
+        ctr.triangles += __shfl_down(ctr.triangles, off, 64);
+        ctr.instances += __shfl_down(ctr.instances, off, 64);
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        atomicAdd(&counters[0], (unsigned long long)ctr.nodes);
+        atomicAdd(&counters[1], (unsigned long long)ctr.triangles);
+        atomicAdd(&counters[2], (unsigned long long)ctr.instances);
+    }
+}
+
+template <bool COUNT, bool BATCH, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK, BF_TRACE_WAVES_PER_SIMD) void k_trace_closest(bf_transport_params P, const uint32_t* queue,
+                                                                      const uint32_t* count_ptr, const uint32_t* order,
+                                                                      uint8_t* route, unsigned long long* counters) {
+    __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
+    const uint32_t n = *count_ptr;
+    trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
+                                            P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
+    trav_counters ctr{0u, 0u, 0u};
+    lane_ray L;
+    struct stepper {
+        const bf_transport_params* P;
+        trav_stack<BF_SHORT_STACK, BLOCK>* stack;
+        lane_ray* L;
+        trav_counters* ctr;
+        double* inv;
+        BF_D uint32_t operator()() const { return closest_step<COUNT, BATCH>(*P, *stack, *L, *ctr, inv); }
+        BF_D bool pending() const { return stack_depth(*stack) != 0u; }
+        BF_D bool leaf_next() const { return ::leaf_next(*stack); }
+    };
+#if BF_WORLD_INV_CACHE
+    /* the lane's world-space reciprocals, kept for the return from each BLAS */
+    __shared__ double s_inv[3 * BLOCK];
+    double* inv = s_inv + threadIdx.x;
+#else
+    double* inv = nullptr;
+#endif
+    lane_loop<BF_TRACE_REFILL, BF_LEAF_PHASE>(
+        n, P.fetch,
+        [&](uint32_t i) {
+            const uint32_t st = closest_start<COUNT, BATCH>(P, queue, order ? order[i] : i, stack, L, ctr);
+            if (inv) {
+                inv[0] = L.ts.space.inv[0];
+                inv[BLOCK] = L.ts.space.inv[1];
+                inv[2u * BLOCK] = L.ts.space.inv[2];
+            }
+            return st;
+        },
+        stepper{&P, &stack, &L, &ctr, inv}, [&](uint32_t st) { closest_finish<BATCH>(P, route, L, st); });
+    if (COUNT) reduce_counters(ctr, counters);
+}
+
+/* World-space shadow ray of a slot, re-read from the pending-shadow columns. */
+struct shadow_world {
+    const bf_dev_paths* paths;
+    uint32_t slot;
+    BF_D void operator()(v3f& o, v3f& d) const {
+        const float4 a = paths->shadow_origin[slot];
+        const float4 b = paths->shadow_direction[slot];
+        o = mk(a.x, a.y, a.z);
+        d = mk(b.x, b.y, b.z);
+    }
+};
+
+template <bool COUNT, bool BATCH, uint32_t BLOCK>
+BF_D uint32_t shadow_start(const bf_transport_params& P, const uint32_t* queue, uint32_t i,
+                           trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L, trav_counters& ctr) {
+    L.item = i;
+    L.slot = queue[i];
+    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
+    const float4 so = P.paths.shadow_origin[L.slot];
+    const float4 sd = P.paths.shadow_direction[L.slot];
+    trav_ray ray;
+    ray.o = mk(so.x, so.y, so.z);
+    ray.d = mk(sd.x, sd.y, sd.z);
+    ray.t_min = 0.0f;
+    ray.t_max = so.w;
+    ray.mask = P.paths.visibility[L.slot];
+    return traverse_begin<COUNT>(J.scene, ray, stack, L.ts, L.best, L.occluded, ctr);
+}
+
+template <bool COUNT, bool BATCH, uint32_t BLOCK>
+BF_D uint32_t shadow_step(const bf_transport_params& P, trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L,
+                          trav_counters& ctr) {
+    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
+    return traverse_step<true, COUNT>(J.scene, shadow_world{&P.paths, L.slot}, stack, L.ts, L.best, L.occluded, ctr);
+}
+
+/* process_shadow (:4772-4908): the frozen contribution is added when the light is visible (and the
+ * vertex's tape bit set), then the path continues or ends with its pending termination. */
+template <bool BATCH>
+BF_D void shadow_finish(const bf_transport_params& P, uint8_t* route, lane_ray& L, uint32_t st) {
+    const uint32_t slot = L.slot;
+    const bf_dev_job& J = job_at<BATCH>(P, slot);
+    const uint32_t packed = __float_as_uint(P.paths.shadow_direction[slot].w);
+    uint8_t r = 0;
+    if (st != BF_HIT_MISS) {
+        fail_path(P, J, slot, 40);
+    } else {
+        bool ok = true;
+        if (!L.occluded) {
+            if (J.tape_visibility) J.tape_visibility[path_of(J, slot)] |= 1ull << ((packed >> 16) & 63u);
+            const float4 c = P.paths.shadow_contribution[slot];
+            float4 Lr = P.paths.radiance[slot];
+            Lr.x += c.x;
+            Lr.y += c.y;
+            Lr.z += c.z;
+            Lr.w += c.w;
+            if (!bf_isfinite(Lr.x) || !bf_isfinite(Lr.y) || !bf_isfinite(Lr.z) || !bf_isfinite(Lr.w) || Lr.x < 0.0f ||
+                Lr.y < 0.0f || Lr.z < 0.0f || Lr.w < 0.0f) {
+                ok = false;
+                fail_path(P, J, slot, 41);
+            } else {
+                P.paths.radiance[slot] = Lr;
+            }
+        }
+        if (ok) {
+            if (packed & 1u) r = 2;
+            else P.paths.status[slot] = (packed >> 8) & 0xFFu;
+        }
+    }
+    route[L.item] = r;
+}
+
+/* ---- shadow stage: gather + any-hit + process_shadow (:4729-4908) ---------------------------- */
+template <bool COUNT, bool BATCH, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK, BF_SHADOW_WAVES_PER_SIMD) void k_trace_shadow(bf_transport_params P, const uint32_t* queue,
+                                                                          const uint32_t* count_ptr, const uint32_t* order,
+                                                                          uint8_t* route, unsigned long long* counters) {
+    __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
+    const uint32_t n = *count_ptr;
+    trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
+                                            P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
+    trav_counters ctr{0u, 0u, 0u};
+    lane_ray L;
+    struct stepper {
+        const bf_transport_params* P;
+        trav_stack<BF_SHORT_STACK, BLOCK>* stack;
+        lane_ray* L;
+        trav_counters* ctr;
+        BF_D uint32_t operator()() const { return shadow_step<COUNT, BATCH>(*P, *stack, *L, *ctr); }
+        BF_D bool pending() const { return stack_depth(*stack) != 0u; }
+        BF_D bool leaf_next() const { return ::leaf_next(*stack); }
+    };
+    lane_loop<BF_SHADOW_REFILL, BF_SHADOW_LEAF_PHASE>(
+        n, P.fetch + 1, [&](uint32_t i) { return shadow_start<COUNT, BATCH>(P, queue, order ? order[i] : i, stack, L, ctr); },
+        stepper{&P, &stack, &L, &ctr}, [&](uint32_t st) { shadow_finish<BATCH>(P, route, L, st); });
+    if (COUNT) reduce_counters(ctr, counters + 3);
+}
+
+/* ---- stand-alone traversal (blackframe_hip_launch_scene_closest_hit / _occlusion) ----------- */
+/* One ray per lane with a 64-entry LDS stack and no spill area: a lane whose TLAS and BLAS entries
+ * together exceed 64 reports stack overflow (the reference allows 64 per structure; a median-split
+ * BVH never holds more than its depth + 1 entries per structure). */
+__global__ __launch_bounds__(BF_API_BLOCK) void k_scene_closest_hit(bf_dev_scene S, const bf_transport_ray* rays,
+                                                                    uint32_t count, bf_closest_hit_result* results,
+                                                                    uint32_t* counters) {
+    __shared__ uint2 s_stack[BF_API_STACK * BF_API_BLOCK];
+    trav_stack<BF_API_STACK, BF_API_BLOCK> stack{s_stack + threadIdx.x, nullptr, 0u, 0u, 0u, BF_API_STACK};
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    const bf_transport_ray r = rays[i];
+    bf_closest_hit_result out;
+    memset(&out, 0, sizeof out);
+    trav_counters ctr{0u, 0u, 0u};
+    if (!valid_traversal_ray(r)) {
+        out.status = BF_HIT_INVALID_RAY;
+    } else {
+        trav_ray ray;
+        ray.o = mk(r.origin_x, r.origin_y, r.origin_z);
+        ray.d = mk(r.direction_x, r.direction_y, r.direction_z);
+        ray.t_min = r.t_min;
+        ray.t_max = r.t_max;
+        ray.mask = r.visibility_mask;
+        trav_hit best;
+        bool occ;
+        const auto world = [&](v3f& o, v3f& d) {
+            o = mk(rays[i].origin_x, rays[i].origin_y, rays[i].origin_z);
+            d = mk(rays[i].direction_x, rays[i].direction_y, rays[i].direction_z);
+        };
+        uint32_t st = traverse<false, true>(S, ray, world, stack, best, occ, ctr);
+        if (st == BF_HIT_MISS && best.present)
+            st = closest_hit_barycentrics(S, ray.o, ray.d, ray.t_min, ray.t_max, best);
+        if (st != BF_HIT_MISS) {
+            out.status = st;
+        } else if (best.present) {
+            const bf_dev_instance& I = S.instances[best.scene_instance];
+            const float4 q0 = S.leaf_triangles[3 * (size_t)best.leaf + 0];
+            const float4 q1 = S.leaf_triangles[3 * (size_t)best.leaf + 1];
+            const float4 q2 = S.leaf_triangles[3 * (size_t)best.leaf + 2];
+            v3f n;
+            if (!world_normal(I.local_to_world, mk(q0.x, q0.y, q0.z), mk(q1.x, q1.y, q1.z), mk(q2.x, q2.y, q2.z), n)) {
+                out.status = BF_HIT_NUMERICAL_FAILURE;
+            } else {
+                out.status = BF_HIT_HIT;
+                out.hit.parameter = best.t;
+                out.hit.barycentric0 = best.b0;
+                out.hit.barycentric1 = best.b1;
+                out.hit.barycentric2 = best.b2;
+                out.hit.normal_x = n.x;
+                out.hit.normal_y = n.y;
+                out.hit.normal_z = n.z;
+                out.hit.ids.object = I.object_id;
+                out.hit.ids.instance = I.id;
+                out.hit.ids.geometry = S.geometries[I.geometry_index].id;
+                out.hit.ids.primitive = best.primitive;
+                out.hit.ids.material = S.materials[I.material_index].id;
+            }
+        }
+    }
+    results[i] = out;
+    if (counters) {
+        counters[3 * (size_t)i] = ctr.nodes;
+        counters[3 * (size_t)i + 1] = ctr.triangles;
+        counters[3 * (size_t)i + 2] = ctr.instances;
+    }
+}
+
+__global__ __launch_bounds__(BF_API_BLOCK) void k_scene_occlusion(bf_dev_scene S, const bf_transport_ray* rays,
+                                                                  uint32_t count, bf_occlusion_result* results) {
+    __shared__ uint2 s_stack[BF_API_STACK * BF_API_BLOCK];
+    trav_stack<BF_API_STACK, BF_API_BLOCK> stack{s_stack + threadIdx.x, nullptr, 0u, 0u, 0u, BF_API_STACK};
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    const bf_transport_ray r = rays[i];
+    bf_occlusion_result out;
+    memset(&out, 0, sizeof out);
+    if (!valid_traversal_ray(r)) {
+        out.status = BF_HIT_INVALID_RAY;
+    } else {
+        trav_ray ray;
+        ray.o = mk(r.origin_x, r.origin_y, r.origin_z);
+        ray.d = mk(r.direction_x, r.direction_y, r.direction_z);
+        ray.t_min = r.t_min;
+        ray.t_max = r.t_max;
+        ray.mask = r.visibility_mask;
+        trav_hit best;
+        bool occ;
+        trav_counters ctr{0u, 0u, 0u};
+        const auto world = [&](v3f& o, v3f& d) {
+            o = mk(rays[i].origin_x, rays[i].origin_y, rays[i].origin_z);
+            d = mk(rays[i].direction_x, rays[i].direction_y, rays[i].direction_z);
+        };
+        const uint32_t st = traverse<true, false>(S, ray, world, stack, best, occ, ctr);
+        out.status = st != BF_HIT_MISS ? st : (occ ? BF_OCCLUDED : BF_VISIBLE);
+    }
+    results[i] = out;
+}
+
+/* ---- stand-alone traversal over the reference's device blobs ----------------------------------
+ * blackframe_hip_launch_scene_closest_hit_blob / _occlusion_blob take the reference launcher's
+ * arguments (SceneClosestHit.hpp, CudaSceneClosestHit.cu:188-1330): "BLKFSOA4" scene bytes and a
+ * "BLKFBVH1" BVH in device memory. The first lane of every workgroup validates both layouts
+ * (validate_scene_layout / validate_bvh_layout, :199-358) and a bad one answers every ray of the
+ * workgroup with invalid_scene / invalid_bvh. Each lane then traverses one ray over the canonical
+ * 48-byte nodes in the reference's order: pop, re-test the node's own box against the current
+ * t_max, push both intersecting children far then near (ties to the first), enter an instance leaf
+ * in object space after checking it against the scene's columns, and test a BLAS leaf's triangle
+ * from the scene's index and position columns. The box and triangle decisions are this library's
+ * binary64 slab and watertight test, so the results equal those of
+ * blackframe_hip_launch_scene_closest_hit on the scene the blobs describe. The TLAS and each BLAS
+ * get their own 64-entry LDS stack, as in the reference. */
+struct blob_view {
+    const uint8_t* scene;
+    const bf_scene_soa_header* sh;
+    const uint8_t* bvh;
+    const bf_bvh_header* bh;
+};
+
+template <typename T>
+BF_D const T* soa_col(const blob_view& b, uint32_t column) {
+    return (const T*)(b.scene + b.sh->columns[column].offset_bytes);
+}
+
+template <typename T>
+BF_D const T* bvh_arr(const blob_view& b, uint32_t array) {
+    return (const T*)(b.bvh + b.bh->arrays[array].offset_bytes);
+}
+
+BF_D uint64_t blob_align(uint64_t v, uint64_t a) { return (v + a - 1u) / a * a; }
+
+/* validate_scene_layout (:199-250) */
+BF_D uint32_t blob_scene_layout(const uint8_t* bytes, size_t n) {
+    if (n < sizeof(bf_scene_soa_header)) return BF_HIT_INVALID_SCENE;
+    const bf_scene_soa_header& h = *(const bf_scene_soa_header*)bytes;
+    if (h.magic != BF_SCENE_SOA_MAGIC || h.abi_major != BF_SCENE_SOA_ABI_MAJOR || h.abi_minor != BF_SCENE_SOA_ABI_MINOR ||
+        h.header_size != sizeof(bf_scene_soa_header) || h.column_count != BF_SCENE_SOA_COLUMN_COUNT ||
+        h.hash_algorithm != BF_SCENE_SOA_HASH_FNV1A64 || h.environment_count > 1u || h.total_size_bytes != n ||
+        h.total_size_bytes < sizeof(bf_scene_soa_header) || h.texture_count > 0xFFFFFFFFull ||
+        h.image_texture_count > 0xFFFFFFFFull || h.image_mip_count > 0xFFFFFFFFull)
+        return BF_HIT_INVALID_SCENE;
+    for (int k = 0; k < 5; ++k)
+        if (h.reserved[k] != 0u) return BF_HIT_INVALID_SCENE;
+    const uint64_t max = ~0ull;
+    uint64_t cursor = blob_align(sizeof(bf_scene_soa_header), BF_SCENE_SOA_COLUMN_ALIGNMENT);
+    for (uint32_t c = 0; c < BF_SCENE_SOA_COLUMN_COUNT; ++c) {
+        const bf_scene_soa_column& d = h.columns[c];
+        const uint64_t count = bf_soa::column_count(h, c);
+        const uint64_t size = bf_soa::column_element_size(c);
+        if (d.element_count != count || d.element_size != size || d.reserved != 0u) return BF_HIT_INVALID_SCENE;
+        if (count == 0u) {
+            if (d.offset_bytes != 0u) return BF_HIT_INVALID_SCENE;
+            continue;
+        }
+        if (cursor > max - (BF_SCENE_SOA_COLUMN_ALIGNMENT - 1u)) return BF_HIT_INVALID_SCENE;
+        cursor = blob_align(cursor, BF_SCENE_SOA_COLUMN_ALIGNMENT);
+        if (d.offset_bytes != cursor || count > max / size) return BF_HIT_INVALID_SCENE;
+        const uint64_t bytes_in_column = count * size;
+        if (cursor > max - bytes_in_column) return BF_HIT_INVALID_SCENE;
+        cursor += bytes_in_column;
+    }
+    return cursor == h.total_size_bytes ? BF_HIT_MISS : BF_HIT_INVALID_SCENE;
+}
+
+/* validate_bvh_layout (:291-358) */
+BF_D uint32_t blob_bvh_layout(const uint8_t* bytes, size_t n, const bf_scene_soa_header& scene) {
+    if (n < sizeof(bf_bvh_header)) return BF_HIT_INVALID_BVH;
+    const bf_bvh_header& h = *(const bf_bvh_header*)bytes;
+    const uint64_t invalid = BF_INVALID_INDEX;
+    if (h.magic != BF_BVH_MAGIC || h.abi_major != BF_BVH_ABI_MAJOR || h.abi_minor != BF_BVH_ABI_MINOR ||
+        h.header_size != sizeof(bf_bvh_header) || h.array_count != BF_BVH_ARRAY_COUNT ||
+        h.hash_algorithm != BF_BVH_HASH_FNV1A64 || h.leaf_capacity != BF_BVH_LEAF_CAPACITY || h.total_size_bytes != n ||
+        h.total_size_bytes < sizeof(bf_bvh_header) || h.source_scene_hash != scene.content_hash ||
+        h.blas_count != scene.geometry_count || h.primitive_reference_count != scene.triangle_count ||
+        h.instance_reference_count != scene.instance_count || h.blas_count > invalid || h.blas_node_count > invalid ||
+        h.primitive_reference_count > invalid || h.tlas_node_count > invalid || h.instance_reference_count > invalid)
+        return BF_HIT_INVALID_BVH;
+    if ((h.blas_count == 0u && (h.blas_node_count != 0u || h.primitive_reference_count != 0u)) ||
+        (h.blas_count != 0u && (h.primitive_reference_count < h.blas_count ||
+                                h.blas_node_count != h.primitive_reference_count * 2u - h.blas_count)) ||
+        (h.instance_reference_count == 0u && h.tlas_node_count != 0u) ||
+        (h.instance_reference_count != 0u && h.tlas_node_count != h.instance_reference_count * 2u - 1u) ||
+        (h.tlas_node_count == 0u && h.tlas_root_node != BF_INVALID_INDEX) ||
+        (h.tlas_node_count != 0u && h.tlas_root_node != 0u))
+        return BF_HIT_INVALID_BVH;
+    for (int k = 0; k < 5; ++k)
+        if (h.reserved[k] != 0u) return BF_HIT_INVALID_BVH;
+    const uint64_t counts[BF_BVH_ARRAY_COUNT] = {h.blas_count, h.blas_node_count, h.primitive_reference_count,
+                                                 h.tlas_node_count, h.instance_reference_count};
+    const uint64_t sizes[BF_BVH_ARRAY_COUNT] = {sizeof(bf_bvh_blas), sizeof(bf_bvh_node), sizeof(uint32_t),
+                                                sizeof(bf_bvh_node), sizeof(bf_bvh_instance_ref)};
+    const uint64_t max = ~0ull;
+    uint64_t cursor = blob_align(sizeof(bf_bvh_header), BF_BVH_ARRAY_ALIGNMENT);
+    for (uint32_t a = 0; a < BF_BVH_ARRAY_COUNT; ++a) {
+        const bf_bvh_array_descriptor& d = h.arrays[a];
+        if (d.element_count != counts[a] || d.element_size != sizes[a] || d.reserved != 0u) return BF_HIT_INVALID_BVH;
+        if (counts[a] == 0u) {
+            if (d.offset_bytes != 0u) return BF_HIT_INVALID_BVH;
+            continue;
+        }
+        if (cursor > max - (BF_BVH_ARRAY_ALIGNMENT - 1u)) return BF_HIT_INVALID_BVH;
+        cursor = blob_align(cursor, BF_BVH_ARRAY_ALIGNMENT);
+        if (d.offset_bytes != cursor || counts[a] > max / sizes[a]) return BF_HIT_INVALID_BVH;
+        const uint64_t bytes_in_array = counts[a] * sizes[a];
+        if (cursor > max - bytes_in_array) return BF_HIT_INVALID_BVH;
+        cursor += bytes_in_array;
+    }
+    return cursor == h.total_size_bytes ? BF_HIT_MISS : BF_HIT_INVALID_BVH;
+}
+
+/* intersect_bounds (:407-455): the node's box, validated, in the reference's binary64 slab */
+BF_D uint32_t blob_box(const bf_bvh_node& n, const trav_space& s, float t_min, float t_max, bool& hit, float& nearv) {
+    if (!bf_isfinite(n.min_x) || !bf_isfinite(n.min_y) || !bf_isfinite(n.min_z) || !bf_isfinite(n.max_x) ||
+        !bf_isfinite(n.max_y) || !bf_isfinite(n.max_z) || n.min_x > n.max_x || n.min_y > n.max_y || n.min_z > n.max_z)
+        return BF_HIT_INVALID_TOPOLOGY;
+    double v = 0.0;
+    const uint32_t st = slab_exact(n.min_x, n.min_y, n.min_z, n.max_x, n.max_y, n.max_z, s, t_min, t_max, hit, v);
+    nearv = (float)v;
+    return st;
+}
+
+/* push_intersecting_children (:466-512) */
+BF_D uint32_t blob_push_children(const bf_bvh_node* nodes, const bf_bvh_node& n, uint32_t begin, uint32_t count,
+                                 const trav_space& s, float t_min, float t_max, uint32_t* stack, uint32_t& size) {
+    const uint64_t end = (uint64_t)begin + count;
+    const uint32_t a = n.first_child, b = n.second_child;
+    if (a == b || a < begin || b < begin || a >= end || b >= end) return BF_HIT_INVALID_TOPOLOGY;
+    bool ha, hb;
+    float na = 0.0f, nb = 0.0f;
+    uint32_t st = blob_box(nodes[a], s, t_min, t_max, ha, na);
+    if (st != BF_HIT_MISS) return st;
+    st = blob_box(nodes[b], s, t_min, t_max, hb, nb);
+    if (st != BF_HIT_MISS) return st;
+    if (!ha && !hb) return BF_HIT_MISS;
+    if (ha != hb) {
+        if (size >= BF_STRUCTURE_STACK) return BF_HIT_STACK_OVERFLOW;
+        stack[(size++) * BF_API_BLOCK] = ha ? a : b;
+        return BF_HIT_MISS;
+    }
+    const bool a_near = na < nb || (na == nb && a < b);
+    if (size >= BF_STRUCTURE_STACK) return BF_HIT_STACK_OVERFLOW;
+    stack[(size++) * BF_API_BLOCK] = a_near ? b : a;
+    if (size >= BF_STRUCTURE_STACK) return BF_HIT_STACK_OVERFLOW;
+    stack[(size++) * BF_API_BLOCK] = a_near ? a : b;
+    return BF_HIT_MISS;
+}
+
+/* a 3x4 affine matrix from one of the scene's 16-element matrix column groups (:513-537) */
+BF_D uint32_t blob_matrix(const blob_view& b, uint32_t first_column, uint32_t instance, float* m) {
+    float full[16];
+    for (uint32_t e = 0; e < 16u; ++e) {
+        full[e] = soa_col<float>(b, first_column + e)[instance];
+        if (!bf_isfinite(full[e])) return BF_HIT_NUMERICAL_FAILURE;
+    }
+    if (full[12] != 0.0f || full[13] != 0.0f || full[14] != 0.0f || full[15] != 1.0f) return BF_HIT_INVALID_TOPOLOGY;
+    for (uint32_t e = 0; e < 12u; ++e) m[e] = full[e];
+    return BF_HIT_MISS;
+}
+
+struct blob_candidate {
+    bool present;
+    float t;
+    uint32_t instance_id, primitive;
+    bf_closest_hit hit;
+};
+
+/* traverse_blas (:895-1085) */
+template <bool ANY>
+BF_D uint32_t blob_blas(const blob_view& b, const bf_bvh_instance_ref& ref, const bf_transport_ray& ray, v3f lo, v3f ld,
+                        uint32_t* stack, blob_candidate& best, bool& occluded) {
+    const bf_bvh_blas* blases = bvh_arr<bf_bvh_blas>(b, 0);
+    const bf_bvh_node* nodes = bvh_arr<bf_bvh_node>(b, 1);
+    const uint32_t* prims = bvh_arr<uint32_t>(b, 2);
+    if (ref.blas_index >= b.bh->blas_count || ref.scene_geometry_index >= b.sh->geometry_count)
+        return BF_HIT_INVALID_TOPOLOGY;
+    const bf_bvh_blas B = blases[ref.blas_index];
+    const uint64_t node_end = (uint64_t)B.node_offset + B.node_count;
+    const uint64_t ref_end = (uint64_t)B.primitive_reference_offset + B.primitive_reference_count;
+    if (B.reserved[0] != 0u || B.reserved[1] != 0u || B.geometry_id != ref.geometry_id || B.root_node != B.node_offset ||
+        B.node_count == 0u || node_end > b.bh->blas_node_count ||
+        B.node_count != (uint64_t)B.primitive_reference_count * 2u - 1u || ref_end > b.bh->primitive_reference_count)
+        return BF_HIT_INVALID_TOPOLOGY;
+    const uint32_t g = ref.scene_geometry_index;
+    const uint64_t vertex_offset = soa_col<uint64_t>(b, bf_soa::C_GEOMETRY_VERTEX_OFFSET)[g];
+    const uint64_t vertex_count = soa_col<uint64_t>(b, bf_soa::C_GEOMETRY_VERTEX_COUNT)[g];
+    const uint64_t triangle_offset = soa_col<uint64_t>(b, bf_soa::C_GEOMETRY_TRIANGLE_OFFSET)[g];
+    const uint64_t triangle_count = soa_col<uint64_t>(b, bf_soa::C_GEOMETRY_TRIANGLE_COUNT)[g];
+    if (soa_col<uint32_t>(b, bf_soa::C_GEOMETRY_ID)[g] != ref.geometry_id || triangle_count != B.primitive_reference_count ||
+        vertex_count == 0u || vertex_offset > b.sh->vertex_count || vertex_count > b.sh->vertex_count - vertex_offset ||
+        triangle_offset > b.sh->triangle_count || triangle_count > b.sh->triangle_count - triangle_offset)
+        return BF_HIT_INVALID_TOPOLOGY;
+    trav_space s;
+    make_space(lo, ld, s);
+    trav_shear sh;
+    make_shear(ld, sh);
+    uint32_t size = 0, visited = 0;
+    stack[(size++) * BF_API_BLOCK] = B.root_node;
+    while (size != 0u) {
+        if (visited++ >= B.node_count) return BF_HIT_INVALID_TOPOLOGY;
+        const uint32_t index = stack[(--size) * BF_API_BLOCK];
+        if (index < B.node_offset || index >= node_end) return BF_HIT_INVALID_TOPOLOGY;
+        const bf_bvh_node n = nodes[index];
+        const float t_max = ANY ? ray.t_max : best.t;
+        bool h;
+        float nearv;
+        uint32_t st = blob_box(n, s, ray.t_min, t_max, h, nearv);
+        if (st != BF_HIT_MISS) return st;
+        if (!h) continue;
+        if (n.kind == 0u) {
+            if (n.split_axis > 2u || n.reference_offset != 0u || n.reference_count != 0u) return BF_HIT_INVALID_TOPOLOGY;
+            st = blob_push_children(nodes, n, B.node_offset, B.node_count, s, ray.t_min, t_max, stack, size);
+            if (st != BF_HIT_MISS) return st;
+            continue;
+        }
+        if (n.kind != 1u || n.split_axis != BF_INVALID_INDEX || n.first_child != BF_INVALID_INDEX ||
+            n.second_child != BF_INVALID_INDEX || n.reference_count != 1u || n.reference_offset < B.primitive_reference_offset ||
+            n.reference_offset >= ref_end)
+            return BF_HIT_INVALID_TOPOLOGY;
+        const uint32_t prim = prims[n.reference_offset];
+        if (prim >= triangle_count) return BF_HIT_INVALID_TOPOLOGY;
+        const uint64_t tri = triangle_offset + prim;
+        v3f v[3];
+        for (uint32_t c = 0; c < 3u; ++c) {
+            const uint32_t local = soa_col<uint32_t>(b, bf_soa::C_TRIANGLE_VERTEX_0 + c)[tri];
+            if (local >= vertex_count) return BF_HIT_INVALID_TOPOLOGY;
+            const uint64_t gv = vertex_offset + local;
+            v[c] = mk(soa_col<float>(b, bf_soa::C_POSITION_X)[gv], soa_col<float>(b, bf_soa::C_POSITION_X + 1)[gv],
+                      soa_col<float>(b, bf_soa::C_POSITION_X + 2)[gv]);
+            if (!fin3(v[c])) return BF_HIT_NUMERICAL_FAILURE;
+        }
+        tri_result tr;
+        tr.hit = false;
+        st = watertight<!ANY>(v[0], v[1], v[2], lo, ld, sh, ray.t_min, t_max, tr);
+        if (st != BF_HIT_MISS) return st;
+        if (!tr.hit) continue;
+        if (ANY) {
+            occluded = true;
+            return BF_HIT_MISS;
+        }
+        if (best.present && !(tr.t < best.t ||
+                              (tr.t == best.t && (ref.instance_id < best.instance_id ||
+                                                  (ref.instance_id == best.instance_id && prim < best.primitive)))))
+            continue;
+        float m[12];
+        st = blob_matrix(b, bf_soa::C_INSTANCE_LOCAL_TO_WORLD, ref.scene_instance_index, m);
+        if (st != BF_HIT_MISS) return st;
+        v3f nrm;
+        if (!world_normal(m, v[0], v[1], v[2], nrm)) return BF_HIT_NUMERICAL_FAILURE;
+        const uint32_t inst = ref.scene_instance_index;
+        if (soa_col<uint32_t>(b, bf_soa::C_INSTANCE_ID)[inst] != ref.instance_id ||
+            soa_col<uint32_t>(b, bf_soa::C_INSTANCE_GEOMETRY_ID)[inst] != ref.geometry_id)
+            return BF_HIT_INVALID_TOPOLOGY;
+        best.present = true;
+        best.t = tr.t;
+        best.instance_id = ref.instance_id;
+        best.primitive = prim;
+        bf_closest_hit& hr = best.hit;
+        memset(&hr, 0, sizeof hr);
+        hr.parameter = tr.t;
+        hr.barycentric0 = tr.b0;
+        hr.barycentric1 = tr.b1;
+        hr.barycentric2 = tr.b2;
+        hr.normal_x = nrm.x;
+        hr.normal_y = nrm.y;
+        hr.normal_z = nrm.z;
+        hr.ids.object = soa_col<uint32_t>(b, bf_soa::C_INSTANCE_OBJECT_ID)[inst];
+        hr.ids.instance = ref.instance_id;
+        hr.ids.geometry = ref.geometry_id;
+        hr.ids.primitive = prim;
+        hr.ids.material = soa_col<uint32_t>(b, bf_soa::C_INSTANCE_MATERIAL_ID)[inst];
+    }
+    return BF_HIT_MISS;
+}
+
+/* trace_scene (:1087-1186) */
+template <bool ANY>
+BF_D uint32_t blob_trace(const blob_view& b, const bf_transport_ray& ray, uint32_t* tlas_stack, uint32_t* blas_stack,
+                         blob_candidate& best, bool& occluded) {
+    if (b.bh->tlas_node_count == 0u) return BF_HIT_MISS;
+    const bf_bvh_node* nodes = bvh_arr<bf_bvh_node>(b, 3);
+    const bf_bvh_instance_ref* refs = bvh_arr<bf_bvh_instance_ref>(b, 4);
+    const uint32_t tlas_count = (uint32_t)b.bh->tlas_node_count;
+    trav_space world;
+    const v3f o = mk(ray.origin_x, ray.origin_y, ray.origin_z), d = mk(ray.direction_x, ray.direction_y, ray.direction_z);
+    make_space(o, d, world);
+    uint32_t size = 0, visited = 0;
+    tlas_stack[(size++) * BF_API_BLOCK] = b.bh->tlas_root_node;
+    while (size != 0u) {
+        if (visited++ >= tlas_count) return BF_HIT_INVALID_TOPOLOGY;
+        const uint32_t index = tlas_stack[(--size) * BF_API_BLOCK];
+        if (index >= tlas_count) return BF_HIT_INVALID_TOPOLOGY;
+        const bf_bvh_node n = nodes[index];
+        const float t_max = ANY ? ray.t_max : best.t;
+        bool h;
+        float nearv;
+        uint32_t st = blob_box(n, world, ray.t_min, t_max, h, nearv);
+        if (st != BF_HIT_MISS) return st;
+        if (!h) continue;
+        if (n.kind == 0u) {
+            if (n.split_axis > 2u || n.reference_offset != 0u || n.reference_count != 0u) return BF_HIT_INVALID_TOPOLOGY;
+            st = blob_push_children(nodes, n, 0u, tlas_count, world, ray.t_min, t_max, tlas_stack, size);
+            if (st != BF_HIT_MISS) return st;
+            continue;
+        }
+        if (n.kind != 1u || n.split_axis != BF_INVALID_INDEX || n.first_child != BF_INVALID_INDEX ||
+            n.second_child != BF_INVALID_INDEX || n.reference_count != 1u ||
+            n.reference_offset >= b.bh->instance_reference_count)
+            return BF_HIT_INVALID_TOPOLOGY;
+        const bf_bvh_instance_ref ref = refs[n.reference_offset];
+        if (ref.reserved[0] != 0u || ref.reserved[1] != 0u || ref.scene_instance_index >= b.sh->instance_count ||
+            ref.scene_geometry_index >= b.sh->geometry_count || ref.blas_index >= b.bh->blas_count)
+            return BF_HIT_INVALID_TOPOLOGY;
+        const uint32_t inst = ref.scene_instance_index;
+        if (soa_col<uint32_t>(b, bf_soa::C_INSTANCE_ID)[inst] != ref.instance_id ||
+            soa_col<uint32_t>(b, bf_soa::C_INSTANCE_GEOMETRY_ID)[inst] != ref.geometry_id ||
+            soa_col<uint32_t>(b, bf_soa::C_INSTANCE_VISIBILITY_MASK)[inst] != ref.visibility_mask)
+            return BF_HIT_INVALID_TOPOLOGY;
+        if ((ray.visibility_mask & ref.visibility_mask) == 0u) continue;
+        float m[12];
+        st = blob_matrix(b, bf_soa::C_INSTANCE_WORLD_TO_LOCAL, inst, m);
+        if (st != BF_HIT_MISS) return st;
+        const v3f lo = xform_point(m, o), ld = xform_vector(m, d);
+        if (!fin3(lo) || !fin3(ld) || (ld.x == 0.0f && ld.y == 0.0f && ld.z == 0.0f)) return BF_HIT_NUMERICAL_FAILURE;
+        st = blob_blas<ANY>(b, ref, ray, lo, ld, blas_stack, best, occluded);
+        if (st != BF_HIT_MISS) return st;
+        if (ANY && occluded) return BF_HIT_MISS;
+    }
+    return BF_HIT_MISS;
+}
+
+template <bool ANY>
+__global__ __launch_bounds__(BF_API_BLOCK) void k_blob_traverse(const uint8_t* scene_bytes, size_t scene_size,
+                                                                const uint8_t* bvh_bytes, size_t bvh_size,
+                                                                const bf_transport_ray* rays, uint32_t count,
+                                                                void* results) {
+    __shared__ uint32_t s_layout;
+    __shared__ uint32_t s_tlas[BF_STRUCTURE_STACK * BF_API_BLOCK];
+    __shared__ uint32_t s_blas[BF_STRUCTURE_STACK * BF_API_BLOCK];
+    if (threadIdx.x == 0u) {
+        uint32_t st = blob_scene_layout(scene_bytes, scene_size);
+        if (st == BF_HIT_MISS) st = blob_bvh_layout(bvh_bytes, bvh_size, *(const bf_scene_soa_header*)scene_bytes);
+        s_layout = st;
+    }
+    __syncthreads();
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    uint32_t status = s_layout;
+    blob_candidate best;
+    best.present = false;
+    bool occluded = false;
+    if (status == BF_HIT_MISS) {
+        const bf_transport_ray r = rays[i];
+        if (!valid_traversal_ray(r)) {
+            status = BF_HIT_INVALID_RAY;
+        } else {
+            const blob_view b{scene_bytes, (const bf_scene_soa_header*)scene_bytes, bvh_bytes,
+                              (const bf_bvh_header*)bvh_bytes};
+            best.t = r.t_max;
+            status = blob_trace<ANY>(b, r, s_tlas + threadIdx.x, s_blas + threadIdx.x, best, occluded);
+        }
+    }
+    if (ANY) {
+        bf_occlusion_result out;
+        memset(&out, 0, sizeof out);
+        out.status = status != BF_HIT_MISS ? status : (occluded ? BF_OCCLUDED : BF_VISIBLE);
+        ((bf_occlusion_result*)results)[i] = out;
+    } else {
+        bf_closest_hit_result out;
+        memset(&out, 0, sizeof out);
+        if (status != BF_HIT_MISS) out.status = status;
+        else if (best.present) {
+            out.status = BF_HIT_HIT;
+            out.hit = best.hit;
+        }
+        ((bf_closest_hit_result*)results)[i] = out;
+    }
+}
+
+/* Workgroups of one persistent traversal launch: enough to fill every CU at the kernels'
+ * occupancy, never more than the workspace's spill area covers, and no more than the items need. */
+static uint32_t trace_blocks(const bf_transport_params* P, uint32_t max_count, uint32_t block) {
+    const uint32_t needed = blocks_for((max_count + 63u) / 64u * 64u, block);
+    const uint32_t resident = P->spill_stride / block;
+    return needed < resident ? needed : resident;
+}
+
+template <bool ANY, bool COUNT, bool BATCH, uint32_t BLOCK>
+static void launch_trace(const bf_transport_params* P, uint32_t max_count, const uint32_t* q, const uint32_t* n,
+                         uint8_t* route, unsigned long long* counters, hipStream_t s) {
+    const dim3 grid(trace_blocks(P, max_count, BLOCK));
+    (void)bfk_set_words(P->fetch + (ANY ? 1 : 0), 1u, 0u, s);
+    /* optional direction-octant order; the route bytes are free until the traversal writes them */
+    uint32_t* order = ANY ? P->shadow_order : P->closest_order;
+    if (order)
+        bfk_work_order(P, ANY ? BF_KEY_SHADOW : BF_KEY_RAY, q, n, max_count, route, order, BATCH, s);
+    if (ANY)
+        hipLaunchKernelGGL((k_trace_shadow<COUNT, BATCH, BLOCK>), grid, dim3(BLOCK), 0, s, *P, q, n, order, route, counters);
+    else
+        hipLaunchKernelGGL((k_trace_closest<COUNT, BATCH, BLOCK>), grid, dim3(BLOCK), 0, s, *P, q, n, order, route, counters);
+}
+
+template <bool ANY, bool COUNT, bool BATCH>
+static void launch_trace_block(const bf_transport_params* P, uint32_t max_count, const uint32_t* q, const uint32_t* n,
+                               uint8_t* route, unsigned long long* counters, hipStream_t s) {
+    if (P->trace_block == 64u) launch_trace<ANY, COUNT, BATCH, 64u>(P, max_count, q, n, route, counters, s);
+    else if (P->trace_block == 256u) launch_trace<ANY, COUNT, BATCH, 256u>(P, max_count, q, n, route, counters, s);
+    else launch_trace<ANY, COUNT, BATCH, 128u>(P, max_count, q, n, route, counters, s);
+}
+
+template <bool ANY>
+static hipError_t trace_stage(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr,
+                              uint32_t max_count, uint8_t* route, unsigned long long* counters, bool batch, hipStream_t s) {
+    if (max_count == 0) return hipSuccess;
+    if (counters) {
+        if (batch) launch_trace_block<ANY, true, true>(P, max_count, queue, count_ptr, route, counters, s);
+        else launch_trace_block<ANY, true, false>(P, max_count, queue, count_ptr, route, counters, s);
+    } else {
+        if (batch) launch_trace_block<ANY, false, true>(P, max_count, queue, count_ptr, route, counters, s);
+        else launch_trace_block<ANY, false, false>(P, max_count, queue, count_ptr, route, counters, s);
+    }
+    return hipGetLastError();
+}
+
+template <uint32_t BLOCK>
+static void trace_kernels(const void** out) {
+    out[0] = (const void*)k_trace_closest<false, false, BLOCK>;
+    out[1] = (const void*)k_trace_closest<true, false, BLOCK>;
+    out[2] = (const void*)k_trace_closest<false, true, BLOCK>;
+    out[3] = (const void*)k_trace_closest<true, true, BLOCK>;
+    out[4] = (const void*)k_trace_shadow<false, false, BLOCK>;
+    out[5] = (const void*)k_trace_shadow<true, false, BLOCK>;
+    out[6] = (const void*)k_trace_shadow<false, true, BLOCK>;
+    out[7] = (const void*)k_trace_shadow<true, true, BLOCK>;
+}
+
+extern "C" {
+
+hipError_t bfk_trace_closest(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr,
+                             uint32_t max_count, uint8_t* route, unsigned long long* counters, bool batch, hipStream_t s) {
+    return trace_stage<false>(P, queue, count_ptr, max_count, route, counters, batch, s);
+}
+
+hipError_t bfk_trace_shadow(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr,
+                            uint32_t max_count, uint8_t* route, unsigned long long* counters, bool batch, hipStream_t s) {
+    return trace_stage<true>(P, queue, count_ptr, max_count, route, counters, batch, s);
+}
+
+/* Lanes the device holds at once for the widest-resident traversal kernel variant: the width of
+ * the spill area, one column per lane. */
+uint32_t bfk_trace_resident_lanes(int device) {
+    const void* k64[8];
+    const void* k128[8];
+    const void* k256[8];
+    trace_kernels<64u>(k64);
+    trace_kernels<128u>(k128);
+    trace_kernels<256u>(k256);
+    const uint32_t a = (uint32_t)bfk_max_resident(k64, 8, 64u, device) * 64u;
+    const uint32_t b = (uint32_t)bfk_max_resident(k128, 8, 128u, device) * 128u;
+    const uint32_t c = (uint32_t)bfk_max_resident(k256, 8, 256u, device) * 256u;
+    if (a == 0 || b == 0 || c == 0) return 0;
+    return std::max(a, std::max(b, c));
+}
+
+hipError_t bfk_scene_closest_hit(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
+                                 bf_closest_hit_result* results, uint32_t* counters, hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_scene_closest_hit, dim3(blocks_for(count, BF_API_BLOCK)), dim3(BF_API_BLOCK), 0, s, *S, rays,
+                       count, results, counters);
+    return hipGetLastError();
+}
+
+hipError_t bfk_blob_traverse(bool any, const uint8_t* scene_bytes, size_t scene_size, const uint8_t* bvh_bytes,
+                             size_t bvh_size, const bf_transport_ray* rays, uint32_t count, void* results, hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    const dim3 grid(blocks_for(count, BF_API_BLOCK)), block(BF_API_BLOCK);
+    if (any)
+        hipLaunchKernelGGL(k_blob_traverse<true>, grid, block, 0, s, scene_bytes, scene_size, bvh_bytes, bvh_size, rays,
+                           count, results);
+    else
+        hipLaunchKernelGGL(k_blob_traverse<false>, grid, block, 0, s, scene_bytes, scene_size, bvh_bytes, bvh_size, rays,
+                           count, results);
+    return hipGetLastError();
+}
+
+hipError_t bfk_scene_occlusion(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
+                               bf_occlusion_result* results, hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_scene_occlusion, dim3(blocks_for(count, BF_API_BLOCK)), dim3(BF_API_BLOCK), 0, s, *S, rays,
+                       count, results);
+    return hipGetLastError();
+}
+
+} /* extern "C" */
