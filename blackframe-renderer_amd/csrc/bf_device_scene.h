@@ -5,7 +5,8 @@
  *  - wide BVH nodes: one 64-byte line per internal node holding both child boxes (bf_wide_node);
  *  - leaf triangles: 48-byte records in BLAS leaf order (3 x float4: vertex xyz + payload word),
  *    so a leaf costs one 48-byte fetch and never a node fetch;
- *  - TLAS leaves: one 64-byte record per instance reference (world->local 3x4 + ids + mask);
+ *  - TLAS leaves: one 96-byte record per instance reference (world->local 3x4, ids, mask, world box,
+ *    BLAS root);
  *  - path state: structure-of-arrays columns indexed by path slot, float4-wide where possible.
  */
 #ifndef BF_DEVICE_SCENE_H
@@ -35,17 +36,16 @@
 #ifndef BF_TRACE_WAVES_PER_SIMD
 #define BF_TRACE_WAVES_PER_SIMD 6 /* register budget of the closest-hit traversal (waves per SIMD) */
 #endif
+#ifndef BF_COUNT_WAVES_PER_SIMD
+#define BF_COUNT_WAVES_PER_SIMD 6 /* the step-exact counting walk */
+#endif
 #ifndef BF_LEAF_PHASE
-/* Traversal waves step interior nodes and leaves in separate iterations: leaves when at least this
- * many lanes (or every active lane) have one next, interior nodes otherwise (0: every kind in
- * every iteration, each under its own lane mask). 16 measured best of {1, 4, 8, 12, 16, 32, 64}. */
-#define BF_LEAF_PHASE 16u
+/* Traversal waves step interior nodes and leaves in separate iterations: leaves once they are this
+ * fraction (1/4) of the running lanes. */
+#define BF_LEAF_PHASE 4u
 #endif
 #ifndef BF_SHADOW_LEAF_PHASE
-#define BF_SHADOW_LEAF_PHASE 16u /* the same for any-hit waves (8, 24 and 32 measured slower) */
-#endif
-#ifndef BF_WORLD_INV_CACHE
-#define BF_WORLD_INV_CACHE 1 /* closest-hit lanes keep their world-space reciprocals in LDS */
+#define BF_SHADOW_LEAF_PHASE 4u /* the same for any-hit waves */
 #endif
 #ifndef BF_SHADOW_WAVES_PER_SIMD
 #define BF_SHADOW_WAVES_PER_SIMD 7 /* the any-hit traversal keeps less state than closest hit; 7 waves (72 VGPRs) measured fastest */
@@ -89,6 +89,9 @@ typedef struct bf_dev_tlas_leaf {
     uint32_t instance_id;
     uint32_t blas_index;
     uint32_t visibility_mask;
+    float box[6];              /* the instance's world box (its TLAS node's) */
+    uint32_t root_ref;         /* its BLAS root: wide-node index, or BF_WIDE_LEAF | leaf-triangle index */
+    uint32_t reserved;
 } bf_dev_tlas_leaf;
 
 typedef struct bf_dev_instance {
@@ -181,6 +184,8 @@ typedef struct bf_dev_scene {
     const bf_dev_image* images;
     const float* image_texels;
     const bf_surface_maps_desc* maps;
+    uint32_t exact_walk;               /* boxes or depths outside the bound engine's range: every launch
+                                        * takes the step-exact walk */
 } bf_dev_scene;
 
 /* Path-state columns (one entry per path slot). */

@@ -711,7 +711,19 @@ int build_scene(const bf_scene_desc* d, bf_hip_scene* s, bool upload) {
         L.instance_id = ir.instance_id;
         L.blas_index = ir.blas_index;
         L.visibility_mask = ir.visibility_mask;
+        std::memcpy(L.box, &tlas_leaf_boxes[6 * r], sizeof L.box);
+        L.root_ref = dev_blases[ir.blas_index].root_ref;
+        L.reserved = 0u;
     }
+    /* the bound engine's range: coordinates within 2^126 and no stack past the reference's 64 entries
+     * (a walk holds at most depth + 1 entries per structure) */
+    bool exact_walk = s->max_blas_depth >= BF_STRUCTURE_STACK || s->tlas_depth >= BF_STRUCTURE_STACK;
+    auto wide_range = [&](const bf_bvh_node& n) {
+        const float v[6] = {n.min_x, n.min_y, n.min_z, n.max_x, n.max_y, n.max_z};
+        for (float c : v) exact_walk = exact_walk || !(std::fabs(c) <= 0x1p126f);
+    };
+    for (const bf_bvh_blas& b : s->blases) wide_range(s->blas_nodes[b.root_node]);
+    wide_range(s->tlas_nodes[s->tlas_root]);
     /* -- shading tables -- */
     std::vector<bf_dev_instance> instances(d->instance_count);
     std::vector<bf_dev_geometry> geometries(d->geometry_count);
@@ -1019,6 +1031,7 @@ int build_scene(const bf_scene_desc* d, bf_hip_scene* s, bool upload) {
     S.tlas_leaves = (const bf_dev_tlas_leaf*)(base + o_leaves);
     S.tlas_root_ref = tlas_ref[s->tlas_root];
     S.instance_count = d->instance_count;
+    S.exact_walk = exact_walk ? 1u : 0u;
     const bf_bvh_node& tr = s->tlas_nodes[s->tlas_root];
     const float trb[6] = {tr.min_x, tr.min_y, tr.min_z, tr.max_x, tr.max_y, tr.max_z};
     std::memcpy(S.tlas_root_box, trb, sizeof trb);
@@ -1089,6 +1102,7 @@ struct bf_hip_workspace {
     bf_dev_job* host_jobs = nullptr;         /* pinned staging of the job table */
     uint2* spill = nullptr;                  /* traversal stack spill, BF_STACK_DEPTH x spill_lanes */
     uint32_t spill_lanes = 0;
+    uint32_t trace_lanes[3] = {0, 0, 0};
     uint32_t shade_blocks = 0, adjoint_shade_blocks = 0;
     int device = 0;
     /* a captured group of bounces, replayed while paths remain (keyed by what its arguments hold) */
@@ -1541,14 +1555,14 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     const uint64_t n = capacity;
     const uint32_t tiles = bfk_compact_tiles((uint32_t)n);
     hipError_t de = hipGetDevice(&w->device);
-    const uint32_t resident = de == hipSuccess ? bfk_trace_resident_lanes(w->device) : 0u;
+    const bool resident = de == hipSuccess && bfk_trace_resident_lanes(w->device, w->trace_lanes);
     w->shade_blocks = de == hipSuccess ? bfk_shade_resident_blocks(w->device, false) : 0u;
     w->adjoint_shade_blocks = de == hipSuccess ? bfk_shade_resident_blocks(w->device, true) : 0u;
-    if (resident == 0 || w->shade_blocks == 0 || w->adjoint_shade_blocks == 0) {
+    if (!resident || w->shade_blocks == 0 || w->adjoint_shade_blocks == 0) {
         delete w;
         return set_error(BF_DEVICE_ERROR, "cannot query the kernels' occupancy on the current device");
     }
-    w->spill_lanes = resident;
+    w->spill_lanes = std::max(w->trace_lanes[0], std::max(w->trace_lanes[1], w->trace_lanes[2]));
     Arena A;
     const size_t o_ro = A.add(nullptr, n * 16), o_rd = A.add(nullptr, n * 16), o_beta = A.add(nullptr, n * 16),
                  o_rad = A.add(nullptr, n * 16), o_wl = A.add(nullptr, n * 16), o_dep = A.add(nullptr, n * 16),
@@ -1839,6 +1853,10 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
         P.shadow_order = w->queues[1];
     }
     P.spill_stride = w->spill_lanes;
+    std::copy(w->trace_lanes, w->trace_lanes + 3, P.trace_lanes);
+    P.step_counters = w->traversal;
+    for (uint32_t j = 0; j < job_count; ++j)
+        if (jobs[j].scene->dev.exact_walk || !(inputs || jobs[j].frame.camera.t_min >= 0.0f)) P.exact_walk = 1u;
     P.shade_blocks = w->shade_blocks;
     P.adjoint_shade_blocks = w->adjoint_shade_blocks;
     const uint32_t block_log2 = (o->launch & BF_LAUNCH_TRACE_BLOCK_MASK) >> 16;

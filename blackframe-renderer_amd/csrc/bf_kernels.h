@@ -86,7 +86,10 @@ typedef struct bf_transport_params {
     float packet[4];
     uint32_t* failure;          /* [0] failed path count, [2..3] lowest (job << 48 | path << 8 | code) */
     uint2* spill;               /* traversal stack spill: BF_STACK_DEPTH entries per persistent lane */
-    uint32_t spill_stride;      /* persistent lanes = resident traversal workgroups * BF_TRACE_BLOCK */
+    uint32_t spill_stride;      /* lanes the spill area covers */
+    uint32_t trace_lanes[3];    /* resident lanes of closest-hit, shadow and counting traversal launches */
+    uint32_t exact_walk;        /* traversal launches take the step-exact walk (see bf_traversal.h) */
+    unsigned long long* step_counters; /* where such a launch counts when the caller asked for no counters */
     uint32_t shade_blocks;      /* resident forward shade workgroups (persistent grid) */
     uint32_t adjoint_shade_blocks; /* resident adjoint shade workgroups */
     uint32_t* fetch;            /* traversal work counters [closest, shadow], cleared before each launch */
@@ -137,8 +140,9 @@ hipError_t bfk_compact(const uint8_t* route, const uint32_t* count_ptr, uint32_t
 /* sizes[0..3] -> history[4 * sizes[7]], sizes[0] = sizes[3], sizes[1..5] = 0, ++sizes[7] */
 hipError_t bfk_bounce_end(uint32_t* sizes, uint32_t* history, uint32_t history_bounces, hipStream_t s);
 hipError_t bfk_film(const bf_dev_paths* paths, const bf_dev_job* job, float pdf, float normalization, hipStream_t s);
-/* Workgroups the device holds at once for the traversal / shade kernels, 0 on error. */
-uint32_t bfk_trace_resident_lanes(int device);
+/* Lanes the device holds at once for closest-hit, shadow and counting traversal; false on error. */
+bool bfk_trace_resident_lanes(int device, uint32_t* lanes);
+/* Workgroups the device holds at once for the shade kernels, 0 on error. */
 uint32_t bfk_shade_resident_blocks(int device, bool adjoint);
 hipError_t bfk_queue_hash(const uint32_t* queue, const uint32_t* count_ptr, unsigned long long* out, hipStream_t s);
 hipError_t bfk_scene_closest_hit(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "bf_paths.h"
 #include "bf_scene_soa.h"
@@ -15,85 +16,101 @@
  * taking 64 consecutive queue items at a time with a static stride, so that the per-lane stack
  * spill area is bounded by the grid and empty tail workgroups cost nothing. */
 
-/* One lane's ray between traversal steps. */
+/* One lane's ray of a counting launch between traversal steps. */
 struct lane_ray {
-    uint32_t item, slot;
-    float t_min, t_max;
+    uint32_t item, slot, status;
     trav_state ts;
     trav_hit best;
     bool occluded;
 };
 
-/* World-space ray of a slot, re-read from the path columns (closest-hit rays). `inv` (optional)
- * holds the lane's world-space reciprocals, entry k at inv[k * stride]. */
+/* One lane's ray of any other launch. */
+struct bound_ray {
+    uint32_t item, slot, status;
+    const bf_dev_scene* scene; /* batched launches: the ray's own scene */
+    bound_state ts;
+    bool occluded;
+};
+
+template <bool BATCH>
+BF_D const bf_dev_scene& scene_of(const bf_transport_params& P, const bound_ray& L) {
+    if constexpr (BATCH) return *L.scene;
+    else return P.job0.scene;
+}
+
+/* A closest-hit ray's parameter range and visibility mask. */
+BF_D void closest_range(const bf_transport_params& P, const bf_dev_job& J, uint32_t slot, float t_min, trav_ray& ray) {
+    ray.t_min = t_min;
+    ray.t_max = (P.paths.depth[slot].z & BF_FIRST_RAY) == 0u
+                    ? BF_INFINITY_F
+                    : (J.in_rays ? J.in_rays[path_of(J, slot)].t_max : J.camera.t_max);
+    ray.mask = P.paths.visibility[slot];
+}
+
+/* World-space ray of a slot, re-read from the path columns (closest-hit rays): the step-exact walk
+ * asks for (o, d) when it leaves a BLAS, the bound one for (d, mask) when it enters an instance. */
 struct closest_world {
     const bf_dev_paths* paths;
     uint32_t slot;
-    double* inv;
-    uint32_t stride;
     BF_D void operator()(v3f& o, v3f& d) const {
         const float4 a = paths->ray_origin[slot];
         const float4 b = paths->ray_direction[slot];
         o = mk(a.x, a.y, a.z);
         d = mk(b.x, b.y, b.z);
     }
+    BF_D void operator()(v3f& d, uint32_t& mask) const {
+        const float4 b = paths->ray_direction[slot];
+        d = mk(b.x, b.y, b.z);
+        mask = paths->visibility[slot];
+    }
 };
 
-BF_D void world_space(const closest_world& world, trav_space& s) {
-    world(s.o, s.d);
-    if (world.inv) {
-        s.inv[0] = world.inv[0];
-        s.inv[1] = world.inv[world.stride];
-        s.inv[2] = world.inv[2u * world.stride];
-        finish_space(s);
-    } else {
-        make_space(s.o, s.d, s);
+/* World-space shadow ray of a slot, from the pending-shadow columns. */
+struct shadow_world {
+    const bf_dev_paths* paths;
+    uint32_t slot;
+    BF_D void operator()(v3f& o, v3f& d) const {
+        const float4 a = paths->shadow_origin[slot];
+        const float4 b = paths->shadow_direction[slot];
+        o = mk(a.x, a.y, a.z);
+        d = mk(b.x, b.y, b.z);
     }
-}
+    BF_D void operator()(v3f& d, uint32_t& mask) const {
+        const float4 b = paths->shadow_direction[slot];
+        d = mk(b.x, b.y, b.z);
+        mask = paths->visibility[slot];
+    }
+};
 
-/* Starts queue item i; returns the traversal status of the root test. */
-template <bool COUNT, bool BATCH, uint32_t BLOCK>
-BF_D uint32_t closest_start(const bf_transport_params& P, const uint32_t* queue, uint32_t i,
-                            trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L, trav_counters& ctr) {
-    L.item = i;
-    L.slot = queue[i];
-    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
-    const float4 ro = P.paths.ray_origin[L.slot];
-    const float4 rd = P.paths.ray_direction[L.slot];
-    trav_ray ray;
-    ray.o = mk(ro.x, ro.y, ro.z);
-    ray.d = mk(rd.x, rd.y, rd.z);
-    ray.t_min = rd.w;
-    ray.t_max = (P.paths.depth[L.slot].z & BF_FIRST_RAY) == 0u
-                    ? BF_INFINITY_F
-                    : (J.in_rays ? J.in_rays[path_of(J, L.slot)].t_max : J.camera.t_max);
-    ray.mask = P.paths.visibility[L.slot];
-    L.t_min = ray.t_min;
-    L.t_max = ray.t_max;
-    bool occluded;
-    return traverse_begin<COUNT>(J.scene, ray, stack, L.ts, L.best, occluded, ctr);
-}
-
-template <bool COUNT, bool BATCH, uint32_t BLOCK>
-BF_D uint32_t closest_step(const bf_transport_params& P, trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L,
-                           trav_counters& ctr, double* inv) {
-    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
-    bool occluded;
-    return traverse_step<false, COUNT>(J.scene, closest_world{&P.paths, L.slot, inv, BLOCK}, stack, L.ts, L.best,
-                                       occluded, ctr);
+/* Reads queue item i's ray. */
+template <bool ANY, bool BATCH>
+BF_D const bf_dev_job& load_ray(const bf_transport_params& P, uint32_t slot, trav_ray& ray) {
+    const bf_dev_job& J = job_at<BATCH>(P, slot);
+    const float4 o = ANY ? P.paths.shadow_origin[slot] : P.paths.ray_origin[slot];
+    const float4 d = ANY ? P.paths.shadow_direction[slot] : P.paths.ray_direction[slot];
+    ray.o = mk(o.x, o.y, o.z);
+    ray.d = mk(d.x, d.y, d.z);
+    if (ANY) {
+        ray.t_min = 0.0f;
+        ray.t_max = o.w;
+        ray.mask = P.paths.visibility[slot];
+    } else {
+        closest_range(P, J, slot, d.w, ray);
+    }
+    return J;
 }
 
 /* Classifies a finished closest-hit query: hit (route 1, barycentrics re-derived for the winner),
  * miss (environment radiance, path escapes) or traversal failure. */
 template <bool BATCH>
-BF_D void closest_finish(const bf_transport_params& P, uint8_t* route, lane_ray& L, uint32_t st) {
-    const uint32_t slot = L.slot;
+BF_D void closest_finish(const bf_transport_params& P, uint8_t* route, uint32_t item, uint32_t slot, uint32_t st,
+                         trav_hit& best) {
     const bf_dev_job& J = job_at<BATCH>(P, slot);
-    trav_hit& best = L.best;
     if (st == BF_HIT_MISS && best.present) {
-        v3f o, d;
-        closest_world{&P.paths, slot, nullptr, 0u}(o, d);
-        st = closest_hit_barycentrics(J.scene, o, d, L.t_min, L.t_max, best);
+        const float4 o = P.paths.ray_origin[slot], d = P.paths.ray_direction[slot];
+        trav_ray ray;
+        closest_range(P, J, slot, d.w, ray);
+        st = closest_hit_barycentrics(J.scene, mk(o.x, o.y, o.z), mk(d.x, d.y, d.z), ray.t_min, ray.t_max, best);
     }
     uint8_t r = 0;
     if (st != BF_HIT_MISS) {
@@ -132,62 +149,100 @@ BF_D void closest_finish(const bf_transport_params& P, uint8_t* route, lane_ray&
             P.paths.status[slot] = BF_TERM_ESCAPED;
         }
     }
-    route[L.item] = r;
+    route[item] = r;
 }
 
 /*
- * The persistent lane loop shared by both traversal stages. Every lane holds one ray; a lane whose
- * ray is done stays idle until REFILL lanes of its wave are (or all are), and then the
- * wave claims that many queue items with one atomic on the launch's fetch counter. A wave
- * therefore keeps working while any ray of the queue is unclaimed instead of waiting for its
- * slowest ray before it moves on. Within a wave, an iteration steps either the lanes whose next
- * entry is an interior node or those whose next entry is a leaf (LEAF lanes), so the wave issues
- * one kind of step code at a time instead of every kind under partial masks. Every ray's
- * traversal is the same sequence of steps in any schedule, so results do not depend on it; the
- * loop ends when the counter has passed the item count and every lane of the wave is idle.
+ * The persistent lane loop shared by the traversal kernels. Every lane holds one ray; a lane whose
+ * ray is done waits until REFILL lanes of its wave do (or none is left running). Then the waiting
+ * rays are finished together and the wave claims as many queue items as it has idle lanes. A wave
+ * therefore keeps working while any ray of the queue is unclaimed, and the finishing code
+ * (barycentrics, environment lookup, shadow contribution) runs under wide masks: one lane at a
+ * time it was about a third of a launch's vector instructions.
+ *
+ * Within a wave an iteration steps either the lanes whose next entry is an interior node or those
+ * whose next entry is a leaf (once they are a LEAF-th of the running ones, or all of them), so one
+ * kind of step code is issued at a time. Every ray's traversal is the same sequence of steps in
+ * any schedule, so results do not depend on it.
+ *
+ * A launch with fewer items than its resident waves have lanes gives each wave an equal share
+ * (`quota` lanes) instead of filling the first waves: the chip's other SIMDs would be idle, and
+ * rays that share a wave wait for each other's steps.
  */
-template <uint32_t REFILL, uint32_t LEAF, typename Start, typename Step, typename Finish>
-BF_D void lane_loop(uint32_t n, uint32_t* fetch, Start start, Step step, Finish finish) {
+template <uint32_t REFILL, uint32_t LEAF, typename Claim, typename Start, typename Step, typename Finish>
+BF_D void lane_loop(uint32_t n, Claim claim, Start start, Step step, Finish finish) {
     const uint32_t lane = threadIdx.x & 63u;
-    bool active = false, exhausted = false;
+    const uint32_t quota = claim.quota, refill = (quota * REFILL + 63u) / 64u;
+    bool active = false, done = false, exhausted = false;
     for (;;) {
-        const uint64_t idle = __ballot(!active);
-        const uint32_t want = (uint32_t)__popcll(idle);
-        if (!exhausted && (want >= REFILL || want == 64u)) {
-            uint32_t base = 0u;
-            if (lane == 0u) base = atomicAdd(fetch, want);
-            base = __shfl(base, 0, 64);
-            exhausted = base >= n || n - base <= want;
+        const uint64_t running = __ballot(active);
+        const uint32_t count = (uint32_t)__popcll(running);
+        if (count == 0u || (!exhausted && count + refill <= quota)) {
+            if (done) {
+                finish();
+                done = false;
+            }
+            if (exhausted) break;
+            const uint32_t want = quota - count;
+            const uint32_t base = claim(n, want, exhausted);
             if (!active) {
-                const uint32_t i = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                if (i < n && base < n) {
-                    const uint32_t st = start(i);
-                    if (st != BF_HIT_MISS || !step.pending()) finish(st);
-                    else active = true;
+                const uint32_t rank = (uint32_t)__popcll(~running & ((1ull << lane) - 1ull));
+                if (rank < want && base < n && rank < n - base) {
+                    active = start(base + rank);
+                    done = !active;
                 }
             }
-        }
-        if (__ballot(active) == 0ull) {
-            if (exhausted) break;
             continue;
         }
-        bool go = active;
-        if (LEAF != 0u) {
-            /* one kind of step per iteration: interior nodes, unless LEAF lanes (or all
-             * active ones) have a leaf next */
-            const bool leaf = active && step.leaf_next();
-            const uint64_t leaves = __ballot(leaf);
-            const bool leaf_phase = (uint32_t)__popcll(leaves) >= LEAF || leaves == __ballot(active);
-            go = active && leaf == leaf_phase;
-        }
-        if (go) {
-            const uint32_t st = step();
-            if (st != BF_HIT_MISS || !step.pending()) {
-                finish(st);
-                active = false;
+        const bool leaf = active && step.leaf_next();
+        const uint64_t leaves = __ballot(leaf);
+        if ((uint32_t)__popcll(leaves) * LEAF >= count) {
+            if (leaf) {
+                active = step.leaf();
+                done = !active;
             }
+        } else if (active && !leaf) {
+            active = step.node();
+            done = !active;
         }
     }
+}
+
+/* Lanes each wave of a launch holds: all 64 unless the items do not fill the waves. */
+BF_D uint32_t wave_quota(uint32_t n, uint32_t waves) {
+    const uint32_t share = (n + waves - 1u) / waves;
+    return share < 1u ? 1u : (share < 64u ? share : 64u);
+}
+
+/* How a wave claims items: first its own share of the queue's head (quota items), then from the
+ * launch's work counter, one atomic per refill, until the queue is exhausted. */
+struct shared_claim {
+    uint32_t* fetch;
+    uint32_t wave, waves, quota;
+    bool opened = false;
+    BF_D uint32_t operator()(uint32_t n, uint32_t want, bool& exhausted) {
+        const uint32_t head = waves * quota;
+        uint32_t base;
+        if (!opened) {
+            opened = true;
+            base = wave * quota;
+            exhausted = head >= n;
+        } else {
+            base = 0u;
+            if ((threadIdx.x & 63u) == 0u) base = atomicAdd(fetch, want);
+            base = head + __shfl(base, 0, 64);
+            exhausted = base >= n || n - base <= want;
+        }
+        return base;
+    }
+};
+
+/* The claim of this wave, with the launch's quota. */
+template <uint32_t BLOCK>
+BF_D shared_claim wave_claim(uint32_t* fetch, uint32_t n) {
+    const uint32_t waves = gridDim.x * (BLOCK / 64u);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64u) + (threadIdx.x >> 6));
+    return shared_claim{fetch, wave, waves, wave_quota(n, waves)};
 }
 
 BF_D void reduce_counters(const trav_counters& c, unsigned long long* counters) {
@@ -204,89 +259,11 @@ BF_D void reduce_counters(const trav_counters& c, unsigned long long* counters) 
     }
 }
 
-template <bool COUNT, bool BATCH, uint32_t BLOCK>
-__global__ __launch_bounds__(BLOCK, BF_TRACE_WAVES_PER_SIMD) void k_trace_closest(bf_transport_params P, const uint32_t* queue,
-                                                                      const uint32_t* count_ptr, const uint32_t* order,
-                                                                      uint8_t* route, unsigned long long* counters) {
-    __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
-    const uint32_t n = *count_ptr;
-    trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
-                                            P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
-    trav_counters ctr{0u, 0u, 0u};
-    lane_ray L;
-    struct stepper {
-        const bf_transport_params* P;
-        trav_stack<BF_SHORT_STACK, BLOCK>* stack;
-        lane_ray* L;
-        trav_counters* ctr;
-        double* inv;
-        BF_D uint32_t operator()() const { return closest_step<COUNT, BATCH>(*P, *stack, *L, *ctr, inv); }
-        BF_D bool pending() const { return stack_depth(*stack) != 0u; }
-        BF_D bool leaf_next() const { return ::leaf_next(*stack); }
-    };
-#if BF_WORLD_INV_CACHE
-    /* the lane's world-space reciprocals, kept for the return from each BLAS */
-    __shared__ double s_inv[3 * BLOCK];
-    double* inv = s_inv + threadIdx.x;
-#else
-    double* inv = nullptr;
-#endif
-    lane_loop<BF_TRACE_REFILL, BF_LEAF_PHASE>(
-        n, P.fetch,
-        [&](uint32_t i) {
-            const uint32_t st = closest_start<COUNT, BATCH>(P, queue, order ? order[i] : i, stack, L, ctr);
-            if (inv) {
-                inv[0] = L.ts.space.inv[0];
-                inv[BLOCK] = L.ts.space.inv[1];
-                inv[2u * BLOCK] = L.ts.space.inv[2];
-            }
-            return st;
-        },
-        stepper{&P, &stack, &L, &ctr, inv}, [&](uint32_t st) { closest_finish<BATCH>(P, route, L, st); });
-    if (COUNT) reduce_counters(ctr, counters);
-}
-
-/* World-space shadow ray of a slot, re-read from the pending-shadow columns. */
-struct shadow_world {
-    const bf_dev_paths* paths;
-    uint32_t slot;
-    BF_D void operator()(v3f& o, v3f& d) const {
-        const float4 a = paths->shadow_origin[slot];
-        const float4 b = paths->shadow_direction[slot];
-        o = mk(a.x, a.y, a.z);
-        d = mk(b.x, b.y, b.z);
-    }
-};
-
-template <bool COUNT, bool BATCH, uint32_t BLOCK>
-BF_D uint32_t shadow_start(const bf_transport_params& P, const uint32_t* queue, uint32_t i,
-                           trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L, trav_counters& ctr) {
-    L.item = i;
-    L.slot = queue[i];
-    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
-    const float4 so = P.paths.shadow_origin[L.slot];
-    const float4 sd = P.paths.shadow_direction[L.slot];
-    trav_ray ray;
-    ray.o = mk(so.x, so.y, so.z);
-    ray.d = mk(sd.x, sd.y, sd.z);
-    ray.t_min = 0.0f;
-    ray.t_max = so.w;
-    ray.mask = P.paths.visibility[L.slot];
-    return traverse_begin<COUNT>(J.scene, ray, stack, L.ts, L.best, L.occluded, ctr);
-}
-
-template <bool COUNT, bool BATCH, uint32_t BLOCK>
-BF_D uint32_t shadow_step(const bf_transport_params& P, trav_stack<BF_SHORT_STACK, BLOCK>& stack, lane_ray& L,
-                          trav_counters& ctr) {
-    const bf_dev_job& J = job_at<BATCH>(P, L.slot);
-    return traverse_step<true, COUNT>(J.scene, shadow_world{&P.paths, L.slot}, stack, L.ts, L.best, L.occluded, ctr);
-}
-
 /* process_shadow (:4772-4908): the frozen contribution is added when the light is visible (and the
  * vertex's tape bit set), then the path continues or ends with its pending termination. */
 template <bool BATCH>
-BF_D void shadow_finish(const bf_transport_params& P, uint8_t* route, lane_ray& L, uint32_t st) {
-    const uint32_t slot = L.slot;
+BF_D void shadow_finish(const bf_transport_params& P, uint8_t* route, uint32_t item, uint32_t slot, uint32_t st,
+                        bool occluded) {
     const bf_dev_job& J = job_at<BATCH>(P, slot);
     const uint32_t packed = __float_as_uint(P.paths.shadow_direction[slot].w);
     uint8_t r = 0;
@@ -294,7 +271,7 @@ BF_D void shadow_finish(const bf_transport_params& P, uint8_t* route, lane_ray& 
         fail_path(P, J, slot, 40);
     } else {
         bool ok = true;
-        if (!L.occluded) {
+        if (!occluded) {
             if (J.tape_visibility) J.tape_visibility[path_of(J, slot)] |= 1ull << ((packed >> 16) & 63u);
             const float4 c = P.paths.shadow_contribution[slot];
             float4 Lr = P.paths.radiance[slot];
@@ -315,33 +292,105 @@ BF_D void shadow_finish(const bf_transport_params& P, uint8_t* route, lane_ray& 
             else P.paths.status[slot] = (packed >> 8) & 0xFFu;
         }
     }
-    route[L.item] = r;
+    route[item] = r;
 }
 
-/* ---- shadow stage: gather + any-hit + process_shadow (:4729-4908) ---------------------------- */
-template <bool COUNT, bool BATCH, uint32_t BLOCK>
-__global__ __launch_bounds__(BLOCK, BF_SHADOW_WAVES_PER_SIMD) void k_trace_shadow(bf_transport_params P, const uint32_t* queue,
-                                                                          const uint32_t* count_ptr, const uint32_t* order,
-                                                                          uint8_t* route, unsigned long long* counters) {
+/* ---- closest-hit and shadow stages: gather + traversal + finish ------------------------------
+ * The step-exact, counting launch. */
+template <bool ANY, bool BATCH, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK, BF_COUNT_WAVES_PER_SIMD) void k_trace_counting(bf_transport_params P, const uint32_t* queue,
+                                                                       const uint32_t* count_ptr, const uint32_t* order,
+                                                                       uint8_t* route, unsigned long long* counters) {
     __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
     const uint32_t n = *count_ptr;
     trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
                                             P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
     trav_counters ctr{0u, 0u, 0u};
     lane_ray L;
+    using world_t = std::conditional_t<ANY, shadow_world, closest_world>;
     struct stepper {
         const bf_transport_params* P;
         trav_stack<BF_SHORT_STACK, BLOCK>* stack;
         lane_ray* L;
         trav_counters* ctr;
-        BF_D uint32_t operator()() const { return shadow_step<COUNT, BATCH>(*P, *stack, *L, *ctr); }
-        BF_D bool pending() const { return stack_depth(*stack) != 0u; }
-        BF_D bool leaf_next() const { return ::leaf_next(*stack); }
+        BF_D bool leaf_next() const { return false; } /* nodes and leaves share one step */
+        BF_D bool leaf() const { return false; }
+        BF_D bool node() const {
+            L->status = traverse_step<ANY, true>(job_at<BATCH>(*P, L->slot).scene, world_t{&P->paths, L->slot}, *stack,
+                                                 L->ts, L->best, L->occluded, *ctr);
+            return L->status == BF_HIT_MISS && stack_depth(*stack) != 0u;
+        }
     };
-    lane_loop<BF_SHADOW_REFILL, BF_SHADOW_LEAF_PHASE>(
-        n, P.fetch + 1, [&](uint32_t i) { return shadow_start<COUNT, BATCH>(P, queue, order ? order[i] : i, stack, L, ctr); },
-        stepper{&P, &stack, &L, &ctr}, [&](uint32_t st) { shadow_finish<BATCH>(P, route, L, st); });
-    if (COUNT) reduce_counters(ctr, counters + 3);
+    lane_loop<24u, 4u>(
+        n, wave_claim<BLOCK>(P.fetch + (ANY ? 1 : 0), n),
+        [&](uint32_t i) {
+            L.item = order ? order[i] : i;
+            L.slot = queue[L.item];
+            trav_ray ray;
+            const bf_dev_job& J = load_ray<ANY, BATCH>(P, L.slot, ray);
+            L.status = traverse_begin<true>(J.scene, ray, stack, L.ts, L.best, L.occluded, ctr);
+            return L.status == BF_HIT_MISS && stack_depth(stack) != 0u;
+        },
+        stepper{&P, &stack, &L, &ctr},
+        [&] {
+            if constexpr (ANY) shadow_finish<BATCH>(P, route, L.item, L.slot, L.status, L.occluded);
+            else closest_finish<BATCH>(P, route, L.item, L.slot, L.status, L.best);
+        });
+    reduce_counters(ctr, counters + (ANY ? 3 : 0));
+}
+
+/* The launch every render takes: the walk on binary32 bounds. Bound by vector issue under
+ * divergence. */
+template <bool ANY, bool BATCH, uint32_t BLOCK>
+__global__ __launch_bounds__(BLOCK, ANY ? BF_SHADOW_WAVES_PER_SIMD : BF_TRACE_WAVES_PER_SIMD) void k_trace(
+    bf_transport_params P, const uint32_t* queue, const uint32_t* count_ptr, const uint32_t* order, uint8_t* route) {
+    __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
+    __shared__ float s_world[6 * BLOCK];
+    const uint32_t n = *count_ptr;
+    trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
+                                            P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
+    bound_ray L;
+    using world_t = std::conditional_t<ANY, shadow_world, closest_world>;
+    struct stepper {
+        const bf_transport_params* P;
+        trav_stack<BF_SHORT_STACK, BLOCK>* stack;
+        bound_ray* L;
+        const float* cache;
+        BF_D bool leaf_next() const { return (L->ts.cur & BF_WIDE_LEAF) != 0u; }
+        BF_D bool node() const {
+            bound_node<ANY>(scene_of<BATCH>(*P, *L), world_t{&P->paths, L->slot}, *stack, L->ts, cache, BLOCK);
+            return L->ts.cur != BF_TRAV_DONE;
+        }
+        BF_D bool leaf() const {
+            L->status = bound_leaf<ANY>(scene_of<BATCH>(*P, *L), world_t{&P->paths, L->slot}, *stack, L->ts, L->occluded,
+                                        cache, BLOCK);
+            return L->status == BF_HIT_MISS && L->ts.cur != BF_TRAV_DONE;
+        }
+    };
+    float* cache = s_world + threadIdx.x;
+    lane_loop<ANY ? BF_SHADOW_REFILL : BF_TRACE_REFILL, ANY ? BF_SHADOW_LEAF_PHASE : BF_LEAF_PHASE>(
+        n, wave_claim<BLOCK>(P.fetch + (ANY ? 1 : 0), n),
+        [&](uint32_t i) {
+            L.item = order ? order[i] : i;
+            L.slot = queue[L.item];
+            L.status = BF_HIT_MISS;
+            L.occluded = false;
+            trav_ray ray;
+            const bf_dev_job& J = load_ray<ANY, BATCH>(P, L.slot, ray);
+            L.scene = &J.scene;
+            bound_begin(J.scene, ray.o, ray.d, ray.t_min, ray.t_max, stack, L.ts, cache, BLOCK);
+            return L.ts.cur != BF_TRAV_DONE;
+        },
+        stepper{&P, &stack, &L, cache},
+        [&] {
+            if constexpr (ANY) {
+                shadow_finish<BATCH>(P, route, L.item, L.slot, L.status, L.occluded);
+            } else {
+                trav_hit best;
+                bound_result(scene_of<BATCH>(P, L), L.ts, best);
+                closest_finish<BATCH>(P, route, L.item, L.slot, L.status, best);
+            }
+        });
 }
 
 /* ---- stand-alone traversal (blackframe_hip_launch_scene_closest_hit / _occlusion) ----------- */
@@ -822,61 +871,50 @@ __global__ __launch_bounds__(BF_API_BLOCK) void k_blob_traverse(const uint8_t* s
     }
 }
 
-/* Workgroups of one persistent traversal launch: enough to fill every CU at the kernels'
- * occupancy, never more than the workspace's spill area covers, and no more than the items need. */
-static uint32_t trace_blocks(const bf_transport_params* P, uint32_t max_count, uint32_t block) {
-    const uint32_t needed = blocks_for((max_count + 63u) / 64u * 64u, block);
-    const uint32_t resident = P->spill_stride / block;
+/* Workgroups of one persistent traversal launch of a kind (0 closest hit, 1 shadow, 2 counting): as
+ * many as the device holds at once, and no more than one wave per `wave_rays` items. */
+static uint32_t trace_blocks(const bf_transport_params* P, uint32_t max_count, uint32_t block, uint32_t wave_rays,
+                             uint32_t kind) {
+    const uint32_t needed = blocks_for(blocks_for(max_count, wave_rays), block / 64u);
+    const uint32_t resident = P->trace_lanes[kind] / block;
     return needed < resident ? needed : resident;
 }
 
-template <bool ANY, bool COUNT, bool BATCH, uint32_t BLOCK>
+template <bool ANY, bool BATCH, uint32_t BLOCK>
 static void launch_trace(const bf_transport_params* P, uint32_t max_count, const uint32_t* q, const uint32_t* n,
-                         uint8_t* route, unsigned long long* counters, hipStream_t s) {
-    const dim3 grid(trace_blocks(P, max_count, BLOCK));
+                         uint8_t* route, unsigned long long* counters, bool exact, hipStream_t s) {
     (void)bfk_set_words(P->fetch + (ANY ? 1 : 0), 1u, 0u, s);
     /* optional direction-octant order; the route bytes are free until the traversal writes them */
     uint32_t* order = ANY ? P->shadow_order : P->closest_order;
     if (order)
         bfk_work_order(P, ANY ? BF_KEY_SHADOW : BF_KEY_RAY, q, n, max_count, route, order, BATCH, s);
-    if (ANY)
-        hipLaunchKernelGGL((k_trace_shadow<COUNT, BATCH, BLOCK>), grid, dim3(BLOCK), 0, s, *P, q, n, order, route, counters);
+    if (exact)
+        hipLaunchKernelGGL((k_trace_counting<ANY, BATCH, BLOCK>), dim3(trace_blocks(P, max_count, BLOCK, 64u, 2u)),
+                           dim3(BLOCK), 0, s, *P, q, n, order, route, counters);
     else
-        hipLaunchKernelGGL((k_trace_closest<COUNT, BATCH, BLOCK>), grid, dim3(BLOCK), 0, s, *P, q, n, order, route, counters);
+        hipLaunchKernelGGL((k_trace<ANY, BATCH, BLOCK>), dim3(trace_blocks(P, max_count, BLOCK, 4u, ANY ? 1u : 0u)),
+                           dim3(BLOCK), 0, s, *P, q, n, order, route);
 }
 
-template <bool ANY, bool COUNT, bool BATCH>
+template <bool ANY, bool BATCH>
 static void launch_trace_block(const bf_transport_params* P, uint32_t max_count, const uint32_t* q, const uint32_t* n,
-                               uint8_t* route, unsigned long long* counters, hipStream_t s) {
-    if (P->trace_block == 64u) launch_trace<ANY, COUNT, BATCH, 64u>(P, max_count, q, n, route, counters, s);
-    else if (P->trace_block == 256u) launch_trace<ANY, COUNT, BATCH, 256u>(P, max_count, q, n, route, counters, s);
-    else launch_trace<ANY, COUNT, BATCH, 128u>(P, max_count, q, n, route, counters, s);
+                               uint8_t* route, unsigned long long* counters, bool exact, hipStream_t s) {
+    if (P->trace_block == 64u) launch_trace<ANY, BATCH, 64u>(P, max_count, q, n, route, counters, exact, s);
+    else if (P->trace_block == 256u) launch_trace<ANY, BATCH, 256u>(P, max_count, q, n, route, counters, exact, s);
+    else launch_trace<ANY, BATCH, 128u>(P, max_count, q, n, route, counters, exact, s);
 }
 
+/* Counted launches, and frames outside the bound engine's range (P->exact_walk), take the step-exact
+ * walk; its counts go to the workspace's own counters when the caller asked for none. */
 template <bool ANY>
 static hipError_t trace_stage(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr,
                               uint32_t max_count, uint8_t* route, unsigned long long* counters, bool batch, hipStream_t s) {
     if (max_count == 0) return hipSuccess;
-    if (counters) {
-        if (batch) launch_trace_block<ANY, true, true>(P, max_count, queue, count_ptr, route, counters, s);
-        else launch_trace_block<ANY, true, false>(P, max_count, queue, count_ptr, route, counters, s);
-    } else {
-        if (batch) launch_trace_block<ANY, false, true>(P, max_count, queue, count_ptr, route, counters, s);
-        else launch_trace_block<ANY, false, false>(P, max_count, queue, count_ptr, route, counters, s);
-    }
+    const bool exact = counters != nullptr || P->exact_walk != 0u;
+    if (!counters) counters = P->step_counters;
+    if (batch) launch_trace_block<ANY, true>(P, max_count, queue, count_ptr, route, counters, exact, s);
+    else launch_trace_block<ANY, false>(P, max_count, queue, count_ptr, route, counters, exact, s);
     return hipGetLastError();
-}
-
-template <uint32_t BLOCK>
-static void trace_kernels(const void** out) {
-    out[0] = (const void*)k_trace_closest<false, false, BLOCK>;
-    out[1] = (const void*)k_trace_closest<true, false, BLOCK>;
-    out[2] = (const void*)k_trace_closest<false, true, BLOCK>;
-    out[3] = (const void*)k_trace_closest<true, true, BLOCK>;
-    out[4] = (const void*)k_trace_shadow<false, false, BLOCK>;
-    out[5] = (const void*)k_trace_shadow<true, false, BLOCK>;
-    out[6] = (const void*)k_trace_shadow<false, true, BLOCK>;
-    out[7] = (const void*)k_trace_shadow<true, true, BLOCK>;
 }
 
 extern "C" {
@@ -891,20 +929,31 @@ hipError_t bfk_trace_shadow(const bf_transport_params* P, const uint32_t* queue,
     return trace_stage<true>(P, queue, count_ptr, max_count, route, counters, batch, s);
 }
 
-/* Lanes the device holds at once for the widest-resident traversal kernel variant: the width of
- * the spill area, one column per lane. */
-uint32_t bfk_trace_resident_lanes(int device) {
-    const void* k64[8];
-    const void* k128[8];
-    const void* k256[8];
-    trace_kernels<64u>(k64);
-    trace_kernels<128u>(k128);
-    trace_kernels<256u>(k256);
-    const uint32_t a = (uint32_t)bfk_max_resident(k64, 8, 64u, device) * 64u;
-    const uint32_t b = (uint32_t)bfk_max_resident(k128, 8, 128u, device) * 128u;
-    const uint32_t c = (uint32_t)bfk_max_resident(k256, 8, 256u, device) * 256u;
-    if (a == 0 || b == 0 || c == 0) return 0;
-    return std::max(a, std::max(b, c));
+} /* extern "C" */
+
+/* Lanes the device holds at once for each kind of traversal launch (0 closest hit, 1 shadow, 2
+ * counting), the least over its workgroup sizes so that a grid of that many is resident in each;
+ * false on error. */
+template <uint32_t BLOCK>
+static void trace_lanes_of(int device, uint32_t* lanes) {
+    const void* kernels[8] = {(const void*)k_trace<false, false, BLOCK>,         (const void*)k_trace<false, true, BLOCK>,
+                              (const void*)k_trace<true, false, BLOCK>,          (const void*)k_trace<true, true, BLOCK>,
+                              (const void*)k_trace_counting<false, false, BLOCK>, (const void*)k_trace_counting<false, true, BLOCK>,
+                              (const void*)k_trace_counting<true, false, BLOCK>, (const void*)k_trace_counting<true, true, BLOCK>};
+    for (int k = 0; k < 8; ++k) {
+        uint32_t& kind = lanes[std::min(k / 2, 2)];
+        kind = std::min(kind, (uint32_t)bfk_max_resident(kernels + k, 1, BLOCK, device) * BLOCK);
+    }
+}
+
+extern "C" {
+
+bool bfk_trace_resident_lanes(int device, uint32_t* lanes) {
+    for (int k = 0; k < 3; ++k) lanes[k] = 0xFFFFFFFFu;
+    trace_lanes_of<64u>(device, lanes);
+    trace_lanes_of<128u>(device, lanes);
+    trace_lanes_of<256u>(device, lanes);
+    return lanes[0] != 0u && lanes[1] != 0u && lanes[2] != 0u;
 }
 
 hipError_t bfk_scene_closest_hit(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,

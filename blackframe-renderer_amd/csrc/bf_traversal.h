@@ -496,12 +496,6 @@ BF_D void world_space(const WorldRay& world, trav_space& s) {
     make_space(o, d, s);
 }
 
-/* True when the next step pops a leaf (a triangle or an instance) rather than an interior node. */
-template <uint32_t S, uint32_t LANES>
-BF_D bool leaf_next(const trav_stack<S, LANES>& s) {
-    return s.sp != 0u && (s.lds[(s.sp - 1u) * LANES].x & BF_WIDE_LEAF) != 0u;
-}
-
 /* Loop state of one ray's traversal between steps (the stack lives in trav_stack). */
 struct trav_state {
     trav_space space;
@@ -679,6 +673,355 @@ BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, WorldRay wor
     uint32_t st = traverse_begin<COUNT>(S_, ray, stack, ts, best, occluded, ctr);
     while (st == BF_HIT_MISS && stack_depth(stack) != 0u) st = traverse_step<ANY, COUNT>(S_, world, stack, ts, best, occluded, ctr);
     return st;
+}
+
+/* ---- traversal on binary32 bounds ------------------------------------------------------------
+ * The engine of every launch that does not count its steps. It returns the reference's result bit
+ * for bit with far fewer operations per step than the step-exact walk above, because the exact
+ * binary64 decisions are only needed where they can reach the result:
+ *
+ *  - A box is tested with binary32 bounds that never reject what the binary64 test accepts, so the
+ *    walk enters a superset of the reference's nodes. A triangle's ancestors contain its box, and
+ *    the binary64 plane distances are monotone in the plane, so a triangle the reference reaches is
+ *    exactly one whose own box passes the binary64 test against [t_min, current t], inside an
+ *    instance whose world box passed when it was popped. Both are decided exactly: the instance's
+ *    when it is entered, the triangle's only when its test reports a hit or a failure (a
+ *    triangle's box is the bounds of the vertices already in registers). Most triangle tests miss
+ *    and never ask.
+ *  - The order of two siblings is the reference's: RN32 of their binary64 near values, ties to the
+ *    first. Bounds decide it unless they overlap; then equal planes (a tie), and last binary64.
+ *
+ * Error of the bounds: q~ = RN(RN(plane - o) * RN(1 / d)) is within 3u (u = 2^-24) of the exact
+ * quotient plus at most 2^-149 of underflow, the binary64 quotient and its one-ulp widening add
+ * less than 2^-51 relative, and x -> x (1 +- 4u) is monotone, so the bound carries over to the
+ * maximum of near and the minimum of far distances. BF_SLAB_REL = 8u and BF_SLAB_ABS leave room
+ * for the rounding of the comparisons themselves. An axis the ray does not move along has
+ * RN(1 / d) = +-inf: its near and far quotients are -inf and +inf inside the slab, (+inf, +inf) or
+ * (-inf, -inf) outside, NaN on a plane, which fmaxf / fminf ignore. A space whose numbers leave
+ * the range of this analysis (subnormal or huge direction components, origins past 2^126) gets NaN
+ * reciprocals: every box is then entered and every order decided in binary64.
+ *
+ * The launchers use this engine where the boxes' coordinates stay within 2^126, no stack can
+ * overflow the reference's 64 entries (both checked when the scene is built) and t_min >= 0;
+ * counting launches and everything else take the step-exact walk. */
+#define BF_SLAB_REL 0x1p-21f
+#define BF_SLAB_ABS 0x1p-120f
+#define BF_TRAV_DONE 0xFFFFFFFFu /* no next reference: the ray is done */
+
+struct bound_state {
+    v3f o, inv, d;     /* the current space; d is kept for BLAS spaces only */
+    float t_min, t;    /* t: the closest hit so far (any-hit: t_max) */
+    uint32_t cur;      /* next reference: node, or BF_WIDE_LEAF | leaf */
+    uint32_t base;     /* stack entries below the current structure */
+    uint32_t tleaf;    /* TLAS leaf of the instance being walked, BF_INVALID_INDEX in the TLAS */
+    uint32_t hit_tleaf, hit_leaf; /* the closest hit: TLAS leaf and triangle */
+    const bf_wide_node* nodes;
+};
+
+/* Binary32 reciprocals of a direction, or NaN where the bounds do not hold. */
+BF_D v3f bound_reciprocals(v3f o, v3f d) {
+    const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
+    const float c = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
+    const bool tiny = (fabsf(d.x) < 0x1p-126f && d.x != 0.0f) || (fabsf(d.y) < 0x1p-126f && d.y != 0.0f) ||
+                      (fabsf(d.z) < 0x1p-126f && d.z != 0.0f);
+    v3f inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    if (tiny || !(m <= 0x1p126f) || !(c <= 0x1p126f)) inv.x = inv.y = inv.z = __builtin_nanf("");
+    return inv;
+}
+
+/* The binary64 verdict on a box against [t_min, t]: the reference's push and pop tests together. */
+BF_D bool box_visited_exact(v3f lo, v3f hi, v3f o, v3f d, float t_min, float t) {
+    trav_space s;
+    make_space(o, d, s);
+    bool hit = false;
+    double near_value = 0.0;
+    (void)slab_exact(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, s, t_min, t, hit, near_value);
+    return hit && near_value <= (double)t;
+}
+
+/* True when the binary64 test certainly passes: every near bound at or below every other axis's
+ * far bound (an axis's own near never exceeds its far), and the near bounds at or below t. */
+BF_D bool box_visited_certain(v3f lo, v3f hi, v3f o, v3f inv, float t_min, float t) {
+    const bool sx = inv.x < 0.0f, sy = inv.y < 0.0f, sz = inv.z < 0.0f;
+    const float nx = fmaxf(((sx ? hi.x : lo.x) - o.x) * inv.x, -3.402823466e38f);
+    const float ny = fmaxf(((sy ? hi.y : lo.y) - o.y) * inv.y, -3.402823466e38f);
+    const float nz = fmaxf(((sz ? hi.z : lo.z) - o.z) * inv.z, -3.402823466e38f);
+    const float fx = fminf(((sx ? lo.x : hi.x) - o.x) * inv.x, 3.402823466e38f);
+    const float fy = fminf(((sy ? lo.y : hi.y) - o.y) * inv.y, 3.402823466e38f);
+    const float fz = fminf(((sz ? lo.z : hi.z) - o.z) * inv.z, 3.402823466e38f);
+    const float ux = fmaf(fabsf(nx), BF_SLAB_REL, nx) + BF_SLAB_ABS;
+    const float uy = fmaf(fabsf(ny), BF_SLAB_REL, ny) + BF_SLAB_ABS;
+    const float uz = fmaf(fabsf(nz), BF_SLAB_REL, nz) + BF_SLAB_ABS;
+    const float wx = fmaf(fabsf(fx), -BF_SLAB_REL, fx) - BF_SLAB_ABS;
+    const float wy = fmaf(fabsf(fy), -BF_SLAB_REL, fy) - BF_SLAB_ABS;
+    const float wz = fmaf(fabsf(fz), -BF_SLAB_REL, fz) - BF_SLAB_ABS;
+    return !bf_isnan(inv.x) && ux <= fminf(wy, wz) && uy <= fminf(wx, wz) && uz <= fminf(wx, wy) &&
+           fmaxf(fmaxf(ux, uy), uz) <= t && t_min <= fminf(fminf(wx, wy), wz) && t_min <= t;
+}
+
+/* near_exact of a node's child k, its planes given */
+BF_D double child_near_exact(v3f n, const trav_space& s, float t_min) {
+    double v = (double)t_min;
+    if (s.d.x != 0.0f) v = fmax(v, bf_next_down(quotient((double)n.x - (double)s.o.x, (double)s.d.x, s.inv[0])));
+    if (s.d.y != 0.0f) v = fmax(v, bf_next_down(quotient((double)n.y - (double)s.o.y, (double)s.d.y, s.inv[1])));
+    if (s.d.z != 0.0f) v = fmax(v, bf_next_down(quotient((double)n.z - (double)s.o.z, (double)s.d.z, s.inv[2])));
+    return v;
+}
+
+/* Next entry of the stack that can still hold a closer hit; leaves the BLAS when it is empty.
+ * `cache` holds the lane's world-space o and 1/d, six floats with the given stride. */
+template <bool ANY, uint32_t S, uint32_t LANES>
+BF_D void bound_pop(const bf_dev_scene& S_, trav_stack<S, LANES>& stack, bound_state& ts, const float* cache,
+                    uint32_t stride) {
+    for (;;) {
+        if (stack_depth(stack) <= ts.base) {
+            if (ts.tleaf == BF_INVALID_INDEX) {
+                ts.cur = BF_TRAV_DONE;
+                return;
+            }
+            ts.o = mk(cache[0], cache[stride], cache[2u * stride]);
+            ts.inv = mk(cache[3u * stride], cache[4u * stride], cache[5u * stride]);
+            ts.nodes = S_.tlas_nodes;
+            ts.tleaf = BF_INVALID_INDEX;
+            ts.base = 0u;
+            continue;
+        }
+        const uint2 e = stack_pop(stack);
+        if (ANY || !(__uint_as_float(e.y) > ts.t)) {
+            ts.cur = e.x;
+            return;
+        }
+    }
+}
+
+/* Starts a ray (its world-space o and 1/d go to the lane's cache). */
+template <uint32_t S, uint32_t LANES>
+BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t_max, trav_stack<S, LANES>& stack,
+                      bound_state& ts, float* cache, uint32_t stride) {
+    stack.sp = 0u;
+    stack.gsp = 0u;
+    ts.o = o;
+    ts.inv = bound_reciprocals(o, d);
+    cache[0] = o.x;
+    cache[stride] = o.y;
+    cache[2u * stride] = o.z;
+    cache[3u * stride] = ts.inv.x;
+    cache[4u * stride] = ts.inv.y;
+    cache[5u * stride] = ts.inv.z;
+    ts.t_min = t_min;
+    ts.t = t_max;
+    ts.base = 0u;
+    ts.tleaf = BF_INVALID_INDEX;
+    ts.hit_leaf = BF_INVALID_INDEX;
+    ts.hit_tleaf = BF_INVALID_INDEX;
+    ts.nodes = S_.tlas_nodes;
+    ts.cur = S_.tlas_root_ref; /* BF_INVALID_INDEX (no instances) is BF_TRAV_DONE */
+}
+
+/* The two child boxes of node ts.cur: the near child becomes ts.cur, the far one is pushed. */
+template <bool ANY, uint32_t S, uint32_t LANES, typename WorldRay>
+BF_D void bound_node(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES>& stack, bound_state& ts,
+                     const float* cache, uint32_t stride) {
+    const float4* p = reinterpret_cast<const float4*>(ts.nodes + ts.cur);
+    const float4 a = p[0], b = p[1], c = p[2];
+    const uint2 child = *reinterpret_cast<const uint2*>(p + 3);
+    const bool sx = ts.inv.x < 0.0f, sy = ts.inv.y < 0.0f, sz = ts.inv.z < 0.0f;
+    /* a: lo_x lo_y, b: lo_z hi_x, c: hi_y hi_z, each for both children */
+    const v3f n0 = mk(sx ? b.z : a.x, sy ? c.x : a.z, sz ? c.z : b.x);
+    const v3f n1 = mk(sx ? b.w : a.y, sy ? c.y : a.w, sz ? c.w : b.y);
+    const v3f f0 = mk(sx ? a.x : b.z, sy ? a.z : c.x, sz ? b.x : c.z);
+    const v3f f1 = mk(sx ? a.y : b.w, sy ? a.w : c.y, sz ? b.y : c.w);
+    const v3f q0 = mk((n0.x - ts.o.x) * ts.inv.x, (n0.y - ts.o.y) * ts.inv.y, (n0.z - ts.o.z) * ts.inv.z);
+    const v3f q1 = mk((n1.x - ts.o.x) * ts.inv.x, (n1.y - ts.o.y) * ts.inv.y, (n1.z - ts.o.z) * ts.inv.z);
+    const v3f r0 = mk((f0.x - ts.o.x) * ts.inv.x, (f0.y - ts.o.y) * ts.inv.y, (f0.z - ts.o.z) * ts.inv.z);
+    const v3f r1 = mk((f1.x - ts.o.x) * ts.inv.x, (f1.y - ts.o.y) * ts.inv.y, (f1.z - ts.o.z) * ts.inv.z);
+    const float nv0 = fmaxf(fmaxf(fmaxf(q0.x, q0.y), q0.z), ts.t_min);
+    const float nv1 = fmaxf(fmaxf(fmaxf(q1.x, q1.y), q1.z), ts.t_min);
+    const float fv0 = fminf(fminf(fminf(r0.x, r0.y), r0.z), ts.t);
+    const float fv1 = fminf(fminf(fminf(r1.x, r1.y), r1.z), ts.t);
+    const float lo0 = fmaf(nv0, 1.0f - BF_SLAB_REL, -BF_SLAB_ABS);
+    const float lo1 = fmaf(nv1, 1.0f - BF_SLAB_REL, -BF_SLAB_ABS);
+    const bool h0 = !(lo0 > fmaf(fv0, 1.0f + BF_SLAB_REL, BF_SLAB_ABS));
+    const bool h1 = !(lo1 > fmaf(fv1, 1.0f + BF_SLAB_REL, BF_SLAB_ABS));
+    if (h0 && h1) {
+        const float lead = nv1 - nv0, band = fmaf(nv0 + nv1, BF_SLAB_REL, 4.0f * BF_SLAB_ABS);
+        bool first_near = lead > 0.0f;
+        if (!(fabsf(lead) > band)) {
+            /* a tie when each axis has equal near planes or lies below both near values */
+            const float below = fmaf(fminf(nv0, nv1), 1.0f - 2.0f * BF_SLAB_REL, -4.0f * BF_SLAB_ABS);
+            const float up = 1.0f + BF_SLAB_REL;
+            const bool tie = (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
+                             (n0.y == n1.y || fmaxf(q0.y, q1.y) * up < below) &&
+                             (n0.z == n1.z || fmaxf(q0.z, q1.z) * up < below);
+            first_near = true;
+            if (!tie) {
+                v3f d = ts.d;
+                uint32_t mask;
+                if (ts.tleaf == BF_INVALID_INDEX) world(d, mask);
+                trav_space s;
+                make_space(ts.o, d, s);
+                /* the near planes by the direction's own signs (the reciprocals may be NaN) */
+                const bool ex = (d.x < 0.0f) != sx, ey = (d.y < 0.0f) != sy, ez = (d.z < 0.0f) != sz;
+                const v3f m0 = mk(ex ? f0.x : n0.x, ey ? f0.y : n0.y, ez ? f0.z : n0.z);
+                const v3f m1 = mk(ex ? f1.x : n1.x, ey ? f1.y : n1.y, ez ? f1.z : n1.z);
+                first_near = (float)child_near_exact(m0, s, ts.t_min) <= (float)child_near_exact(m1, s, ts.t_min);
+            }
+        }
+        stack_push(stack, make_uint2(first_near ? child.y : child.x, __float_as_uint(first_near ? lo1 : lo0)));
+        ts.cur = first_near ? child.x : child.y;
+    } else if (h0 || h1) {
+        ts.cur = h0 ? child.x : child.y;
+    } else {
+        bound_pop<ANY>(S_, stack, ts, cache, stride);
+    }
+}
+
+/* watertight<false> with the same verdict and t for fewer operations: non-finite terms are looked
+ * for once (an infinite or NaN input makes one of the six values non-finite), and the binary64
+ * re-decision of mixed edge signs is filtered with one bound for the three edges. */
+BF_D uint32_t watertight_bound(v3f v0, v3f v1, v3f v2, v3f o, v3f d, v3f inv, float t_min, float t_max, tri_result& r) {
+    uint32_t kz = 0u;
+    float maxd = fabsf(d.x);
+    if (fabsf(d.y) > maxd) {
+        kz = 1u;
+        maxd = fabsf(d.y);
+    }
+    if (fabsf(d.z) > maxd) kz = 2u;
+    uint32_t kx = kz == 2u ? 0u : kz + 1u;
+    uint32_t ky = kx == 2u ? 0u : kx + 1u;
+    const float dz = comp3(d, kz);
+    if (dz < 0.0f) {
+        const uint32_t t = kx;
+        kx = ky;
+        ky = t;
+    }
+    /* 1 / d_kz as the space already holds it */
+    float rz = comp3(inv, kz);
+    if (bf_isnan(rz)) rz = 1.0f / dz;
+    const float sx = comp3(d, kx) * rz, sy = comp3(d, ky) * rz;
+    const v3f t0 = sub3(v0, o), t1 = sub3(v1, o), t2 = sub3(v2, o);
+    const float t0x = comp3(t0, kx), t0y = comp3(t0, ky), t0z = comp3(t0, kz);
+    const float t1x = comp3(t1, kx), t1y = comp3(t1, ky), t1z = comp3(t1, kz);
+    const float t2x = comp3(t2, kx), t2y = comp3(t2, ky), t2z = comp3(t2, kz);
+    const float ax = fmaf(-sx, t0z, t0x), ay = fmaf(-sy, t0z, t0y);
+    const float bx = fmaf(-sx, t1z, t1x), by = fmaf(-sy, t1z, t1y);
+    const float cx = fmaf(-sx, t2z, t2x), cy = fmaf(-sy, t2z, t2y);
+    const float az = t0z * rz, bz = t1z * rz, cz = t2z * rz;
+    const float e0 = bx * cy - by * cx;
+    const float e1 = cx * ay - cy * ax;
+    const float e2 = ax * by - ay * bx;
+    if (!__builtin_isfinite(e0) || !__builtin_isfinite(e1) || !__builtin_isfinite(e2) || !__builtin_isfinite(az) ||
+        !__builtin_isfinite(bz) || !__builtin_isfinite(cz))
+        return BF_HIT_NUMERICAL_FAILURE;
+    const float emin = fminf(fminf(e0, e1), e2), emax = fmaxf(fmaxf(e0, e1), e2);
+    const bool mixed = emin < 0.0f && emax > 0.0f;
+    if (mixed) {
+        /* each sheared coordinate is within 4u of its exact value relative to |t_x| + |s t_z|, so
+         * with X and Y the largest of those sums each edge function is within 20.01u X Y of the
+         * exact one and the binary64 re-decision within 2^-49 X Y: signs certain beyond 24u X Y
+         * (and a floor for underflow) are mixed there too, and the ray misses. */
+        const float X = fmaxf(fmaxf(fmaf(fabsf(sx), fabsf(t0z), fabsf(t0x)), fmaf(fabsf(sx), fabsf(t1z), fabsf(t1x))),
+                              fmaf(fabsf(sx), fabsf(t2z), fabsf(t2x))) +
+                        0x1p-60f;
+        const float Y = fmaxf(fmaxf(fmaf(fabsf(sy), fabsf(t0z), fabsf(t0y)), fmaf(fabsf(sy), fabsf(t1z), fabsf(t1y))),
+                              fmaf(fabsf(sy), fabsf(t2z), fabsf(t2y))) +
+                        0x1p-60f;
+        const float bound = (X * Y) * (24.0f * 0x1p-24f) + 0x1p-100f;
+        if (emin < -bound && emax > bound) return BF_HIT_MISS;
+    }
+    if (mixed || emin == 0.0f || emax == 0.0f)
+        return refine_edges<false>(v0, v1, v2, o, d, kx, ky, kz, t_min, t_max, r);
+    const float det = e0 + e1 + e2;
+    if (!bf_isfinite(det)) return BF_HIT_NUMERICAL_FAILURE;
+    if (det == 0.0f) return BF_HIT_MISS;
+    const float sp = fmaf(e0, az, fmaf(e1, bz, e2 * cz));
+    if (!bf_isfinite(sp)) return BF_HIT_NUMERICAL_FAILURE;
+    const float smin = t_min * det, smax = t_max * det;
+    if (bf_isnan(smin) || bf_isnan(smax)) return BF_HIT_NUMERICAL_FAILURE;
+    if ((det > 0.0f && (sp < smin || sp > smax)) || (det < 0.0f && (sp > smin || sp < smax))) return BF_HIT_MISS;
+    const float rcp = 1.0f / det;
+    const float t = sp * rcp;
+    if (!bf_isfinite(t)) return BF_HIT_NUMERICAL_FAILURE;
+    if (t < t_min || t > t_max) return BF_HIT_MISS;
+    r.hit = true;
+    r.t = t == 0.0f ? 0.0f : t;
+    return BF_HIT_MISS;
+}
+
+/* The leaf ts.cur: an instance is entered, a triangle is tested. Returns a traversal status;
+ * `occluded` is set by an any-hit walk, whose ray is then done. */
+template <bool ANY, uint32_t S, uint32_t LANES, typename WorldRay>
+BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES>& stack, bound_state& ts,
+                         bool& occluded, const float* cache, uint32_t stride) {
+    const uint32_t leaf = ts.cur & BF_REF_MASK;
+    if (ts.tleaf == BF_INVALID_INDEX) {
+        const bf_dev_tlas_leaf& L = S_.tlas_leaves[leaf];
+        v3f d;
+        uint32_t mask;
+        world(d, mask);
+        const v3f lo = mk(L.box[0], L.box[1], L.box[2]), hi = mk(L.box[3], L.box[4], L.box[5]);
+        const v3f po = xform_point(L.world_to_local, ts.o), pd = xform_vector(L.world_to_local, d);
+        bool enter = (mask & L.visibility_mask) != 0u;
+        if (enter && !box_visited_certain(lo, hi, ts.o, ts.inv, ts.t_min, ts.t))
+            enter = box_visited_exact(lo, hi, ts.o, d, ts.t_min, ts.t);
+        if (enter) {
+            if (!fin3(po) || !fin3(pd) || (pd.x == 0.0f && pd.y == 0.0f && pd.z == 0.0f)) return BF_HIT_NUMERICAL_FAILURE;
+            ts.o = po;
+            ts.d = pd;
+            ts.inv = bound_reciprocals(po, pd);
+            ts.tleaf = leaf;
+            ts.base = stack_depth(stack);
+            ts.nodes = S_.blas_nodes;
+            ts.cur = L.root_ref;
+            return BF_HIT_MISS;
+        }
+    } else {
+        const float4 w0 = S_.leaf_triangles[3 * (size_t)leaf + 0];
+        const float4 w1 = S_.leaf_triangles[3 * (size_t)leaf + 1];
+        const float4 w2 = S_.leaf_triangles[3 * (size_t)leaf + 2];
+        const v3f v0 = mk(w0.x, w0.y, w0.z), v1 = mk(w1.x, w1.y, w1.z), v2 = mk(w2.x, w2.y, w2.z);
+        tri_result tr;
+        tr.hit = false;
+        const uint32_t st = watertight_bound(v0, v1, v2, ts.o, ts.d, ts.inv, ts.t_min, ts.t, tr);
+        if (st != BF_HIT_MISS || tr.hit) {
+            const v3f lo = mk(fminf(fminf(v0.x, v1.x), v2.x), fminf(fminf(v0.y, v1.y), v2.y), fminf(fminf(v0.z, v1.z), v2.z));
+            const v3f hi = mk(fmaxf(fmaxf(v0.x, v1.x), v2.x), fmaxf(fmaxf(v0.y, v1.y), v2.y), fmaxf(fmaxf(v0.z, v1.z), v2.z));
+            if (box_visited_certain(lo, hi, ts.o, ts.inv, ts.t_min, ts.t) ||
+                box_visited_exact(lo, hi, ts.o, ts.d, ts.t_min, ts.t)) {
+                if (st != BF_HIT_MISS) return st;
+                if (ANY) {
+                    occluded = true;
+                    ts.cur = BF_TRAV_DONE;
+                    return BF_HIT_MISS;
+                }
+                /* precedes(): by t, then instance id, then primitive */
+                bool closer = ts.hit_leaf == BF_INVALID_INDEX || tr.t < ts.t;
+                if (!closer && tr.t == ts.t) {
+                    const uint32_t i0 = S_.tlas_leaves[ts.tleaf].instance_id, i1 = S_.tlas_leaves[ts.hit_tleaf].instance_id;
+                    closer = i0 < i1 || (i0 == i1 && __float_as_uint(w0.w) <
+                                                         __float_as_uint(S_.leaf_triangles[3 * (size_t)ts.hit_leaf].w));
+                }
+                if (closer) {
+                    ts.t = tr.t;
+                    ts.hit_leaf = leaf;
+                    ts.hit_tleaf = ts.tleaf;
+                }
+            }
+        }
+    }
+    bound_pop<ANY>(S_, stack, ts, cache, stride);
+    return BF_HIT_MISS;
+}
+
+/* The closest hit of a finished walk in the form closest_hit_barycentrics takes. */
+BF_D void bound_result(const bf_dev_scene& S_, const bound_state& ts, trav_hit& best) {
+    best.present = ts.hit_leaf != BF_INVALID_INDEX;
+    if (!best.present) return;
+    best.t = ts.t;
+    best.leaf = ts.hit_leaf;
+    best.instance_id = S_.tlas_leaves[ts.hit_tleaf].instance_id;
+    best.scene_instance = S_.tlas_leaves[ts.hit_tleaf].scene_instance;
+    best.primitive = __float_as_uint(S_.leaf_triangles[3 * (size_t)ts.hit_leaf].w);
 }
 
 /* Barycentrics of the winning candidate: the triangle test is a pure function of the triangle, the
