@@ -303,8 +303,8 @@ __global__ __launch_bounds__(BLOCK, BF_COUNT_WAVES_PER_SIMD) void k_trace_counti
                                                                        uint8_t* route, unsigned long long* counters) {
     __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
     const uint32_t n = *count_ptr;
-    trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
-                                            P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
+    trav_stack<BF_SHORT_STACK, BLOCK> stack{
+        s_stack + threadIdx.x, {P.spill + blockIdx.x * BLOCK + threadIdx.x, P.spill_stride}, 0u, 0u, BF_STACK_DEPTH};
     trav_counters ctr{0u, 0u, 0u};
     lane_ray L;
     using world_t = std::conditional_t<ANY, shadow_world, closest_world>;
@@ -347,8 +347,8 @@ __global__ __launch_bounds__(BLOCK, ANY ? BF_SHADOW_WAVES_PER_SIMD : BF_TRACE_WA
     __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
     __shared__ float s_world[6 * BLOCK];
     const uint32_t n = *count_ptr;
-    trav_stack<BF_SHORT_STACK, BLOCK> stack{s_stack + threadIdx.x, P.spill + blockIdx.x * BLOCK + threadIdx.x,
-                                            P.spill_stride, 0u, 0u, BF_STACK_DEPTH};
+    trav_stack<BF_SHORT_STACK, BLOCK> stack{
+        s_stack + threadIdx.x, {P.spill + blockIdx.x * BLOCK + threadIdx.x, P.spill_stride}, 0u, 0u, BF_STACK_DEPTH};
     bound_ray L;
     using world_t = std::conditional_t<ANY, shadow_world, closest_world>;
     struct stepper {
@@ -394,66 +394,89 @@ __global__ __launch_bounds__(BLOCK, ANY ? BF_SHADOW_WAVES_PER_SIMD : BF_TRACE_WA
 }
 
 /* ---- stand-alone traversal (blackframe_hip_launch_scene_closest_hit / _occlusion) ----------- */
-/* One ray per lane with a 64-entry LDS stack and no spill area: a lane whose TLAS and BLAS entries
- * together exceed 64 reports stack overflow (the reference allows 64 per structure; a median-split
- * BVH never holds more than its depth + 1 entries per structure). */
-__global__ __launch_bounds__(BF_API_BLOCK) void k_scene_closest_hit(bf_dev_scene S, const bf_transport_ray* rays,
-                                                                    uint32_t count, bf_closest_hit_result* results,
-                                                                    uint32_t* counters) {
+/* A closest-hit record from the traversal's result. */
+BF_D void closest_record(const bf_dev_scene& S, const trav_ray& ray, uint32_t st, trav_hit& best, bf_closest_hit_result& out) {
+    memset(&out, 0, sizeof out);
+    if (st == BF_HIT_MISS && best.present) st = closest_hit_barycentrics(S, ray.o, ray.d, ray.t_min, ray.t_max, best);
+    if (st != BF_HIT_MISS) {
+        out.status = st;
+        return;
+    }
+    if (!best.present) return;
+    const bf_dev_instance& I = S.instances[best.scene_instance];
+    const float4 q0 = S.leaf_triangles[3 * (size_t)best.leaf + 0];
+    const float4 q1 = S.leaf_triangles[3 * (size_t)best.leaf + 1];
+    const float4 q2 = S.leaf_triangles[3 * (size_t)best.leaf + 2];
+    v3f n;
+    if (!world_normal(I.local_to_world, mk(q0.x, q0.y, q0.z), mk(q1.x, q1.y, q1.z), mk(q2.x, q2.y, q2.z), n)) {
+        out.status = BF_HIT_NUMERICAL_FAILURE;
+        return;
+    }
+    out.status = BF_HIT_HIT;
+    out.hit.parameter = best.t;
+    out.hit.barycentric0 = best.b0;
+    out.hit.barycentric1 = best.b1;
+    out.hit.barycentric2 = best.b2;
+    out.hit.normal_x = n.x;
+    out.hit.normal_y = n.y;
+    out.hit.normal_z = n.z;
+    out.hit.ids.object = I.object_id;
+    out.hit.ids.instance = I.id;
+    out.hit.ids.geometry = S.geometries[I.geometry_index].id;
+    out.hit.ids.primitive = best.primitive;
+    out.hit.ids.material = S.materials[I.material_index].id;
+}
+
+BF_D trav_ray api_ray(const bf_transport_ray& r) {
+    trav_ray ray;
+    ray.o = mk(r.origin_x, r.origin_y, r.origin_z);
+    ray.d = mk(r.direction_x, r.direction_y, r.direction_z);
+    ray.t_min = r.t_min;
+    ray.t_max = r.t_max;
+    ray.mask = r.visibility_mask;
+    return ray;
+}
+
+/* World-space ray of a stand-alone query (see closest_world). */
+struct api_world {
+    const bf_transport_ray* ray;
+    BF_D void operator()(v3f& o, v3f& d) const {
+        o = mk(ray->origin_x, ray->origin_y, ray->origin_z);
+        d = mk(ray->direction_x, ray->direction_y, ray->direction_z);
+    }
+    BF_D void operator()(v3f& d, uint32_t& mask) const {
+        d = mk(ray->direction_x, ray->direction_y, ray->direction_z);
+        mask = ray->visibility_mask;
+    }
+};
+
+/* The step-exact walk, for queries that count their steps and scenes outside the bound engine's
+ * range: one ray per lane with a 64-entry LDS stack and no spill area. A lane whose TLAS and BLAS
+ * entries together exceed 64 reports stack overflow (the reference allows 64 per structure; a
+ * median-split BVH never holds more than its depth + 1 entries per structure). */
+template <bool ANY>
+__global__ __launch_bounds__(BF_API_BLOCK) void k_scene_counting(bf_dev_scene S, const bf_transport_ray* rays, uint32_t count,
+                                                                 void* results, uint32_t* counters) {
     __shared__ uint2 s_stack[BF_API_STACK * BF_API_BLOCK];
-    trav_stack<BF_API_STACK, BF_API_BLOCK> stack{s_stack + threadIdx.x, nullptr, 0u, 0u, 0u, BF_API_STACK};
+    trav_stack<BF_API_STACK, BF_API_BLOCK> stack{s_stack + threadIdx.x, {nullptr, 0u}, 0u, 0u, BF_API_STACK};
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= count) return;
     const bf_transport_ray r = rays[i];
-    bf_closest_hit_result out;
-    memset(&out, 0, sizeof out);
     trav_counters ctr{0u, 0u, 0u};
-    if (!valid_traversal_ray(r)) {
-        out.status = BF_HIT_INVALID_RAY;
+    trav_hit best;
+    best.present = false;
+    bool occluded = false;
+    uint32_t st = BF_HIT_INVALID_RAY;
+    const trav_ray ray = api_ray(r);
+    if (valid_traversal_ray(r)) st = traverse<ANY, true>(S, ray, api_world{rays + i}, stack, best, occluded, ctr);
+    if constexpr (ANY) {
+        bf_occlusion_result out;
+        memset(&out, 0, sizeof out);
+        out.status = st != BF_HIT_MISS ? st : (occluded ? BF_OCCLUDED : BF_VISIBLE);
+        ((bf_occlusion_result*)results)[i] = out;
     } else {
-        trav_ray ray;
-        ray.o = mk(r.origin_x, r.origin_y, r.origin_z);
-        ray.d = mk(r.direction_x, r.direction_y, r.direction_z);
-        ray.t_min = r.t_min;
-        ray.t_max = r.t_max;
-        ray.mask = r.visibility_mask;
-        trav_hit best;
-        bool occ;
-        const auto world = [&](v3f& o, v3f& d) {
-            o = mk(rays[i].origin_x, rays[i].origin_y, rays[i].origin_z);
-            d = mk(rays[i].direction_x, rays[i].direction_y, rays[i].direction_z);
-        };
-        uint32_t st = traverse<false, true>(S, ray, world, stack, best, occ, ctr);
-        if (st == BF_HIT_MISS && best.present)
-            st = closest_hit_barycentrics(S, ray.o, ray.d, ray.t_min, ray.t_max, best);
-        if (st != BF_HIT_MISS) {
-            out.status = st;
-        } else if (best.present) {
-            const bf_dev_instance& I = S.instances[best.scene_instance];
-            const float4 q0 = S.leaf_triangles[3 * (size_t)best.leaf + 0];
-            const float4 q1 = S.leaf_triangles[3 * (size_t)best.leaf + 1];
-            const float4 q2 = S.leaf_triangles[3 * (size_t)best.leaf + 2];
-            v3f n;
-            if (!world_normal(I.local_to_world, mk(q0.x, q0.y, q0.z), mk(q1.x, q1.y, q1.z), mk(q2.x, q2.y, q2.z), n)) {
-                out.status = BF_HIT_NUMERICAL_FAILURE;
-            } else {
-                out.status = BF_HIT_HIT;
-                out.hit.parameter = best.t;
-                out.hit.barycentric0 = best.b0;
-                out.hit.barycentric1 = best.b1;
-                out.hit.barycentric2 = best.b2;
-                out.hit.normal_x = n.x;
-                out.hit.normal_y = n.y;
-                out.hit.normal_z = n.z;
-                out.hit.ids.object = I.object_id;
-                out.hit.ids.instance = I.id;
-                out.hit.ids.geometry = S.geometries[I.geometry_index].id;
-                out.hit.ids.primitive = best.primitive;
-                out.hit.ids.material = S.materials[I.material_index].id;
-            }
-        }
+        closest_record(S, ray, st, best, ((bf_closest_hit_result*)results)[i]);
     }
-    results[i] = out;
     if (counters) {
         counters[3 * (size_t)i] = ctr.nodes;
         counters[3 * (size_t)i + 1] = ctr.triangles;
@@ -461,35 +484,83 @@ __global__ __launch_bounds__(BF_API_BLOCK) void k_scene_closest_hit(bf_dev_scene
     }
 }
 
-__global__ __launch_bounds__(BF_API_BLOCK) void k_scene_occlusion(bf_dev_scene S, const bf_transport_ray* rays,
-                                                                  uint32_t count, bf_occlusion_result* results) {
-    __shared__ uint2 s_stack[BF_API_STACK * BF_API_BLOCK];
-    trav_stack<BF_API_STACK, BF_API_BLOCK> stack{s_stack + threadIdx.x, nullptr, 0u, 0u, 0u, BF_API_STACK};
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    const bf_transport_ray r = rays[i];
-    bf_occlusion_result out;
-    memset(&out, 0, sizeof out);
-    if (!valid_traversal_ray(r)) {
-        out.status = BF_HIT_INVALID_RAY;
-    } else {
-        trav_ray ray;
-        ray.o = mk(r.origin_x, r.origin_y, r.origin_z);
-        ray.d = mk(r.direction_x, r.direction_y, r.direction_z);
-        ray.t_min = r.t_min;
-        ray.t_max = r.t_max;
-        ray.mask = r.visibility_mask;
-        trav_hit best;
-        bool occ;
-        trav_counters ctr{0u, 0u, 0u};
-        const auto world = [&](v3f& o, v3f& d) {
-            o = mk(rays[i].origin_x, rays[i].origin_y, rays[i].origin_z);
-            d = mk(rays[i].direction_x, rays[i].direction_y, rays[i].direction_z);
-        };
-        const uint32_t st = traverse<true, false>(S, ray, world, stack, best, occ, ctr);
-        out.status = st != BF_HIT_MISS ? st : (occ ? BF_OCCLUDED : BF_VISIBLE);
+/* Items of one wave's own chunk of the rays, claimed without atomics. */
+struct chunk_claim {
+    uint32_t next, quota;
+    BF_D uint32_t operator()(uint32_t n, uint32_t want, bool& exhausted) {
+        const uint32_t base = next;
+        next += want;
+        exhausted = base >= n || n - base <= want;
+        return base;
     }
-    results[i] = out;
+};
+
+/* The bound walk over the caller's rays: one wave per workgroup, each with a chunk of consecutive
+ * rays that it takes through lane_loop, so that a lane whose ray is done takes the chunk's next
+ * ones. BF_SHORT_STACK entries of the stack are in LDS, the rest (deep walks only) in the lane's
+ * scratch: a full 64-entry LDS stack holds the CU to 5 waves, and this walk is bound by vector
+ * issue and latency under divergence. */
+template <bool ANY>
+__global__ __launch_bounds__(BF_API_BLOCK, BF_TRACE_WAVES_PER_SIMD) void k_scene_trace(
+    bf_dev_scene S, const bf_transport_ray* rays, uint32_t count, uint32_t chunk, void* results) {
+    __shared__ uint2 s_stack[BF_SHORT_STACK * BF_API_BLOCK];
+    __shared__ float s_world[6 * BF_API_BLOCK];
+    using stack_t = trav_stack<BF_SHORT_STACK, BF_API_BLOCK, scratch_spill>;
+    stack_t stack;
+    stack.lds = s_stack + threadIdx.x;
+    bound_state ts;
+    uint32_t item = 0u, status = BF_HIT_MISS;
+    bool occluded = false;
+    float* cache = s_world + threadIdx.x;
+    struct stepper {
+        const bf_dev_scene* S;
+        const bf_transport_ray* rays;
+        stack_t* stack;
+        bound_state* ts;
+        uint32_t *item, *status;
+        bool* occluded;
+        const float* cache;
+        BF_D bool leaf_next() const { return (ts->cur & BF_WIDE_LEAF) != 0u; }
+        BF_D bool node() const {
+            bound_node<ANY>(*S, api_world{rays + *item}, *stack, *ts, cache, BF_API_BLOCK);
+            return ts->cur != BF_TRAV_DONE;
+        }
+        BF_D bool leaf() const {
+            *status = bound_leaf<ANY>(*S, api_world{rays + *item}, *stack, *ts, *occluded, cache, BF_API_BLOCK);
+            return *status == BF_HIT_MISS && ts->cur != BF_TRAV_DONE;
+        }
+    };
+    const uint32_t begin = blockIdx.x * chunk;
+    const uint32_t end = count - begin < chunk ? count : begin + chunk;
+    lane_loop<ANY ? BF_SHADOW_REFILL : BF_TRACE_REFILL, ANY ? BF_SHADOW_LEAF_PHASE : BF_LEAF_PHASE>(
+        end, chunk_claim{begin, chunk < 64u ? chunk : 64u},
+        [&](uint32_t i) {
+            item = i;
+            status = BF_HIT_INVALID_RAY;
+            occluded = false;
+            ts.hit_leaf = BF_INVALID_INDEX;
+            const bf_transport_ray r = rays[i];
+            if (!valid_traversal_ray(r)) return false;
+            status = BF_HIT_MISS;
+            const trav_ray ray = api_ray(r);
+            bound_begin(S, ray.o, ray.d, ray.t_min, ray.t_max, stack, ts, cache, BF_API_BLOCK);
+            return ts.cur != BF_TRAV_DONE;
+        },
+        stepper{&S, rays, &stack, &ts, &item, &status, &occluded, cache},
+        [&] {
+            if constexpr (ANY) {
+                bf_occlusion_result out;
+                memset(&out, 0, sizeof out);
+                out.status = status != BF_HIT_MISS ? status : (occluded ? BF_OCCLUDED : BF_VISIBLE);
+                ((bf_occlusion_result*)results)[item] = out;
+            } else {
+                trav_hit best;
+                bound_result(S, ts, best);
+                bf_closest_hit_result out;
+                closest_record(S, api_ray(rays[item]), status, best, out);
+                ((bf_closest_hit_result*)results)[item] = out;
+            }
+        });
 }
 
 /* ---- stand-alone traversal over the reference's device blobs ----------------------------------
@@ -956,12 +1027,35 @@ bool bfk_trace_resident_lanes(int device, uint32_t* lanes) {
     return lanes[0] != 0u && lanes[1] != 0u && lanes[2] != 0u;
 }
 
+} /* extern "C" */
+
+/* Rays a wave of the bound walk takes: an equal share of one resident generation of waves (6 on
+ * each of the device's SIMDs), at most 256 so that the last waves of a large launch even out. */
+static uint32_t ray_chunk(uint32_t count) {
+    const uint32_t waves = 6u * 4u * 256u;
+    return std::min(blocks_for(count, waves), 256u);
+}
+
+template <bool ANY>
+static hipError_t scene_trace(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count, void* results,
+                              uint32_t* counters, hipStream_t s) {
+    if (count == 0) return hipSuccess;
+    if (counters || S->exact_walk) {
+        hipLaunchKernelGGL(k_scene_counting<ANY>, dim3(blocks_for(count, BF_API_BLOCK)), dim3(BF_API_BLOCK), 0, s, *S, rays,
+                           count, results, counters);
+    } else {
+        const uint32_t chunk = ray_chunk(count);
+        hipLaunchKernelGGL(k_scene_trace<ANY>, dim3(blocks_for(count, chunk)), dim3(BF_API_BLOCK), 0, s, *S, rays, count,
+                           chunk, results);
+    }
+    return hipGetLastError();
+}
+
+extern "C" {
+
 hipError_t bfk_scene_closest_hit(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
                                  bf_closest_hit_result* results, uint32_t* counters, hipStream_t s) {
-    if (count == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scene_closest_hit, dim3(blocks_for(count, BF_API_BLOCK)), dim3(BF_API_BLOCK), 0, s, *S, rays,
-                       count, results, counters);
-    return hipGetLastError();
+    return scene_trace<false>(S, rays, count, results, counters, s);
 }
 
 hipError_t bfk_blob_traverse(bool any, const uint8_t* scene_bytes, size_t scene_size, const uint8_t* bvh_bytes,
@@ -979,10 +1073,7 @@ hipError_t bfk_blob_traverse(bool any, const uint8_t* scene_bytes, size_t scene_
 
 hipError_t bfk_scene_occlusion(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
                                bf_occlusion_result* results, hipStream_t s) {
-    if (count == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scene_occlusion, dim3(blocks_for(count, BF_API_BLOCK)), dim3(BF_API_BLOCK), 0, s, *S, rays,
-                       count, results);
-    return hipGetLastError();
+    return scene_trace<true>(S, rays, count, results, nullptr, s);
 }
 
 } /* extern "C" */

@@ -441,23 +441,40 @@ BF_D bool precedes(float t, uint32_t inst, uint32_t prim, const trav_hit& c) {
  * finds them full, the lower half moves to the lane's column of a global spill area and comes
  * back when the LDS part runs empty. With S = BF_STACK_DEPTH nothing ever spills.
  */
-template <uint32_t S, uint32_t LANES>
+/* A lane's column of a global spill area. */
+struct column_spill {
+    uint2* area;
+    uint32_t stride;
+    BF_D void put(uint32_t k, uint2 e) { area[(size_t)k * stride] = e; }
+    BF_D uint2 get(uint32_t k) const { return area[(size_t)k * stride]; }
+};
+
+/* A spill area in the lane's scratch, for launches without a workspace. */
+struct scratch_spill {
+    uint32_t ref[BF_STACK_DEPTH], near_word[BF_STACK_DEPTH];
+    BF_D void put(uint32_t k, uint2 e) {
+        ref[k] = e.x;
+        near_word[k] = e.y;
+    }
+    BF_D uint2 get(uint32_t k) const { return make_uint2(ref[k], near_word[k]); }
+};
+
+template <uint32_t S, uint32_t LANES, typename Spill = column_spill>
 struct trav_stack {
     uint2* lds;             /* entry k at lds[k * LANES] (LANES = lanes of the workgroup) */
-    uint2* spill;           /* entry k at spill[k * spill_stride] */
-    uint32_t spill_stride;
+    Spill spill;
     uint32_t sp, gsp;       /* entries in LDS, entries spilled */
     uint32_t cap;           /* entries the lane may hold in all: S without a spill area */
 };
 
-template <uint32_t S, uint32_t LANES>
-BF_D uint32_t stack_depth(const trav_stack<S, LANES>& s) { return s.sp + s.gsp; }
+template <uint32_t S, uint32_t LANES, typename Spill>
+BF_D uint32_t stack_depth(const trav_stack<S, LANES, Spill>& s) { return s.sp + s.gsp; }
 
-template <uint32_t S, uint32_t LANES>
-BF_D void stack_push(trav_stack<S, LANES>& s, uint2 entry) {
+template <uint32_t S, uint32_t LANES, typename Spill>
+BF_D void stack_push(trav_stack<S, LANES, Spill>& s, uint2 entry) {
     if (S < BF_STACK_DEPTH && s.sp == S) {
 #pragma unroll
-        for (uint32_t k = 0; k < S / 2; ++k) s.spill[(size_t)(s.gsp + k) * s.spill_stride] = s.lds[k * LANES];
+        for (uint32_t k = 0; k < S / 2; ++k) s.spill.put(s.gsp + k, s.lds[k * LANES]);
 #pragma unroll
         for (uint32_t k = 0; k < S / 2; ++k) s.lds[k * LANES] = s.lds[(k + S / 2) * LANES];
         s.gsp += S / 2;
@@ -467,12 +484,12 @@ BF_D void stack_push(trav_stack<S, LANES>& s, uint2 entry) {
     ++s.sp;
 }
 
-template <uint32_t S, uint32_t LANES>
-BF_D uint2 stack_pop(trav_stack<S, LANES>& s) {
+template <uint32_t S, uint32_t LANES, typename Spill>
+BF_D uint2 stack_pop(trav_stack<S, LANES, Spill>& s) {
     if (S < BF_STACK_DEPTH && s.sp == 0u) {
         s.gsp -= S / 2;
 #pragma unroll
-        for (uint32_t k = 0; k < S / 2; ++k) s.lds[k * LANES] = s.spill[(size_t)(s.gsp + k) * s.spill_stride];
+        for (uint32_t k = 0; k < S / 2; ++k) s.lds[k * LANES] = s.spill.get(s.gsp + k);
         s.sp = S / 2;
     }
     --s.sp;
@@ -507,8 +524,8 @@ struct trav_state {
 
 /* Starts a ray: empties the stack and pushes the TLAS root when the ray meets its box. On a normal
  * return an empty stack means the ray is already done. */
-template <bool COUNT, uint32_t S, uint32_t LANES>
-BF_D uint32_t traverse_begin(const bf_dev_scene& S_, const trav_ray& ray, trav_stack<S, LANES>& stack, trav_state& ts,
+template <bool COUNT, uint32_t S, uint32_t LANES, typename Spill>
+BF_D uint32_t traverse_begin(const bf_dev_scene& S_, const trav_ray& ray, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
                              trav_hit& best, bool& occluded, trav_counters& ctr) {
     best.present = false;
     best.t = ray.t_max;
@@ -542,8 +559,8 @@ BF_D uint32_t traverse_begin(const bf_dev_scene& S_, const trav_ray& ray, trav_s
  * or a triangle). Returns a traversal status (BF_HIT_MISS = no error); the ray is done when the
  * stack is empty. `world(o, d)` re-reads the world-space ray when a BLAS is left, so that no copy
  * of it stays live between steps. */
-template <bool ANY, bool COUNT, uint32_t S, uint32_t LANES, typename WorldRay>
-BF_D uint32_t traverse_step(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES>& stack, trav_state& ts,
+template <bool ANY, bool COUNT, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
+BF_D uint32_t traverse_step(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
                             trav_hit& best, bool& occluded, trav_counters& ctr) {
     if (ts.in_blas && stack_depth(stack) <= ts.blas_base) {
         ts.in_blas = 0u;
@@ -666,8 +683,8 @@ BF_D uint32_t traverse_step(const bf_dev_scene& S_, WorldRay world, trav_stack<S
  * The winning candidate keeps (t, ids, leaf); its barycentrics are re-derived by
  * closest_hit_barycentrics from the same deterministic triangle test.
  */
-template <bool ANY, bool COUNT, uint32_t S, uint32_t LANES, typename WorldRay>
-BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, WorldRay world, trav_stack<S, LANES>& stack, trav_hit& best,
+template <bool ANY, bool COUNT, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
+BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, WorldRay world, trav_stack<S, LANES, Spill>& stack, trav_hit& best,
                        bool& occluded, trav_counters& ctr) {
     trav_state ts;
     uint32_t st = traverse_begin<COUNT>(S_, ray, stack, ts, best, occluded, ctr);
@@ -770,8 +787,8 @@ BF_D double child_near_exact(v3f n, const trav_space& s, float t_min) {
 
 /* Next entry of the stack that can still hold a closer hit; leaves the BLAS when it is empty.
  * `cache` holds the lane's world-space o and 1/d, six floats with the given stride. */
-template <bool ANY, uint32_t S, uint32_t LANES>
-BF_D void bound_pop(const bf_dev_scene& S_, trav_stack<S, LANES>& stack, bound_state& ts, const float* cache,
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill>
+BF_D void bound_pop(const bf_dev_scene& S_, trav_stack<S, LANES, Spill>& stack, bound_state& ts, const float* cache,
                     uint32_t stride) {
     for (;;) {
         if (stack_depth(stack) <= ts.base) {
@@ -795,8 +812,8 @@ BF_D void bound_pop(const bf_dev_scene& S_, trav_stack<S, LANES>& stack, bound_s
 }
 
 /* Starts a ray (its world-space o and 1/d go to the lane's cache). */
-template <uint32_t S, uint32_t LANES>
-BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t_max, trav_stack<S, LANES>& stack,
+template <uint32_t S, uint32_t LANES, typename Spill>
+BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t_max, trav_stack<S, LANES, Spill>& stack,
                       bound_state& ts, float* cache, uint32_t stride) {
     stack.sp = 0u;
     stack.gsp = 0u;
@@ -819,8 +836,8 @@ BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t
 }
 
 /* The two child boxes of node ts.cur: the near child becomes ts.cur, the far one is pushed. */
-template <bool ANY, uint32_t S, uint32_t LANES, typename WorldRay>
-BF_D void bound_node(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES>& stack, bound_state& ts,
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
+BF_D void bound_node(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES, Spill>& stack, bound_state& ts,
                      const float* cache, uint32_t stride) {
     const float4* p = reinterpret_cast<const float4*>(ts.nodes + ts.cur);
     const float4 a = p[0], b = p[1], c = p[2];
@@ -950,8 +967,8 @@ BF_D uint32_t watertight_bound(v3f v0, v3f v1, v3f v2, v3f o, v3f d, v3f inv, fl
 
 /* The leaf ts.cur: an instance is entered, a triangle is tested. Returns a traversal status;
  * `occluded` is set by an any-hit walk, whose ray is then done. */
-template <bool ANY, uint32_t S, uint32_t LANES, typename WorldRay>
-BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES>& stack, bound_state& ts,
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
+BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES, Spill>& stack, bound_state& ts,
                          bool& occluded, const float* cache, uint32_t stride) {
     const uint32_t leaf = ts.cur & BF_REF_MASK;
     if (ts.tleaf == BF_INVALID_INDEX) {
