@@ -32,6 +32,9 @@
 #ifndef BF_SHORT_STACK
 #define BF_SHORT_STACK 8u    /* of which the transport kernels keep this many in LDS */
 #endif
+#ifndef BF_SHADOW_STACK
+#define BF_SHADOW_STACK 16u /* the same for any-hit walks, whose entries are half the size */
+#endif
 #define BF_TRACE_BLOCK 128u  /* lanes per traversal workgroup */
 #ifndef BF_TRACE_WAVES_PER_SIMD
 #define BF_TRACE_WAVES_PER_SIMD 6 /* register budget of the closest-hit traversal (waves per SIMD) */
@@ -41,20 +44,20 @@
 #endif
 #ifndef BF_LEAF_PHASE
 /* Traversal waves step interior nodes and leaves in separate iterations: leaves once they are this
- * fraction (1/4) of the running lanes. */
-#define BF_LEAF_PHASE 4u
+ * fraction (1/2) of the running lanes (1/3, 1/4 and 1/6 measured slower). */
+#define BF_LEAF_PHASE 2u
 #endif
 #ifndef BF_SHADOW_LEAF_PHASE
-#define BF_SHADOW_LEAF_PHASE 4u /* the same for any-hit waves */
+#define BF_SHADOW_LEAF_PHASE 2u
 #endif
 #ifndef BF_SHADOW_WAVES_PER_SIMD
-#define BF_SHADOW_WAVES_PER_SIMD 7 /* the any-hit traversal keeps less state than closest hit; 7 waves (72 VGPRs) measured fastest */
+#define BF_SHADOW_WAVES_PER_SIMD 6 /* 5, 7 and 8 measured slower */
 #endif
 #ifndef BF_TRACE_REFILL
-#define BF_TRACE_REFILL 24u /* idle lanes of a closest-hit wave that trigger a fetch of new rays (16, 20, 28, 32, 40 measured slower) */
+#define BF_TRACE_REFILL 40u /* idle lanes of a closest-hit wave that trigger a refill (16, 24, 32 measured slower, 48 equal) */
 #endif
 #ifndef BF_SHADOW_REFILL
-#define BF_SHADOW_REFILL 16u /* the same for an any-hit wave (8 and 24 measured slower) */
+#define BF_SHADOW_REFILL 32u /* the same for an any-hit wave (16, 24 measured slower, 40 equal) */
 #endif
 #ifndef BF_SHADE_WAVES_PER_SIMD
 #define BF_SHADE_WAVES_PER_SIMD 3 /* register budget of the forward shade kernels (waves per SIMD; 1 and 2 measured slower) */

@@ -1090,7 +1090,7 @@ struct bf_hip_workspace {
     uint32_t* failure = nullptr;   /* [0] count, [2..3] lowest (job << 48 | path << 8 | failure code) */
     uint32_t* sample_counts = nullptr;
     unsigned long long* traversal = nullptr; /* 6 counters */
-    uint32_t* fetch = nullptr;               /* traversal work counters (2 words after the counters) */
+    uint32_t* fetch = nullptr;               /* traversal work counters */
     float* replicas = nullptr;               /* BF_GRADIENT_REPLICAS x BF_GRADIENT_ROW adjoint scratch */
     uint32_t* bucket_counts = nullptr;       /* shade-order grouping: per-tile bucket counts / offsets */
     uint32_t* bucket_offsets = nullptr;
@@ -1575,7 +1575,7 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     const size_t o_bc = A.add(nullptr, (size_t)tiles * 32), o_bo = A.add(nullptr, (size_t)tiles * 32);
     const size_t o_route = A.add(nullptr, n), o_tc = A.add(nullptr, (size_t)tiles * 8), o_to = A.add(nullptr, (size_t)tiles * 8),
                  o_sizes = A.add(nullptr, 64), o_hist = A.add(nullptr, BF_HISTORY_BOUNCES * 16), o_fail = A.add(nullptr, 16),
-                 o_samp = A.add(nullptr, 16), o_trav = A.add(nullptr, 64), o_hash = A.add(nullptr, BF_REPORT_MAX_BOUNCES * 16),
+                 o_samp = A.add(nullptr, 16), o_trav = A.add(nullptr, 64), o_fetch = A.add(nullptr, 2 * BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE * 4), o_hash = A.add(nullptr, BF_REPORT_MAX_BOUNCES * 16),
                  o_jobs = A.add(nullptr, BF_MAX_BATCH_JOBS * sizeof(bf_dev_job)),
                  o_replicas = A.add(nullptr, (size_t)BF_GRADIENT_REPLICAS * BF_GRADIENT_ROW * sizeof(float)),
                  o_spill = A.add(nullptr, (size_t)w->spill_lanes * BF_STACK_DEPTH * sizeof(uint2));
@@ -1624,7 +1624,7 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     w->failure = (uint32_t*)(b + o_fail);
     w->sample_counts = (uint32_t*)(b + o_samp);
     w->traversal = (unsigned long long*)(b + o_trav);
-    w->fetch = (uint32_t*)(b + o_trav + 48);
+    w->fetch = (uint32_t*)(b + o_fetch);
     w->hashes = (unsigned long long*)(b + o_hash);
     w->jobs = (bf_dev_job*)(b + o_jobs);
     w->replicas = (float*)(b + o_replicas);

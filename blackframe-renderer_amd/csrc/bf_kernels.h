@@ -65,6 +65,12 @@ typedef struct bf_dev_job {
 #define BF_GRADIENT_SMALL 4096u
 #define BF_GRADIENT_ROW 16384u
 
+/* segments of a traversal launch's queue, one per XCD, and their counters' distance (a 128-byte line) */
+#ifndef BF_CLAIM_SEGMENTS
+#define BF_CLAIM_SEGMENTS 8u
+#endif
+#define BF_CLAIM_STRIDE 32u
+
 #define BF_SHADE_PLAIN 0u
 #define BF_SHADE_TEXTURED 1u
 #define BF_SHADE_ADJOINT 2u
@@ -92,7 +98,8 @@ typedef struct bf_transport_params {
     unsigned long long* step_counters; /* where such a launch counts when the caller asked for no counters */
     uint32_t shade_blocks;      /* resident forward shade workgroups (persistent grid) */
     uint32_t adjoint_shade_blocks; /* resident adjoint shade workgroups */
-    uint32_t* fetch;            /* traversal work counters [closest, shadow], cleared before each launch */
+    uint32_t* fetch;            /* traversal work counters of closest-hit, then shadow launches, cleared
+                                 * before each: BF_CLAIM_SEGMENTS each, BF_CLAIM_STRIDE words apart */
     uint32_t trace_block;       /* lanes per traversal workgroup: 64, 128 or 256 */
     float film_pdf;             /* wavelength pdf and sensor normalisation of the film (adjoint) */
     float film_normalization;

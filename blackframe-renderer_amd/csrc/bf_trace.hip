@@ -184,10 +184,11 @@ BF_D void lane_loop(uint32_t n, Claim claim, Start start, Step step, Finish fini
             }
             if (exhausted) break;
             const uint32_t want = quota - count;
-            const uint32_t base = claim(n, want, exhausted);
+            uint32_t end;
+            const uint32_t base = claim(n, want, end, exhausted);
             if (!active) {
                 const uint32_t rank = (uint32_t)__popcll(~running & ((1ull << lane) - 1ull));
-                if (rank < want && base < n && rank < n - base) {
+                if (base < end && rank < end - base) {
                     active = start(base + rank);
                     done = !active;
                 }
@@ -196,53 +197,82 @@ BF_D void lane_loop(uint32_t n, Claim claim, Start start, Step step, Finish fini
         }
         const bool leaf = active && step.leaf_next();
         const uint64_t leaves = __ballot(leaf);
-        if ((uint32_t)__popcll(leaves) * LEAF >= count) {
-            if (leaf) {
-                active = step.leaf();
-                done = !active;
-            }
+        const bool leaf_phase = (uint32_t)__popcll(leaves) * LEAF >= count;
+        if (leaf_phase) {
+            if (leaf) step.leaf();
         } else if (active && !leaf) {
-            active = step.node();
+            step.node();
+        }
+        if (active && leaf == leaf_phase) {
+            active = step.next();
             done = !active;
         }
     }
 }
 
-/* Lanes each wave of a launch holds: all 64 unless the items do not fill the waves. */
-BF_D uint32_t wave_quota(uint32_t n, uint32_t waves) {
-    const uint32_t share = (n + waves - 1u) / waves;
-    return share < 1u ? 1u : (share < 64u ? share : 64u);
-}
-
-/* How a wave claims items: first its own share of the queue's head (quota items), then from the
- * launch's work counter, one atomic per refill, until the queue is exhausted. */
+/*
+ * How the waves of a launch claim its items. The queue is cut into BF_CLAIM_SEGMENTS contiguous
+ * segments, and workgroup b starts in segment b mod BF_CLAIM_SEGMENTS: workgroups go to the eight
+ * XCDs in turn, so each XCD works through its own part of the queue, whose neighbouring rays meet
+ * neighbouring nodes, and its 4 MB L2 holds one part's nodes instead of every part's. A wave first
+ * takes a fixed share of its segment's head, then draws from the segment's counter (one atomic per
+ * refill), then from the other segments in turn. When the shares cover the queue nothing is drawn:
+ * `quota` lanes of each wave hold the whole queue at once.
+ */
 struct shared_claim {
-    uint32_t* fetch;
-    uint32_t wave, waves, quota;
-    bool opened = false;
-    BF_D uint32_t operator()(uint32_t n, uint32_t want, bool& exhausted) {
-        const uint32_t head = waves * quota;
-        uint32_t base;
+    uint32_t* fetch; /* the segments' counters */
+    uint32_t per;    /* items of a segment (the last may have fewer) */
+    uint32_t segment, segments;
+    uint32_t wave, share_waves; /* the wave's number in its segment; waves of a full segment's share */
+    uint32_t quota;
+    uint32_t tried;
+    bool opened, covered;
+    BF_D uint32_t heads(uint32_t s) const {
+        /* items of segment s given out as fixed shares */
+        const uint32_t blocks = (gridDim.x - s + segments - 1u) / segments;
+        return blocks * (blockDim.x / 64u) * quota;
+    }
+    /* items [result, end) are the wave's; at most `want` */
+    BF_D uint32_t operator()(uint32_t n, uint32_t want, uint32_t& end, bool& exhausted) {
         if (!opened) {
             opened = true;
-            base = wave * quota;
-            exhausted = head >= n;
-        } else {
-            base = 0u;
-            if ((threadIdx.x & 63u) == 0u) base = atomicAdd(fetch, want);
-            base = head + __shfl(base, 0, 64);
-            exhausted = base >= n || n - base <= want;
+            exhausted = covered;
+            const uint32_t base = segment * per + wave * quota;
+            end = min(min(n, segment * per + per), base + want);
+            return base;
         }
-        return base;
+        for (; tried < segments; ++tried) {
+            uint32_t drawn = 0u;
+            if ((threadIdx.x & 63u) == 0u) drawn = atomicAdd(fetch + segment * BF_CLAIM_STRIDE, want);
+            drawn = heads(segment) + __shfl(drawn, 0, 64);
+            const uint32_t base = segment * per + drawn, stop = min(n, segment * per + per);
+            if (drawn < per && base < stop) {
+                end = min(stop, base + want);
+                return base;
+            }
+            segment = segment + 1u == segments ? 0u : segment + 1u;
+        }
+        exhausted = true;
+        end = 0u;
+        return 0u;
     }
 };
 
-/* The claim of this wave, with the launch's quota. */
 template <uint32_t BLOCK>
 BF_D shared_claim wave_claim(uint32_t* fetch, uint32_t n) {
-    const uint32_t waves = gridDim.x * (BLOCK / 64u);
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (BLOCK / 64u) + (threadIdx.x >> 6));
-    return shared_claim{fetch, wave, waves, wave_quota(n, waves)};
+    shared_claim c;
+    c.fetch = fetch;
+    c.segments = gridDim.x < BF_CLAIM_SEGMENTS ? 1u : BF_CLAIM_SEGMENTS;
+    c.per = (n + c.segments - 1u) / c.segments;
+    c.segment = blockIdx.x % c.segments;
+    c.wave = __builtin_amdgcn_readfirstlane(blockIdx.x / c.segments * (BLOCK / 64u) + (threadIdx.x >> 6));
+    c.share_waves = gridDim.x / c.segments * (BLOCK / 64u);
+    const uint32_t share = (c.per + c.share_waves - 1u) / c.share_waves;
+    c.covered = share <= 64u;
+    c.quota = share < 1u ? 1u : (share < 64u ? share : 64u);
+    c.tried = 0u;
+    c.opened = false;
+    return c;
 }
 
 BF_D void reduce_counters(const trav_counters& c, unsigned long long* counters) {
@@ -314,15 +344,15 @@ __global__ __launch_bounds__(BLOCK, BF_COUNT_WAVES_PER_SIMD) void k_trace_counti
         lane_ray* L;
         trav_counters* ctr;
         BF_D bool leaf_next() const { return false; } /* nodes and leaves share one step */
-        BF_D bool leaf() const { return false; }
-        BF_D bool node() const {
+        BF_D void leaf() const {}
+        BF_D bool next() const { return L->status == BF_HIT_MISS && stack_depth(*stack) != 0u; }
+        BF_D void node() const {
             L->status = traverse_step<ANY, true>(job_at<BATCH>(*P, L->slot).scene, world_t{&P->paths, L->slot}, *stack,
                                                  L->ts, L->best, L->occluded, *ctr);
-            return L->status == BF_HIT_MISS && stack_depth(*stack) != 0u;
         }
     };
     lane_loop<24u, 4u>(
-        n, wave_claim<BLOCK>(P.fetch + (ANY ? 1 : 0), n),
+        n, wave_claim<BLOCK>(P.fetch + (ANY ? BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE : 0u), n),
         [&](uint32_t i) {
             L.item = order ? order[i] : i;
             L.slot = queue[L.item];
@@ -344,32 +374,34 @@ __global__ __launch_bounds__(BLOCK, BF_COUNT_WAVES_PER_SIMD) void k_trace_counti
 template <bool ANY, bool BATCH, uint32_t BLOCK>
 __global__ __launch_bounds__(BLOCK, ANY ? BF_SHADOW_WAVES_PER_SIMD : BF_TRACE_WAVES_PER_SIMD) void k_trace(
     bf_transport_params P, const uint32_t* queue, const uint32_t* count_ptr, const uint32_t* order, uint8_t* route) {
-    __shared__ uint2 s_stack[BF_SHORT_STACK * BLOCK];
+    using entry_t = std::conditional_t<ANY, uint32_t, uint2>;
+    __shared__ entry_t s_stack[(ANY ? BF_SHADOW_STACK : BF_SHORT_STACK) * BLOCK];
     __shared__ float s_world[6 * BLOCK];
     const uint32_t n = *count_ptr;
-    trav_stack<BF_SHORT_STACK, BLOCK> stack{
-        s_stack + threadIdx.x, {P.spill + blockIdx.x * BLOCK + threadIdx.x, P.spill_stride}, 0u, 0u, BF_STACK_DEPTH};
+    using stack_t = ring_stack<entry_t, ANY ? BF_SHADOW_STACK : BF_SHORT_STACK, BLOCK, column_spill>;
+    stack_t stack{reinterpret_cast<uint8_t*>(s_stack), threadIdx.x * (uint32_t)sizeof(entry_t),
+                  {P.spill + blockIdx.x * BLOCK + threadIdx.x, P.spill_stride}, 0u, 0u};
     bound_ray L;
     using world_t = std::conditional_t<ANY, shadow_world, closest_world>;
     struct stepper {
         const bf_transport_params* P;
-        trav_stack<BF_SHORT_STACK, BLOCK>* stack;
+        stack_t* stack;
         bound_ray* L;
         const float* cache;
         BF_D bool leaf_next() const { return (L->ts.cur & BF_WIDE_LEAF) != 0u; }
-        BF_D bool node() const {
-            bound_node<ANY>(scene_of<BATCH>(*P, *L), world_t{&P->paths, L->slot}, *stack, L->ts, cache, BLOCK);
-            return L->ts.cur != BF_TRAV_DONE;
+        BF_D void node() const { bound_node(world_t{&P->paths, L->slot}, *stack, L->ts); }
+        BF_D void leaf() const {
+            L->status = bound_leaf<ANY>(scene_of<BATCH>(*P, *L), world_t{&P->paths, L->slot}, *stack, L->ts, L->occluded);
+            if (L->status != BF_HIT_MISS) L->ts.cur = BF_TRAV_DONE;
         }
-        BF_D bool leaf() const {
-            L->status = bound_leaf<ANY>(scene_of<BATCH>(*P, *L), world_t{&P->paths, L->slot}, *stack, L->ts, L->occluded,
-                                        cache, BLOCK);
-            return L->status == BF_HIT_MISS && L->ts.cur != BF_TRAV_DONE;
+        BF_D bool next() const {
+            bound_pop<ANY>(scene_of<BATCH>(*P, *L), *stack, L->ts, cache, BLOCK);
+            return L->ts.cur != BF_TRAV_DONE;
         }
     };
     float* cache = s_world + threadIdx.x;
     lane_loop<ANY ? BF_SHADOW_REFILL : BF_TRACE_REFILL, ANY ? BF_SHADOW_LEAF_PHASE : BF_LEAF_PHASE>(
-        n, wave_claim<BLOCK>(P.fetch + (ANY ? 1 : 0), n),
+        n, wave_claim<BLOCK>(P.fetch + (ANY ? BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE : 0u), n),
         [&](uint32_t i) {
             L.item = order ? order[i] : i;
             L.slot = queue[L.item];
@@ -378,7 +410,7 @@ __global__ __launch_bounds__(BLOCK, ANY ? BF_SHADOW_WAVES_PER_SIMD : BF_TRACE_WA
             trav_ray ray;
             const bf_dev_job& J = load_ray<ANY, BATCH>(P, L.slot, ray);
             L.scene = &J.scene;
-            bound_begin(J.scene, ray.o, ray.d, ray.t_min, ray.t_max, stack, L.ts, cache, BLOCK);
+            bound_begin<ANY>(J.scene, ray.o, ray.d, ray.t_min, ray.t_max, stack, L.ts, cache, BLOCK);
             return L.ts.cur != BF_TRAV_DONE;
         },
         stepper{&P, &stack, &L, cache},
@@ -487,10 +519,11 @@ __global__ __launch_bounds__(BF_API_BLOCK) void k_scene_counting(bf_dev_scene S,
 /* Items of one wave's own chunk of the rays, claimed without atomics. */
 struct chunk_claim {
     uint32_t next, quota;
-    BF_D uint32_t operator()(uint32_t n, uint32_t want, bool& exhausted) {
+    BF_D uint32_t operator()(uint32_t n, uint32_t want, uint32_t& end, bool& exhausted) {
         const uint32_t base = next;
         next += want;
         exhausted = base >= n || n - base <= want;
+        end = exhausted ? n : base + want;
         return base;
     }
 };
@@ -503,11 +536,13 @@ struct chunk_claim {
 template <bool ANY>
 __global__ __launch_bounds__(BF_API_BLOCK, BF_TRACE_WAVES_PER_SIMD) void k_scene_trace(
     bf_dev_scene S, const bf_transport_ray* rays, uint32_t count, uint32_t chunk, void* results) {
-    __shared__ uint2 s_stack[BF_SHORT_STACK * BF_API_BLOCK];
+    using entry_t = std::conditional_t<ANY, uint32_t, uint2>;
+    __shared__ entry_t s_stack[(ANY ? BF_SHADOW_STACK : BF_SHORT_STACK) * BF_API_BLOCK];
     __shared__ float s_world[6 * BF_API_BLOCK];
-    using stack_t = trav_stack<BF_SHORT_STACK, BF_API_BLOCK, scratch_spill>;
-    stack_t stack;
-    stack.lds = s_stack + threadIdx.x;
+    using stack_t = ring_stack<entry_t, ANY ? BF_SHADOW_STACK : BF_SHORT_STACK, BF_API_BLOCK, scratch_spill>;
+    uint32_t spilled[ANY ? 1 : 2][BF_STACK_DEPTH];
+    stack_t stack{reinterpret_cast<uint8_t*>(s_stack), threadIdx.x * (uint32_t)sizeof(entry_t),
+                  {spilled[0], spilled[ANY ? 0 : 1]}, 0u, 0u};
     bound_state ts;
     uint32_t item = 0u, status = BF_HIT_MISS;
     bool occluded = false;
@@ -521,13 +556,14 @@ __global__ __launch_bounds__(BF_API_BLOCK, BF_TRACE_WAVES_PER_SIMD) void k_scene
         bool* occluded;
         const float* cache;
         BF_D bool leaf_next() const { return (ts->cur & BF_WIDE_LEAF) != 0u; }
-        BF_D bool node() const {
-            bound_node<ANY>(*S, api_world{rays + *item}, *stack, *ts, cache, BF_API_BLOCK);
-            return ts->cur != BF_TRAV_DONE;
+        BF_D void node() const { bound_node(api_world{rays + *item}, *stack, *ts); }
+        BF_D void leaf() const {
+            *status = bound_leaf<ANY>(*S, api_world{rays + *item}, *stack, *ts, *occluded);
+            if (*status != BF_HIT_MISS) ts->cur = BF_TRAV_DONE;
         }
-        BF_D bool leaf() const {
-            *status = bound_leaf<ANY>(*S, api_world{rays + *item}, *stack, *ts, *occluded, cache, BF_API_BLOCK);
-            return *status == BF_HIT_MISS && ts->cur != BF_TRAV_DONE;
+        BF_D bool next() const {
+            bound_pop<ANY>(*S, *stack, *ts, cache, BF_API_BLOCK);
+            return ts->cur != BF_TRAV_DONE;
         }
     };
     const uint32_t begin = blockIdx.x * chunk;
@@ -543,7 +579,7 @@ __global__ __launch_bounds__(BF_API_BLOCK, BF_TRACE_WAVES_PER_SIMD) void k_scene
             if (!valid_traversal_ray(r)) return false;
             status = BF_HIT_MISS;
             const trav_ray ray = api_ray(r);
-            bound_begin(S, ray.o, ray.d, ray.t_min, ray.t_max, stack, ts, cache, BF_API_BLOCK);
+            bound_begin<ANY>(S, ray.o, ray.d, ray.t_min, ray.t_max, stack, ts, cache, BF_API_BLOCK);
             return ts.cur != BF_TRAV_DONE;
         },
         stepper{&S, rays, &stack, &ts, &item, &status, &occluded, cache},
@@ -954,7 +990,7 @@ static uint32_t trace_blocks(const bf_transport_params* P, uint32_t max_count, u
 template <bool ANY, bool BATCH, uint32_t BLOCK>
 static void launch_trace(const bf_transport_params* P, uint32_t max_count, const uint32_t* q, const uint32_t* n,
                          uint8_t* route, unsigned long long* counters, bool exact, hipStream_t s) {
-    (void)bfk_set_words(P->fetch + (ANY ? 1 : 0), 1u, 0u, s);
+    (void)bfk_set_words(P->fetch + (ANY ? BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE : 0u), BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE, 0u, s);
     /* optional direction-octant order; the route bytes are free until the traversal writes them */
     uint32_t* order = ANY ? P->shadow_order : P->closest_order;
     if (order)

@@ -447,16 +447,21 @@ struct column_spill {
     uint32_t stride;
     BF_D void put(uint32_t k, uint2 e) { area[(size_t)k * stride] = e; }
     BF_D uint2 get(uint32_t k) const { return area[(size_t)k * stride]; }
+    BF_D void put(uint32_t k, uint32_t e) { area[(size_t)k * stride].x = e; }
+    BF_D void get(uint32_t k, uint2& e) const { e = area[(size_t)k * stride]; }
+    BF_D void get(uint32_t k, uint32_t& e) const { e = area[(size_t)k * stride].x; }
 };
 
 /* A spill area in the lane's scratch, for launches without a workspace. */
 struct scratch_spill {
-    uint32_t ref[BF_STACK_DEPTH], near_word[BF_STACK_DEPTH];
+    uint32_t *ref, *near_word; /* BF_STACK_DEPTH words each, the lane's own */
     BF_D void put(uint32_t k, uint2 e) {
         ref[k] = e.x;
         near_word[k] = e.y;
     }
-    BF_D uint2 get(uint32_t k) const { return make_uint2(ref[k], near_word[k]); }
+    BF_D void put(uint32_t k, uint32_t e) { ref[k] = e; }
+    BF_D void get(uint32_t k, uint2& e) const { e = make_uint2(ref[k], near_word[k]); }
+    BF_D void get(uint32_t k, uint32_t& e) const { e = ref[k]; }
 };
 
 template <uint32_t S, uint32_t LANES, typename Spill = column_spill>
@@ -723,16 +728,58 @@ BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, WorldRay wor
  * counting launches and everything else take the step-exact walk. */
 #define BF_SLAB_REL 0x1p-21f
 #define BF_SLAB_ABS 0x1p-120f
-#define BF_TRAV_DONE 0xFFFFFFFFu /* no next reference: the ray is done */
-
+/* State references beside nodes and leaves: the ray is done (also the root reference of a scene
+ * without instances), a BLAS is left, or the next entry has yet to be popped. All have BF_WIDE_LEAF
+ * set. */
+#define BF_TRAV_DONE 0xFFFFFFFFu
+#define BF_TRAV_POP 0xFFFFFFFEu
+#define BF_TRAV_LEAVE 0xFFFFFFFDu
 struct bound_state {
     v3f o, inv, d;     /* the current space; d is kept for BLAS spaces only */
     float t_min, t;    /* t: the closest hit so far (any-hit: t_max) */
-    uint32_t cur;      /* next reference: node, or BF_WIDE_LEAF | leaf */
-    uint32_t base;     /* stack entries below the current structure */
+    uint32_t cur;      /* next reference: node, BF_WIDE_LEAF | leaf, or one of the above */
+    uint32_t base;     /* stack.sp below the current structure's entries */
     uint32_t tleaf;    /* TLAS leaf of the instance being walked, BF_INVALID_INDEX in the TLAS */
     uint32_t hit_tleaf, hit_leaf; /* the closest hit: TLAS leaf and triangle */
     const bf_wide_node* nodes;
+};
+
+/* Stack of the bound walk: entry k of a lane is in LDS slot k mod S of its column while it is among
+ * the top ones, in the lane's spill area otherwise. A push into a full column moves the oldest half
+ * to the spill area and a pop below the column brings half back (one entry at a time, a lane working
+ * around a full column pays a memory access for every push and pop: 1.7 times the vector-memory
+ * instructions of a launch). `sp` and `low` (the first entry in LDS) count in units of a slot row's
+ * bytes, so that a slot's address is one and-or. */
+template <typename Entry, uint32_t S, uint32_t LANES, typename Spill>
+struct ring_stack {
+    static_assert((S & (S - 1u)) == 0u && (LANES & (LANES - 1u)) == 0u, "slots and lanes are powers of two");
+    static constexpr uint32_t ROW = LANES * (uint32_t)sizeof(Entry);
+    using entry = Entry;
+    uint8_t* column; /* LDS rows, row 0 */
+    uint32_t lane;   /* byte offset of the lane in a row */
+    Spill spill;
+    uint32_t sp, low;
+
+    BF_D Entry* slot(uint32_t at) { return reinterpret_cast<Entry*>(column + ((at & ((S - 1u) * ROW)) | lane)); }
+    BF_D void reset() { sp = low = 0u; }
+    BF_D void push(Entry e) {
+        if (sp - low == S * ROW) {
+#pragma unroll
+            for (uint32_t k = 0; k < S / 2u; ++k) spill.put(low / ROW + k, *slot(low + k * ROW));
+            low += S / 2u * ROW;
+        }
+        *slot(sp) = e;
+        sp += ROW;
+    }
+    BF_D Entry pop() {
+        if (sp == low) {
+            low -= S / 2u * ROW;
+#pragma unroll
+            for (uint32_t k = 0; k < S / 2u; ++k) spill.get(low / ROW + k, *slot(low + k * ROW));
+        }
+        sp -= ROW;
+        return *slot(sp);
+    }
 };
 
 /* Binary32 reciprocals of a direction, or NaN where the bounds do not hold. */
@@ -785,38 +832,64 @@ BF_D double child_near_exact(v3f n, const trav_space& s, float t_min) {
     return v;
 }
 
-/* Next entry of the stack that can still hold a closer hit; leaves the BLAS when it is empty.
- * `cache` holds the lane's world-space o and 1/d, six floats with the given stride. */
-template <bool ANY, uint32_t S, uint32_t LANES, typename Spill>
-BF_D void bound_pop(const bf_dev_scene& S_, trav_stack<S, LANES, Spill>& stack, bound_state& ts, const float* cache,
-                    uint32_t stride) {
-    for (;;) {
-        if (stack_depth(stack) <= ts.base) {
-            if (ts.tleaf == BF_INVALID_INDEX) {
-                ts.cur = BF_TRAV_DONE;
-                return;
+/* A stack entry of a closest-hit walk is (reference, near bound); any-hit walks, whose t never
+ * shrinks, keep the reference alone. */
+BF_D void push_entry(uint2& e, uint32_t ref, float lo) { e = make_uint2(ref, __float_as_uint(lo)); }
+BF_D void push_entry(uint32_t& e, uint32_t ref, float) { e = ref; }
+BF_D uint32_t entry_ref(uint2 e) { return e.x; }
+BF_D uint32_t entry_ref(uint32_t e) { return e; }
+BF_D bool entry_live(uint2 e, float t) { return !(__uint_as_float(e.y) > t); }
+BF_D bool entry_live(uint32_t, float) { return true; }
+
+template <typename Stack>
+BF_D void push_ref(Stack& stack, uint32_t ref, float lo) {
+    typename Stack::entry e;
+    push_entry(e, ref, lo);
+    stack.push(e);
+}
+
+/* Back to world space: `cache` holds the lane's world-space o and 1/d, six floats with the given
+ * stride. */
+BF_D void bound_leave(const bf_dev_scene& S_, bound_state& ts, const float* cache, uint32_t stride) {
+    ts.o = mk(cache[0], cache[stride], cache[2u * stride]);
+    ts.inv = mk(cache[3u * stride], cache[4u * stride], cache[5u * stride]);
+    ts.nodes = S_.tlas_nodes;
+    ts.tleaf = BF_INVALID_INDEX;
+    ts.base = 0u;
+}
+
+/* Takes the next entry that can still hold a closer hit where one is due (ts.cur is BF_TRAV_POP),
+ * leaving the BLAS on the way. Any-hit walks find the ends of the BLAS and of the ray as entries of
+ * their own (16 half-size slots have room for them: 49.3 ms of shadow rays in the 1080p x 64 frame,
+ * 52.5 with a compare against the structure's first entry); closest-hit walks compare, since two
+ * entries more of their 8 slots spill more often (98.3 ms of closest-hit rays, 102.9 with entries). */
+template <bool ANY, typename Stack>
+BF_D void bound_pop(const bf_dev_scene& S_, Stack& stack, bound_state& ts, const float* cache, uint32_t stride) {
+    while (ts.cur == BF_TRAV_POP) {
+        if constexpr (ANY) {
+            const auto e = stack.pop();
+            const uint32_t ref = entry_ref(e);
+            if (ref == BF_TRAV_LEAVE) bound_leave(S_, ts, cache, stride);
+            else if (entry_live(e, ts.t)) ts.cur = ref;
+        } else {
+            if (stack.sp == ts.base) {
+                if (ts.tleaf == BF_INVALID_INDEX) ts.cur = BF_TRAV_DONE;
+                else bound_leave(S_, ts, cache, stride);
+            } else {
+                const auto e = stack.pop();
+                if (entry_live(e, ts.t)) ts.cur = entry_ref(e);
             }
-            ts.o = mk(cache[0], cache[stride], cache[2u * stride]);
-            ts.inv = mk(cache[3u * stride], cache[4u * stride], cache[5u * stride]);
-            ts.nodes = S_.tlas_nodes;
-            ts.tleaf = BF_INVALID_INDEX;
-            ts.base = 0u;
-            continue;
-        }
-        const uint2 e = stack_pop(stack);
-        if (ANY || !(__uint_as_float(e.y) > ts.t)) {
-            ts.cur = e.x;
-            return;
         }
     }
 }
 
 /* Starts a ray (its world-space o and 1/d go to the lane's cache). */
-template <uint32_t S, uint32_t LANES, typename Spill>
-BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t_max, trav_stack<S, LANES, Spill>& stack,
-                      bound_state& ts, float* cache, uint32_t stride) {
-    stack.sp = 0u;
-    stack.gsp = 0u;
+template <bool ANY, typename Stack>
+BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t_max, Stack& stack, bound_state& ts,
+                      float* cache, uint32_t stride) {
+    stack.reset();
+    ts.base = 0u;
+    if constexpr (ANY) push_ref(stack, BF_TRAV_DONE, -BF_INFINITY_F);
     ts.o = o;
     ts.inv = bound_reciprocals(o, d);
     cache[0] = o.x;
@@ -827,7 +900,6 @@ BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t
     cache[5u * stride] = ts.inv.z;
     ts.t_min = t_min;
     ts.t = t_max;
-    ts.base = 0u;
     ts.tleaf = BF_INVALID_INDEX;
     ts.hit_leaf = BF_INVALID_INDEX;
     ts.hit_tleaf = BF_INVALID_INDEX;
@@ -836,9 +908,8 @@ BF_D void bound_begin(const bf_dev_scene& S_, v3f o, v3f d, float t_min, float t
 }
 
 /* The two child boxes of node ts.cur: the near child becomes ts.cur, the far one is pushed. */
-template <bool ANY, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
-BF_D void bound_node(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES, Spill>& stack, bound_state& ts,
-                     const float* cache, uint32_t stride) {
+template <typename Stack, typename WorldRay>
+BF_D void bound_node(WorldRay world, Stack& stack, bound_state& ts) {
     const float4* p = reinterpret_cast<const float4*>(ts.nodes + ts.cur);
     const float4 a = p[0], b = p[1], c = p[2];
     const uint2 child = *reinterpret_cast<const uint2*>(p + 3);
@@ -860,37 +931,33 @@ BF_D void bound_node(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES
     const float lo1 = fmaf(nv1, 1.0f - BF_SLAB_REL, -BF_SLAB_ABS);
     const bool h0 = !(lo0 > fmaf(fv0, 1.0f + BF_SLAB_REL, BF_SLAB_ABS));
     const bool h1 = !(lo1 > fmaf(fv1, 1.0f + BF_SLAB_REL, BF_SLAB_ABS));
-    if (h0 && h1) {
-        const float lead = nv1 - nv0, band = fmaf(nv0 + nv1, BF_SLAB_REL, 4.0f * BF_SLAB_ABS);
-        bool first_near = lead > 0.0f;
-        if (!(fabsf(lead) > band)) {
-            /* a tie when each axis has equal near planes or lies below both near values */
-            const float below = fmaf(fminf(nv0, nv1), 1.0f - 2.0f * BF_SLAB_REL, -4.0f * BF_SLAB_ABS);
-            const float up = 1.0f + BF_SLAB_REL;
-            const bool tie = (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
-                             (n0.y == n1.y || fmaxf(q0.y, q1.y) * up < below) &&
-                             (n0.z == n1.z || fmaxf(q0.z, q1.z) * up < below);
-            first_near = true;
-            if (!tie) {
-                v3f d = ts.d;
-                uint32_t mask;
-                if (ts.tleaf == BF_INVALID_INDEX) world(d, mask);
-                trav_space s;
-                make_space(ts.o, d, s);
-                /* the near planes by the direction's own signs (the reciprocals may be NaN) */
-                const bool ex = (d.x < 0.0f) != sx, ey = (d.y < 0.0f) != sy, ez = (d.z < 0.0f) != sz;
-                const v3f m0 = mk(ex ? f0.x : n0.x, ey ? f0.y : n0.y, ez ? f0.z : n0.z);
-                const v3f m1 = mk(ex ? f1.x : n1.x, ey ? f1.y : n1.y, ez ? f1.z : n1.z);
-                first_near = (float)child_near_exact(m0, s, ts.t_min) <= (float)child_near_exact(m1, s, ts.t_min);
-            }
+    const bool both = h0 && h1;
+    const float lead = nv1 - nv0;
+    bool first = both ? lead > 0.0f : h0;
+    if (both && !(fabsf(lead) > fmaf(nv0 + nv1, BF_SLAB_REL, 4.0f * BF_SLAB_ABS))) {
+        /* a tie when each axis has equal near planes or lies below both near values */
+        const float below = fmaf(fminf(nv0, nv1), 1.0f - 2.0f * BF_SLAB_REL, -4.0f * BF_SLAB_ABS);
+        const float up = 1.0f + BF_SLAB_REL;
+        const bool tie = (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
+                         (n0.y == n1.y || fmaxf(q0.y, q1.y) * up < below) &&
+                         (n0.z == n1.z || fmaxf(q0.z, q1.z) * up < below);
+        first = true;
+        if (!tie) {
+            v3f d = ts.d;
+            uint32_t mask;
+            if (ts.tleaf == BF_INVALID_INDEX) world(d, mask);
+            trav_space s;
+            make_space(ts.o, d, s);
+            /* the near planes by the direction's own signs (the reciprocals may be NaN) */
+            const bool ex = (d.x < 0.0f) != sx, ey = (d.y < 0.0f) != sy, ez = (d.z < 0.0f) != sz;
+            const v3f m0 = mk(ex ? f0.x : n0.x, ey ? f0.y : n0.y, ez ? f0.z : n0.z);
+            const v3f m1 = mk(ex ? f1.x : n1.x, ey ? f1.y : n1.y, ez ? f1.z : n1.z);
+            first = (float)child_near_exact(m0, s, ts.t_min) <= (float)child_near_exact(m1, s, ts.t_min);
         }
-        stack_push(stack, make_uint2(first_near ? child.y : child.x, __float_as_uint(first_near ? lo1 : lo0)));
-        ts.cur = first_near ? child.x : child.y;
-    } else if (h0 || h1) {
-        ts.cur = h0 ? child.x : child.y;
-    } else {
-        bound_pop<ANY>(S_, stack, ts, cache, stride);
     }
+    if (both) push_ref(stack, first ? child.y : child.x, first ? lo1 : lo0);
+    ts.cur = first ? child.x : child.y;
+    if (!h0 && !h1) ts.cur = BF_TRAV_POP;
 }
 
 /* watertight<false> with the same verdict and t for fewer operations: non-finite terms are looked
@@ -933,17 +1000,20 @@ BF_D uint32_t watertight_bound(v3f v0, v3f v1, v3f v2, v3f o, v3f d, v3f inv, fl
     const float emin = fminf(fminf(e0, e1), e2), emax = fmaxf(fmaxf(e0, e1), e2);
     const bool mixed = emin < 0.0f && emax > 0.0f;
     if (mixed) {
-        /* each sheared coordinate is within 4u of its exact value relative to |t_x| + |s t_z|, so
-         * with X and Y the largest of those sums each edge function is within 20.01u X Y of the
-         * exact one and the binary64 re-decision within 2^-49 X Y: signs certain beyond 24u X Y
-         * (and a floor for underflow) are mixed there too, and the ray misses. */
-        const float X = fmaxf(fmaxf(fmaf(fabsf(sx), fabsf(t0z), fabsf(t0x)), fmaf(fabsf(sx), fabsf(t1z), fabsf(t1x))),
-                              fmaf(fabsf(sx), fabsf(t2z), fabsf(t2x))) +
-                        0x1p-60f;
-        const float Y = fmaxf(fmaxf(fmaf(fabsf(sy), fabsf(t0z), fabsf(t0y)), fmaf(fabsf(sy), fabsf(t1z), fabsf(t1y))),
-                              fmaf(fabsf(sy), fabsf(t2z), fabsf(t2y))) +
-                        0x1p-60f;
-        const float bound = (X * Y) * (24.0f * 0x1p-24f) + 0x1p-100f;
+        /* Binary32 filter in front of the binary64 re-decision (u = 2^-24). With M at least every
+         * |t_x| + |s t_z| (|s| <= 1 + 3u), a sheared coordinate is within 4.1u M of its exact value;
+         * with R the largest of the six, an edge function is then within 4 R 4.1u M + 2 (4.1u M)^2
+         * of the exact one for its inputs' errors and 4.1u R^2 for its own roundings, and the
+         * binary64 edge functions (the exact ones times d_kz^2) within 2^-48 of the same terms.
+         * Signs beyond 25u M (R + 25u M) are therefore the binary64 signs. R, the distance of the
+         * triangle's edges from the ray, and not M, the distance of the ray's origin, keeps this
+         * tight for small far triangles: with M^2 for R M about half the far tests went to binary64. */
+        const float M = fmaxf(fmaxf(fmaxf(fabsf(t0x), fabsf(t1x)), fabsf(t2x)),
+                              fmaxf(fmaxf(fabsf(t0y), fabsf(t1y)), fabsf(t2y))) +
+                        fmaxf(fmaxf(fabsf(t0z), fabsf(t1z)), fabsf(t2z)) + 0x1p-60f;
+        const float R = fmaxf(fmaxf(fmaxf(fabsf(ax), fabsf(bx)), fabsf(cx)), fmaxf(fmaxf(fabsf(ay), fabsf(by)), fabsf(cy)));
+        const float m = M * (25.0f * 0x1p-24f);
+        const float bound = fmaf(m, R + m, 0x1p-100f);
         if (emin < -bound && emax > bound) return BF_HIT_MISS;
     }
     if (mixed || emin == 0.0f || emax == 0.0f)
@@ -967,10 +1037,10 @@ BF_D uint32_t watertight_bound(v3f v0, v3f v1, v3f v2, v3f o, v3f d, v3f inv, fl
 
 /* The leaf ts.cur: an instance is entered, a triangle is tested. Returns a traversal status;
  * `occluded` is set by an any-hit walk, whose ray is then done. */
-template <bool ANY, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
-BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES, Spill>& stack, bound_state& ts,
-                         bool& occluded, const float* cache, uint32_t stride) {
+template <bool ANY, typename Stack, typename WorldRay>
+BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, Stack& stack, bound_state& ts, bool& occluded) {
     const uint32_t leaf = ts.cur & BF_REF_MASK;
+    ts.cur = BF_TRAV_POP;
     if (ts.tleaf == BF_INVALID_INDEX) {
         const bf_dev_tlas_leaf& L = S_.tlas_leaves[leaf];
         v3f d;
@@ -987,7 +1057,8 @@ BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, trav_stack<S, L
             ts.d = pd;
             ts.inv = bound_reciprocals(po, pd);
             ts.tleaf = leaf;
-            ts.base = stack_depth(stack);
+            ts.base = stack.sp;
+            if constexpr (ANY) push_ref(stack, BF_TRAV_LEAVE, 0.0f);
             ts.nodes = S_.blas_nodes;
             ts.cur = L.root_ref;
             return BF_HIT_MISS;
@@ -1026,7 +1097,6 @@ BF_D uint32_t bound_leaf(const bf_dev_scene& S_, WorldRay world, trav_stack<S, L
             }
         }
     }
-    bound_pop<ANY>(S_, stack, ts, cache, stride);
     return BF_HIT_MISS;
 }
 

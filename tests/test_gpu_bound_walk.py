@@ -95,3 +95,32 @@ def test_any_item_count_matches_the_oracle(bf, abi, oracle, hip, count):
     options = bf.scenes.transport_options(max_depth=2, rr_first_depth=0)
     options.failure_policy = abi.FAILURES_COUNT
     compare(hip, oracle, lattice(bf), path_inputs(abi, rays), options)
+
+
+@pytest.mark.parametrize("count,tiny", [(1, 0.0), (65, 0.0), (6145, 0.0), (30001, 0.0), (3000, 1e-42)])
+def test_ray_queries_match_the_oracle(bf, abi, oracle, hip, count, tiny):
+    """Uncounted stand-alone queries; 6145 rays are one more than the waves the share is cut for."""
+    scene = lattice(bf)
+    xs, want = hip.XpuScene(scene), oracle.scene(scene)
+    rays = lattice_rays(abi, count, 7 + count, tiny=tiny)
+    rays[count // 2].t_min = -1.0  # an invalid ray answers alone
+    assert result_bytes(xs.closest_hit(rays)) == result_bytes(want.closest_hit(rays))
+    rays = lattice_rays(abi, count, 8 + count, tiny=tiny, t_max=2.5)
+    assert result_bytes(xs.occlusion(rays)) == result_bytes(want.occlusion(rays))
+
+
+def test_deep_stacks_match_the_oracle(bf, abi, oracle, hip):
+    """Walks that hold more entries than the LDS part of the stack: many overlapping boxes per ray."""
+    scene, _ = bf.scenes.icosphere_grid(grid=6, subdivisions=3)
+    rng = np.random.default_rng(1)
+    n = 8000
+    rays = (abi.TransportRay * n)()
+    view = np.frombuffer(rays, dtype=np.float32).reshape(n, 12)
+    view[:, 0:3] = rng.uniform([-9, -1, -9], [9, 1, 9], size=(n, 3))
+    d = rng.normal(size=(n, 3)) * [1.0, 0.02, 1.0]
+    view[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    view[:, 7], view[:, 8] = np.inf, 0.5
+    np.frombuffer(rays, dtype=np.uint32).reshape(n, 12)[:, 9] = 0xFFFFFFFF
+    xs, want = hip.XpuScene(scene), oracle.scene(scene)
+    assert result_bytes(xs.closest_hit(rays)) == result_bytes(want.closest_hit(rays))
+    assert result_bytes(xs.occlusion(rays)) == result_bytes(want.occlusion(rays))
