@@ -79,52 +79,103 @@ BF_D uint64_t indexed_bits(const sample_key& k, uint64_t dim) {
     return mix_bits(state ^ dim);
 }
 
-/* Owen-scrambled Sobol, evaluated only to the 24 leading bits the binary32 sample keeps: the
- * nested scramble of OwenScrambling.cpp:22-36 decides output bit 63-d from input bits above it,
- * so depths 24..63 never reach (bits >> 40). */
-BF_D uint32_t owen_sobol_top24(const sample_key& k, const uint64_t* directions, uint32_t dims, uint64_t sobol_dim,
-                               bool* ok) {
-    if (sobol_dim >= dims) {
-        *ok = false;
-        return 0u;
-    }
-    uint64_t gray = k.s ^ (k.s >> 1);
-    const uint64_t* d = directions + sobol_dim * 64u;
-    uint64_t sample = 0;
-    while (gray != 0) {
-        sample ^= d[__builtin_ctzll(gray)];
-        gray &= gray - 1u;
-    }
-    const uint64_t packed = ((uint64_t)k.px << 32) | (uint64_t)k.py;
-    const uint64_t key = mix_bits(k.seed ^ mix_bits(sobol_dim + 1u)) ^ mix_bits(packed);
-    const uint32_t input = (uint32_t)(sample >> 40);
-    uint32_t prefix = 0u, output = 0u;
-    for (uint32_t depth = 0; depth < 24u; ++depth) {
-        const uint32_t bit = (input >> (23u - depth)) & 1u;
-        const uint64_t node = (1ull << depth) | (uint64_t)prefix;
-        const uint32_t flip = (uint32_t)(mix_bits(key ^ node) >> 63);
-        output |= (bit ^ flip) << (23u - depth);
-        prefix = (prefix << 1) | bit;
-    }
-    *ok = true;
-    return output;
-}
-
 struct sampler_ctx {
     uint32_t kind;
     uint32_t sobol_dims;
-    const uint64_t* directions;
+    const uint32_t* directions; /* [dimension][64]: the 24 leading bits of each direction number */
+    const uint64_t* dimension_keys; /* [dimension]: mix_bits(dimension + 1) */
 };
+
+/*
+ * Owen-scrambled Sobol, evaluated only to the 24 leading bits the binary32 sample keeps: the nested
+ * scramble of OwenScrambling.cpp:22-36 decides output bit 63-d from input bits above it, so depths
+ * 24..63 never reach (bits >> 40), and bits above 24 of the direction numbers suffice. The scramble's
+ * flips are what a light or closure sample costs (24 64-bit hashes a dimension, about a fifth of the
+ * shade stage's vector cycles), so each is cut to what its one result bit needs.
+ */
+struct owen_stream {
+    uint32_t input;     /* Sobol point, 24 bits */
+    uint32_t key_low;   /* the hash input of node n is (key ^ key >> 30) ^ n: n stays in the low word */
+    uint64_t product;   /* its high word's share of the first product */
+};
+
+BF_D bool owen_open(const sampler_ctx& sc, const sample_key& k, uint64_t sobol_dim, owen_stream& o) {
+    if (sobol_dim >= sc.sobol_dims) return false;
+    const uint64_t gray = k.s ^ (k.s >> 1);
+    const uint32_t* d = sc.directions + (uint32_t)sobol_dim * 64u;
+    /* the first eight bits of the index (frames of up to 256 samples) without a loop of dependent loads */
+    const uint4 d0 = reinterpret_cast<const uint4*>(d)[0], d1 = reinterpret_cast<const uint4*>(d)[1];
+    const uint32_t low = (uint32_t)gray;
+    const uint32_t bits[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+    uint32_t point = 0u;
+#pragma unroll
+    for (uint32_t b = 0; b < 8u; ++b) point ^= bits[b] & (uint32_t)__builtin_amdgcn_sbfe((int)low, b, 1u);
+    for (uint64_t rest = gray & ~0xFFull; rest != 0u; rest &= rest - 1u) point ^= d[__builtin_ctzll(rest)];
+    const uint64_t packed = ((uint64_t)k.px << 32) | (uint64_t)k.py;
+    const uint64_t key = mix_bits(k.seed ^ sc.dimension_keys[(uint32_t)sobol_dim]) ^ mix_bits(packed);
+    const uint64_t first = key ^ (key >> 30); /* nodes have 25 bits: they never reach this shift */
+    o.input = point;
+    o.key_low = (uint32_t)first;
+    o.product = (uint64_t)((uint32_t)(first >> 32) * 0x1CE4E5B9u) << 32;
+    return true;
+}
+
+/* Sample bits of depths [FROM, TO) (leading bit first), in the low TO - FROM bits: each is the input's
+ * bit flipped by bit 63 of mix_bits(key ^ node), node = 1 followed by the input's leading bits. The
+ * last xor-shift of mix_bits leaves bit 63 alone, and of the last product only the high word is
+ * formed. */
+template <uint32_t FROM, uint32_t TO>
+BF_D uint32_t owen_bits(const owen_stream& o) {
+    const uint32_t tagged = o.input | 0x1000000u;
+    uint32_t flips = 0u;
+#pragma unroll
+    for (uint32_t depth = FROM; depth < TO; ++depth) {
+        const uint32_t v = o.key_low ^ (tagged >> (24u - depth));
+        const uint64_t w = (uint64_t)v * 0x1CE4E5B9u + o.product;
+        const uint32_t wl = (uint32_t)w, wh = (uint32_t)(w >> 32) + v * 0xBF58476Du;
+        const uint32_t xl = wl ^ __builtin_amdgcn_alignbit(wh, wl, 27u), xh = wh ^ (wh >> 27);
+        const uint32_t yh = __umulhi(xl, 0x133111EBu) + xl * 0x94D049BBu + xh * 0x133111EBu;
+        flips = (flips << 1) | (yh >> 31);
+    }
+    return ((o.input >> (24u - TO)) & ((1u << (TO - FROM)) - 1u)) ^ flips;
+}
+
+BF_D uint64_t sobol_dimension(uint64_t dim) {
+    return dim == BF_DIM_RASTER_X ? 0ull : (dim == BF_DIM_RASTER_Y ? 1ull : dim + 2u);
+}
 
 /* One transport dimension -> binary32 in [0, 1): (bits >> 40) * 2^-24 (SampleStreamDevice.cuh:29-32). */
 BF_D float sample_1d(const sampler_ctx& sc, const sample_key& k, uint64_t dim) {
     if (sc.kind == BF_SAMPLER_SOBOL_OWEN) {
-        const uint64_t sd = dim == BF_DIM_RASTER_X ? 0ull : (dim == BF_DIM_RASTER_Y ? 1ull : dim + 2u);
-        bool ok;
-        const uint32_t top = owen_sobol_top24(k, sc.directions, sc.sobol_dims, sd, &ok);
-        return ok ? (float)top * 0x1p-24f : -1.0f;
+        owen_stream o;
+        return owen_open(sc, k, sobol_dimension(dim), o) ? (float)owen_bits<0u, 24u>(o) * 0x1p-24f : -1.0f;
     }
     return (float)(indexed_bits(k, dim) >> 40) * 0x1p-24f;
+}
+
+/* sample_1d(dim) < p, formed from as many leading bits as decide it (eight, but for one lane in
+ * 256); false when the dimension has no sample. */
+BF_D bool sample_below(const sampler_ctx& sc, const sample_key& k, uint64_t dim, float p, bool& below) {
+    if (sc.kind == BF_SAMPLER_SOBOL_OWEN) {
+        owen_stream o;
+        if (!owen_open(sc, k, sobol_dimension(dim), o)) return false;
+        const uint32_t head = owen_bits<0u, 8u>(o);
+        below = (float)(head + 1u) * 0x1p-8f <= p;
+        if (!below && (float)head * 0x1p-8f < p) below = (float)((head << 16) | owen_bits<8u, 24u>(o)) * 0x1p-24f < p;
+        return true;
+    }
+    below = (float)(indexed_bits(k, dim) >> 40) * 0x1p-24f < p;
+    return true;
+}
+
+/* The leading eight bits of sample_1d(dim), as a binary32 value: the sample rounded down to a multiple of
+ * 1/256. Negative when the dimension has no sample. */
+BF_D float sample_head(const sampler_ctx& sc, const sample_key& k, uint64_t dim) {
+    if (sc.kind == BF_SAMPLER_SOBOL_OWEN) {
+        owen_stream o;
+        return owen_open(sc, k, sobol_dimension(dim), o) ? (float)owen_bits<0u, 8u>(o) * 0x1p-8f : -1.0f;
+    }
+    return (float)(indexed_bits(k, dim) >> 56) * 0x1p-8f;
 }
 
 /* ---- checked arithmetic: TransportDevice.cuh:196-259 --------------------------------------- */
@@ -225,34 +276,10 @@ BF_D bool mis_weight(uint32_t heuristic, float sampled, float competing, float& 
     return true;
 }
 
-/* TransportDevice.cuh:711-782 */
-/* The roulette decision with survival probability p: u < p survives and divides the throughput
- * by p. */
-BF_D bool russian_roulette_at(float4& t, float p, float u, bool& survived) {
-    if (!bf_isfinite(u) || u < 0.0f || !(u < 1.0f)) return false;
-    const float v[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (!bf_isfinite(v[k]) || v[k] < 0.0f) return false;
-    if (!bf_isfinite(p) || !(p > 0.0f) || p > 1.0f) return false;
-    if (!(u < p)) {
-        survived = false;
-        return true;
-    }
-    float o[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        o[k] = v[k] / p;
-        if (!bf_isfinite(o[k]) || (v[k] != 0.0f && o[k] == 0.0f)) return false;
-    }
-    t = make_float4(o[0], o[1], o[2], o[3]);
-    survived = true;
-    return true;
-}
-
-/* The survival probability clamp(max(throughput) * eta, minimum, maximum), then the decision. */
-BF_D bool russian_roulette(float4& t, float eta, float u, float minimum, float maximum, bool& survived, float& p) {
-    if (!bf_isfinite(eta) || !(eta > 0.0f) || !bf_isfinite(u) || u < 0.0f || !(u < 1.0f)) return false;
+/* Russian roulette (TransportDevice.cuh:711-782): the survival probability clamp(max(throughput) *
+ * eta, minimum, maximum). */
+BF_D bool roulette_probability(float4 t, float eta, float minimum, float maximum, float& p) {
+    if (!bf_isfinite(eta) || !(eta > 0.0f)) return false;
     const float v[4] = {t.x, t.y, t.z, t.w};
     float m = 0.0f;
 #pragma unroll
@@ -267,7 +294,25 @@ BF_D bool russian_roulette(float4& t, float eta, float u, float minimum, float m
         const float c = m * eta;
         p = c < minimum ? minimum : (maximum < c ? maximum : c);
     }
-    return russian_roulette_at(t, p, u, survived);
+    return true;
+}
+
+/* The survivor's throughput, divided by its survival probability p. */
+BF_D bool roulette_survive(float4& t, float p) {
+    const float v[4] = {t.x, t.y, t.z, t.w};
+    float o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        o[k] = v[k] / p;
+        if (!bf_isfinite(o[k]) || (v[k] != 0.0f && o[k] == 0.0f)) return false;
+    }
+    t = make_float4(o[0], o[1], o[2], o[3]);
+    return true;
+}
+
+BF_D bool finite_nonnegative4(float4 t) {
+    return bf_isfinite(t.x) && t.x >= 0.0f && bf_isfinite(t.y) && t.y >= 0.0f && bf_isfinite(t.z) && t.z >= 0.0f &&
+           bf_isfinite(t.w) && t.w >= 0.0f;
 }
 
 /* TransportDevice.cuh:327-333 */

@@ -91,26 +91,47 @@ std::vector<uint64_t> sobol_directions() {
     return d;
 }
 
+/* mix_bits (SampleStreamDevice.cuh:12-18), as the device's samplers hash */
+uint64_t mix_bits_host(uint64_t v) {
+    v ^= v >> 30;
+    v *= 0xBF58476D1CE4E5B9ull;
+    v ^= v >> 27;
+    v *= 0x94D049BB133111EBull;
+    return v ^ (v >> 31);
+}
+
 struct SobolTable {
     std::mutex lock;
     int device = -1;
-    uint64_t* directions = nullptr;
+    uint64_t* keys = nullptr; /* dimension keys, then the direction table */
 };
 SobolTable g_sobol;
 
-int sobol_table_for_current_device(const uint64_t** out) {
+/* The sampler tables of the current device: per dimension the 24 leading bits of its 64 direction
+ * numbers (rows 256-byte aligned) and its hash key. */
+int sampler_for_current_device(uint32_t kind, sampler_ctx* out) {
     std::lock_guard<std::mutex> guard(g_sobol.lock);
     int device = 0;
     HIP_TRY(hipGetDevice(&device));
-    if (g_sobol.directions == nullptr || g_sobol.device != device) {
-        const std::vector<uint64_t> table = sobol_directions();
+    const size_t key_words = ((size_t)kSobolDimensions + 31u) / 32u * 64u; /* 32-bit words, whole rows */
+    if (g_sobol.keys == nullptr || g_sobol.device != device) {
+        const std::vector<uint64_t> directions = sobol_directions();
+        std::vector<uint32_t> table(key_words + directions.size(), 0u);
+        for (uint32_t d = 0; d < kSobolDimensions; ++d) {
+            const uint64_t key = mix_bits_host((uint64_t)d + 1u);
+            std::memcpy(&table[2u * (size_t)d], &key, sizeof key);
+        }
+        for (size_t k = 0; k < directions.size(); ++k) table[key_words + k] = (uint32_t)(directions[k] >> 40);
         uint64_t* ptr = nullptr;
-        HIP_TRY(hipMalloc(&ptr, table.size() * sizeof(uint64_t)));
-        HIP_TRY(hipMemcpy(ptr, table.data(), table.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
-        g_sobol.directions = ptr; /* one table per process and device, kept until exit */
+        HIP_TRY(hipMalloc(&ptr, table.size() * sizeof(uint32_t)));
+        HIP_TRY(hipMemcpy(ptr, table.data(), table.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        g_sobol.keys = ptr; /* one table per process and device, kept until exit */
         g_sobol.device = device;
     }
-    *out = g_sobol.directions;
+    out->kind = kind;
+    out->sobol_dims = kSobolDimensions;
+    out->dimension_keys = g_sobol.keys;
+    out->directions = (const uint32_t*)g_sobol.keys + key_words;
     return BF_OK;
 }
 
@@ -1538,10 +1559,10 @@ int blackframe_hip_launch_sample_dump(uint32_t sampler, const bf_sample_stream_i
                                       uint32_t count, float* samples, void* stream) {
     if (sampler > BF_SAMPLER_SOBOL_OWEN) return set_error(BF_INVALID_ARGUMENT, "unknown sampler %u", sampler);
     if (count != 0 && (!indices || !dimensions || !samples)) return set_error(BF_INVALID_ARGUMENT, "NULL argument");
-    const uint64_t* directions = nullptr;
-    const int st = sobol_table_for_current_device(&directions);
+    sampler_ctx tables{};
+    const int st = sampler_for_current_device(sampler, &tables);
     if (st != BF_OK) return st;
-    HIP_TRY(bfk_sample_dump(sampler, directions, kSobolDimensions, indices, dimensions, count, samples, (hipStream_t)stream));
+    HIP_TRY(bfk_sample_dump(&tables, indices, dimensions, count, samples, (hipStream_t)stream));
     return BF_OK;
 }
 
@@ -1821,12 +1842,8 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
 
     bf_transport_params P{};
     P.paths = w->paths;
-    const uint64_t* directions = nullptr;
-    const int sst = sobol_table_for_current_device(&directions);
+    const int sst = sampler_for_current_device(o->sampler, &P.sampler);
     if (sst != BF_OK) return sst;
-    P.sampler.kind = o->sampler;
-    P.sampler.sobol_dims = kSobolDimensions;
-    P.sampler.directions = directions;
     P.mis = o->mis_heuristic;
     P.wavelength_mode = o->wavelength_mode;
     P.limits[0] = o->diffuse_depth_limit;
@@ -2658,8 +2675,8 @@ int blackframe_hip_fit_graph_create(bf_hip_workspace* w, const bf_fit_step_desc*
     const uint64_t in_flight = w->capacity >> ((o->launch & BF_LAUNCH_INFLIGHT_MASK) >> 22);
     const size_t rows = pack_launches(d->frames, d->frame_count, in_flight).size();
     if (rows == 0) return set_error(BF_RESOURCE_EXHAUSTED, "the frames do not fit the workspace's paths in flight");
-    const uint64_t* directions = nullptr;
-    int st = sobol_table_for_current_device(&directions); /* uploaded before the capture */
+    sampler_ctx sampler{};
+    int st = sampler_for_current_device(o->sampler, &sampler); /* tables uploaded before the capture */
     if (st != BF_OK) return st;
 
     bf_hip_fit_graph* g = new bf_hip_fit_graph;

@@ -160,7 +160,7 @@ hipError_t bfk_blob_traverse(bool any, const uint8_t* scene_bytes, size_t scene_
                              size_t bvh_size, const bf_transport_ray* rays, uint32_t count, void* results, hipStream_t s);
 hipError_t bfk_scene_occlusion(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
                                bf_occlusion_result* results, hipStream_t s);
-hipError_t bfk_sample_dump(uint32_t kind, const uint64_t* directions, uint32_t dims, const bf_sample_stream_index* indices,
+hipError_t bfk_sample_dump(const sampler_ctx* sampler, const bf_sample_stream_index* indices,
                            const uint64_t* dimensions, uint32_t count, float* out, hipStream_t s);
 hipError_t bfk_sample_stream_dump(const bf_sample_dump_request* requests, uint32_t count,
                                   bf_sample_dimension_manifest* manifest, bf_sample_dump_result* results);

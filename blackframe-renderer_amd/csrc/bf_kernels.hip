@@ -1316,14 +1316,10 @@ hipError_t bfk_queue_hash(const uint32_t* queue, const uint32_t* count_ptr, unsi
     return hipGetLastError();
 }
 
-hipError_t bfk_sample_dump(uint32_t kind, const uint64_t* directions, uint32_t dims, const bf_sample_stream_index* indices,
+hipError_t bfk_sample_dump(const sampler_ctx* sampler, const bf_sample_stream_index* indices,
                            const uint64_t* dimensions, uint32_t count, float* out, hipStream_t s) {
     if (count == 0) return hipSuccess;
-    sampler_ctx sc;
-    sc.kind = kind;
-    sc.sobol_dims = dims;
-    sc.directions = directions;
-    hipLaunchKernelGGL(k_sample_dump, dim3(blocks_for(count, BF_BLOCK)), dim3(BF_BLOCK), 0, s, sc, indices, dimensions, count,
+    hipLaunchKernelGGL(k_sample_dump, dim3(blocks_for(count, BF_BLOCK)), dim3(BF_BLOCK), 0, s, *sampler, indices, dimensions, count,
                        out);
     return hipGetLastError();
 }

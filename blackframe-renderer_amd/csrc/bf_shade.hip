@@ -252,9 +252,11 @@ BF_D bool contract_point_endpoint(v3f p, v3f err, v3f to_light, v3f& out) {
 BF_D bool sample_light(const bf_transport_params& P, const bf_dev_scene& S, const sample_key& k, uint64_t first_dim,
                        const float* wl, uint32_t visibility, const surface_t& surf, incident_t& inc) {
     inc.present = false;
-    const float u_sel = sample_1d(P.sampler, k, first_dim + 0);
     uint32_t li;
     float sel;
+    /* a power-of-two number of lights (up to 256) is selected by the sample's leading bits alone */
+    const bool head = !S.light_cdf && S.light_count <= 256u && (S.light_count & (S.light_count - 1u)) == 0u;
+    const float u_sel = head ? sample_head(P.sampler, k, first_dim + 0) : sample_1d(P.sampler, k, first_dim + 0);
     if (S.light_cdf ? !cdf_light_selection(S.light_cdf, S.light_count, u_sel, li, sel)
                     : !uniform_light_selection(S.light_count, u_sel, li, sel))
         return false;
@@ -743,16 +745,19 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
             cont_pending = false;
             pending_term = BF_TERM_ZERO_THROUGHPUT;
         } else if (P.rr_enabled && depth >= P.rr_first) {
-            const float u = sample_1d(P.sampler, key, first_dim + 9);
-            bool survived;
             float* frozen = J.tape_survival ? J.tape_survival + path_of(J, slot) * J.survival_stride + vertex : nullptr;
-            if (frozen && J.survival_mode == BF_SURVIVAL_REPLAY) {
-                if (!russian_roulette_at(beta4, *frozen, u, survived)) return fail_path(P, J, slot, 32);
-            } else {
-                float p;
-                if (!russian_roulette(beta4, eta_scale, u, P.rr_min, P.rr_max, survived, p)) return fail_path(P, J, slot, 32);
-                if (frozen && !ADJ) *frozen = p;
+            const bool replay = frozen && J.survival_mode == BF_SURVIVAL_REPLAY;
+            float p = 1.0f;
+            bool survived = false;
+            if (replay) {
+                p = *frozen;
+                if (!finite_nonnegative4(beta4) || !bf_isfinite(p) || !(p > 0.0f) || p > 1.0f) return fail_path(P, J, slot, 32);
+            } else if (!roulette_probability(beta4, eta_scale, P.rr_min, P.rr_max, p)) {
+                return fail_path(P, J, slot, 32);
             }
+            if (!sample_below(P.sampler, key, first_dim + 9, p, survived) || (survived && !roulette_survive(beta4, p)))
+                return fail_path(P, J, slot, 32);
+            if (frozen && !replay && !ADJ) *frozen = p;
             if (!survived) {
                 cont_pending = false;
                 pending_term = BF_TERM_RUSSIAN_ROULETTE;

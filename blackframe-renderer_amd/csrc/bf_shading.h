@@ -233,23 +233,27 @@ BF_D bool geometric_event_support(v3f ng, v3f wo, v3f wi, uint32_t lobes, bool& 
     return true;
 }
 
-/* uniform selection: TransportDevice.cuh:479-551 */
+/* uniform selection: TransportDevice.cuh:479-551. Light i owns [i / count, (i + 1) / count) with
+ * binary32 boundaries; u * count lands on the light or beside it, so the boundaries around that
+ * guess replace the reference's binary search over all of them. */
 BF_D bool uniform_light_selection(uint32_t count, float u, uint32_t& index, float& probability) {
     if (count == 0 || !bf_isfinite(u) || u < 0.0f || !(u < 1.0f) || count > (1u << 24)) return false;
     const float sc = (float)count;
-    uint32_t first = 1, last = count + 1;
-    while (first < last) {
-        const uint32_t mid = first + (last - first) / 2;
-        const float boundary = mid == count ? 1.0f : (float)mid / sc;
-        if (!(u < boundary)) first = mid + 1;
-        else last = mid;
+    uint32_t i = (uint32_t)(u * sc);
+    i = i < count ? i : count - 1u;
+    float lower = (float)i / sc, upper = i + 1u == count ? 1.0f : (float)(i + 1u) / sc;
+    while (u < lower) {
+        --i;
+        upper = lower;
+        lower = (float)i / sc;
     }
-    if (first == 0 || first > count) return false;
-    const uint32_t i = first - 1;
-    const float lower = i == 0 ? 0.0f : (float)i / sc;
-    const float upper = first == count ? 1.0f : (float)first / sc;
+    while (!(u < upper)) {
+        ++i;
+        lower = upper;
+        upper = i + 1u == count ? 1.0f : (float)(i + 1u) / sc;
+    }
     const float interval = upper - lower;
-    if (!(lower <= u) || !(u < upper) || !(interval > 0.0f) || interval > 1.0f) return false;
+    if (!(interval > 0.0f) || interval > 1.0f) return false;
     index = i;
     probability = interval;
     return true;

@@ -56,8 +56,15 @@ BF_HD double bf_bits_double(uint64_t bits) {
     return value;
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+/* gfx950 classifies and takes floats apart in one instruction each (the values of the bit forms
+ * below for every float; ldexp rounds once, to nearest even, as a correctly rounded one must) */
+BF_HD int bf_isnan(float v) { return __builtin_isnan(v); }
+BF_HD int bf_isfinite(float v) { return __builtin_isfinite(v); }
+#else
 BF_HD int bf_isnan(float v) { return (bf_float_bits(v) & 0x7FFFFFFFu) > 0x7F800000u; }
 BF_HD int bf_isfinite(float v) { return (bf_float_bits(v) & 0x7F800000u) != 0x7F800000u; }
+#endif
 BF_HD int bf_isnand(double v) { return (bf_double_bits(v) & 0x7FFFFFFFFFFFFFFFull) > 0x7FF0000000000000ull; }
 BF_HD int bf_isfinited(double v) { return (bf_double_bits(v) & 0x7FF0000000000000ull) != 0x7FF0000000000000ull; }
 BF_HD int bf_signbit(float v) { return (bf_float_bits(v) >> 31) != 0u; }
@@ -96,6 +103,13 @@ BF_HD double bf_next_down(double x) {
     return bf_bits_double(x > 0.0 ? b - 1ull : b + 1ull);
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+BF_HD float bf_frexpf(float x, int* exponent) {
+    *exponent = __builtin_amdgcn_frexp_expf(x);
+    return __builtin_amdgcn_frexp_mantf(x);
+}
+BF_HD float bf_ldexpf(float x, int n) { return __builtin_amdgcn_ldexpf(x, n); }
+#else
 /* frexpf for finite non-zero x: x = m * 2^e with 0.5 <= |m| < 1 (subnormals normalised). */
 BF_HD float bf_frexpf(float x, int* exponent) {
     uint32_t b = bf_float_bits(x);
@@ -135,6 +149,7 @@ BF_HD float bf_ldexpf(float x, int n) {
     }
     return (float)scaled;
 }
+#endif
 
 BF_HD float bf_hypotf(float x, float y) {
     double dx = (double)x;
