@@ -14,16 +14,20 @@ struct closure_t {
     float parameters[10];
 };
 
+/* A material's closures at a vertex, N at most. With N = 1 every index below is a constant, so the
+ * records stay in registers; with BF_MAX_CLOSURES they are indexed in scratch. */
+template <uint32_t N>
 struct mixture_t {
     uint32_t active_count;
-    closure_t closures[BF_MAX_CLOSURES];
-    float probabilities[BF_MAX_CLOSURES];
-    float cdf[BF_MAX_CLOSURES + 1];
+    closure_t closures[N];
+    float probabilities[N];
+    float cdf[N + 1];
 };
 
+template <uint32_t N>
 struct filter_t {
-    uint32_t source_indices[BF_MAX_CLOSURES];
-    uint32_t allowed[BF_MAX_CLOSURES];
+    uint32_t source_indices[N];
+    uint32_t allowed[N];
     uint32_t source_count;
     uint32_t blocked;
     int status;
@@ -364,18 +368,20 @@ BF_D bool compensated_add(float value, float& sum, float& correction) {
     return true;
 }
 
-BF_D bool mixture_nonblack(const mixture_t& m) {
-    for (uint32_t c = 0; c < m.active_count; ++c)
+template <uint32_t N>
+BF_D bool mixture_nonblack(const mixture_t<N>& m) {
+    for (uint32_t c = 0; c < N && c < m.active_count; ++c)
         for (int k = 0; k < 4; ++k)
             if (m.closures[c].weight[k] != 0.0f) return true;
     return false;
 }
 
 /* TransportLobesDevice.cuh:2863-2887 */
-BF_D int mixture_eval(const mixture_t& m, const filter_t& f, v3f wo, v3f wi, float* out) {
+template <uint32_t N>
+BF_D int mixture_eval(const mixture_t<N>& m, const filter_t<N>& f, v3f wo, v3f wi, float* out) {
     if (!unit_vector(wo) || !unit_vector(wi)) return BF_L_INVALID;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t i = 0; i < m.active_count; ++i) {
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
         float comp[4];
         const int st = record_eval(m.closures[i], f.allowed[i], wo, wi, comp);
         if (st != BF_L_OK) return st;
@@ -392,15 +398,16 @@ BF_D int mixture_eval(const mixture_t& m, const filter_t& f, v3f wo, v3f wi, flo
 }
 
 /* TransportLobesDevice.cuh:2889-2958 */
-BF_D int mixture_pdf(const mixture_t& m, const filter_t& f, v3f wo, v3f wi, float& out) {
+template <uint32_t N>
+BF_D int mixture_pdf(const mixture_t<N>& m, const filter_t<N>& f, v3f wo, v3f wi, float& out) {
     if (!unit_vector(wo) || !unit_vector(wi)) return BF_L_INVALID;
     if (m.active_count == 0) {
         out = 0.0f;
         return BF_L_OK;
     }
-    float conditional[BF_MAX_CLOSURES];
+    float conditional[N];
     float maximum = 0.0f;
-    for (uint32_t i = 0; i < m.active_count; ++i) {
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
         float p;
         const int st = record_pdf(m.closures[i], f.allowed[i], wo, wi, p);
         if (st != BF_L_OK) return st;
@@ -408,7 +415,7 @@ BF_D int mixture_pdf(const mixture_t& m, const filter_t& f, v3f wo, v3f wi, floa
         conditional[i] = p;
         maximum = fmaxf(maximum, p);
     }
-    if (m.active_count == 1) {
+    if (N == 1u || m.active_count == 1) {
         out = conditional[0];
         return BF_L_OK;
     }
@@ -417,7 +424,7 @@ BF_D int mixture_pdf(const mixture_t& m, const filter_t& f, v3f wo, v3f wi, floa
         return BF_L_OK;
     }
     float sum = 0.0f, correction = 0.0f;
-    for (uint32_t i = 0; i < m.active_count; ++i) {
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
         const float ratio = conditional[i] / maximum;
         float contribution;
         if (!checked_product(m.probabilities[i], ratio, contribution) || !compensated_add(contribution, sum, correction))
@@ -442,7 +449,8 @@ BF_D uint32_t depth_blocked(const uint32_t* limits, const uint32_t* counters, ui
 }
 
 /* TransportLobesDevice.cuh:2643-2718 */
-BF_D bool build_filtered_distribution(mixture_t& m) {
+template <uint32_t N>
+BF_D bool build_filtered_distribution(mixture_t<N>& m) {
     if (m.active_count == 0) return true;
     if (m.active_count == 1) {
         m.probabilities[0] = 1.0f;
@@ -451,15 +459,15 @@ BF_D bool build_filtered_distribution(mixture_t& m) {
         return true;
     }
     float ts = 0.0f, tc = 0.0f;
-    for (uint32_t i = 0; i < m.active_count; ++i)
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i)
         if (!compensated_add(m.probabilities[i], ts, tc)) return false;
     const float total = ts + tc;
     if (!bf_isfinite(total) || !(total > 0.0f)) return false;
     const uint64_t scale = 1ull << 24;
-    uint64_t masses[BF_MAX_CLOSURES];
-    float rem[BF_MAX_CLOSURES];
+    uint64_t masses[N];
+    float rem[N];
     uint64_t base_mass = 0;
-    for (uint32_t i = 0; i < m.active_count; ++i) {
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
         const float normalized = m.probabilities[i] / total;
         if (!bf_isfinite(normalized) || !(normalized > 0.0f) || !(normalized < 1.0f)) return false;
         const float scaled = bf_ldexpf(normalized, 24);
@@ -472,16 +480,16 @@ BF_D bool build_filtered_distribution(mixture_t& m) {
     }
     if (base_mass > scale) return false;
     float rs = 0.0f, rc = 0.0f;
-    for (uint32_t i = 0; i < m.active_count; ++i)
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i)
         if (!compensated_add(rem[i], rs, rc)) return false;
     const uint64_t missing = scale - base_mass;
     const float rtotal = rs + rc;
     if (missing > m.active_count || fabsf(rtotal - (float)missing) > 0.5f + 0x1p-23f * 16.0f) return false;
-    bool received[BF_MAX_CLOSURES];
-    for (uint32_t i = 0; i < BF_MAX_CLOSURES; ++i) received[i] = false;
+    bool received[N];
+    for (uint32_t i = 0; i < N; ++i) received[i] = false;
     for (uint64_t unit = 0; unit < missing; ++unit) {
         uint32_t sel = m.active_count;
-        for (uint32_t i = 0; i < m.active_count; ++i) {
+        for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
             if (received[i] || !(rem[i] > 0.0f)) continue;
             if (sel == m.active_count || rem[i] > rem[sel]) sel = i;
         }
@@ -491,7 +499,7 @@ BF_D bool build_filtered_distribution(mixture_t& m) {
     }
     uint64_t cumulative = 0;
     m.cdf[0] = 0.0f;
-    for (uint32_t i = 0; i < m.active_count; ++i) {
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
         if (masses[i] == 0 || cumulative > scale - masses[i]) return false;
         cumulative += masses[i];
         m.probabilities[i] = bf_ldexpf((float)masses[i], -24);
@@ -501,8 +509,9 @@ BF_D bool build_filtered_distribution(mixture_t& m) {
 }
 
 /* TransportLobesDevice.cuh:2720-2795 */
-BF_D void filter_by_depth(mixture_t& m, const uint32_t* limits, const uint32_t* counters, uint32_t expected_total,
-                          filter_t& r) {
+template <uint32_t N>
+BF_D void filter_by_depth(mixture_t<N>& m, const uint32_t* limits, const uint32_t* counters, uint32_t expected_total,
+                          filter_t<N>& r) {
     r.source_count = m.active_count;
     r.blocked = 0;
     r.status = BF_L_OK;
@@ -514,7 +523,7 @@ BF_D void filter_by_depth(mixture_t& m, const uint32_t* limits, const uint32_t* 
         return;
     }
     uint32_t filtered = 0;
-    for (uint32_t si = 0; si < r.source_count; ++si) {
+    for (uint32_t si = 0; si < N && si < r.source_count; ++si) {
         const closure_t src = m.closures[si];
         const float prob = m.probabilities[si];
         uint32_t allowed = 0;
@@ -535,16 +544,17 @@ BF_D void filter_by_depth(mixture_t& m, const uint32_t* limits, const uint32_t* 
             else r.blocked |= blocked;
         }
         if (allowed == 0) continue;
-        m.closures[filtered] = src;
-        m.probabilities[filtered] = prob;
-        r.source_indices[filtered] = si;
-        r.allowed[filtered] = allowed;
+        const uint32_t at = N == 1u ? 0u : filtered;
+        m.closures[at] = src;
+        m.probabilities[at] = prob;
+        r.source_indices[at] = si;
+        r.allowed[at] = allowed;
         ++filtered;
     }
     m.active_count = filtered;
     if (filtered == r.source_count) return;
-    for (uint32_t i = filtered; i < BF_MAX_CLOSURES; ++i) m.probabilities[i] = 0.0f;
-    for (uint32_t i = 0; i <= BF_MAX_CLOSURES; ++i) m.cdf[i] = 0.0f;
+    for (uint32_t i = filtered; i < N; ++i) m.probabilities[N == 1u ? 0u : i] = 0.0f;
+    for (uint32_t i = 0; i <= N; ++i) m.cdf[i] = 0.0f;
     if (!build_filtered_distribution(m)) r.status = BF_L_NOT_REPRESENTABLE;
 }
 
@@ -560,7 +570,8 @@ struct mixture_sample_t {
 };
 
 /* TransportLobesDevice.cuh:2960-3062 */
-BF_D void sample_mixture(const mixture_t& m, const filter_t& f, v3f wo, float component, float u, float v,
+template <uint32_t N>
+BF_D void sample_mixture(const mixture_t<N>& m, const filter_t<N>& f, v3f wo, float component, float u, float v,
                          mixture_sample_t& out) {
     out.eta_scale = 1.0f;
     out.discrete = 0u;
@@ -577,7 +588,7 @@ BF_D void sample_mixture(const mixture_t& m, const filter_t& f, v3f wo, float co
         return;
     }
     uint32_t sel = m.active_count;
-    for (uint32_t i = 0; i < m.active_count; ++i) {
+    for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
         if (component < m.cdf[i + 1]) {
             sel = i;
             break;
@@ -587,6 +598,7 @@ BF_D void sample_mixture(const mixture_t& m, const filter_t& f, v3f wo, float co
         out.status = BF_L_NOT_REPRESENTABLE;
         return;
     }
+    if (N == 1u) sel = 0u;
     const float event = (component - m.cdf[sel]) / m.probabilities[sel];
     if (!bf_isfinite(event) || event < 0.0f || !(event < 1.0f)) {
         out.status = BF_L_NOT_REPRESENTABLE;
@@ -601,7 +613,7 @@ BF_D void sample_mixture(const mixture_t& m, const filter_t& f, v3f wo, float co
     out.incoming = s.incoming;
     out.lobes = s.lobes;
     out.eta_scale = s.eta_scale;
-    if (m.active_count == 1) {
+    if (N == 1u || m.active_count == 1) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) out.value[k] = s.value[k];
         out.pdf = s.pdf;
@@ -627,7 +639,7 @@ BF_D void sample_mixture(const mixture_t& m, const filter_t& f, v3f wo, float co
         float sums[4] = {0.0f, 0.0f, 0.0f, 0.0f}, corrections[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         float psum = 0.0f, pcorrection = 0.0f;
         uint32_t matching = 0;
-        for (uint32_t i = 0; i < m.active_count; ++i) {
+        for (uint32_t i = 0; i < N && i < m.active_count; ++i) {
             const uint32_t kind = m.closures[i].kind;
             if (kind != BF_CLOSURE_SPECULAR_REFLECTION && kind != BF_CLOSURE_SPECULAR_TRANSMISSION) continue;
             /* record_sample restricted to the two delta kinds: the microfacet samplers are not

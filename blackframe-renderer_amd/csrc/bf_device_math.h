@@ -31,7 +31,7 @@ struct v3f {
 };
 
 BF_D v3f mk(float x, float y, float z) { return v3f{x, y, z}; }
-BF_D bool fin3(v3f v) { return bf_isfinite(v.x) && bf_isfinite(v.y) && bf_isfinite(v.z); }
+BF_D bool fin3(v3f v) { return (bool)(bf_isfinite(v.x) & bf_isfinite(v.y) & bf_isfinite(v.z)); }
 BF_D v3f add3(v3f a, v3f b) { return mk(a.x + b.x, a.y + b.y, a.z + b.z); }
 BF_D v3f sub3(v3f a, v3f b) { return mk(a.x - b.x, a.y - b.y, a.z - b.z); }
 BF_D v3f mul3(v3f a, float s) { return mk(a.x * s, a.y * s, a.z * s); }
@@ -120,23 +120,24 @@ BF_D bool owen_open(const sampler_ctx& sc, const sample_key& k, uint64_t sobol_d
     return true;
 }
 
-/* Sample bits of depths [FROM, TO) (leading bit first), in the low TO - FROM bits: each is the input's
- * bit flipped by bit 63 of mix_bits(key ^ node), node = 1 followed by the input's leading bits. The
- * last xor-shift of mix_bits leaves bit 63 alone, and of the last product only the high word is
- * formed. */
+/* Sample bit of one depth: the input's bit flipped by bit 63 of mix_bits(key ^ node), node = 1 followed by
+ * the input's leading bits. The last xor-shift of mix_bits leaves bit 63 alone, and of the last
+ * product only the high word is formed. Returns it in bit 31. */
+BF_D uint32_t owen_flip(const owen_stream& o, uint32_t depth) {
+    const uint32_t v = o.key_low ^ ((o.input | 0x1000000u) >> (24u - depth));
+    const uint64_t w = (uint64_t)v * 0x1CE4E5B9u + o.product;
+    const uint32_t wl = (uint32_t)w, wh = (uint32_t)(w >> 32) + v * 0xBF58476Du;
+    const uint32_t xl = wl ^ __builtin_amdgcn_alignbit(wh, wl, 27u), xh = wh ^ (wh >> 27);
+    return __umulhi(xl, 0x133111EBu) + xl * 0x94D049BBu + xh * 0x133111EBu;
+}
+
+/* Sample bits of depths [FROM, TO) (leading bit first), in the low TO - FROM bits. Rolled loops: the
+ * shade kernels are longer than the instruction cache. */
 template <uint32_t FROM, uint32_t TO>
 BF_D uint32_t owen_bits(const owen_stream& o) {
-    const uint32_t tagged = o.input | 0x1000000u;
     uint32_t flips = 0u;
-#pragma unroll
-    for (uint32_t depth = FROM; depth < TO; ++depth) {
-        const uint32_t v = o.key_low ^ (tagged >> (24u - depth));
-        const uint64_t w = (uint64_t)v * 0x1CE4E5B9u + o.product;
-        const uint32_t wl = (uint32_t)w, wh = (uint32_t)(w >> 32) + v * 0xBF58476Du;
-        const uint32_t xl = wl ^ __builtin_amdgcn_alignbit(wh, wl, 27u), xh = wh ^ (wh >> 27);
-        const uint32_t yh = __umulhi(xl, 0x133111EBu) + xl * 0x94D049BBu + xh * 0x133111EBu;
-        flips = (flips << 1) | (yh >> 31);
-    }
+#pragma unroll 4
+    for (uint32_t depth = FROM; depth < TO; ++depth) flips = (flips << 1) | (owen_flip(o, depth) >> 31);
     return ((o.input >> (24u - TO)) & ((1u << (TO - FROM)) - 1u)) ^ flips;
 }
 
@@ -151,6 +152,31 @@ BF_D float sample_1d(const sampler_ctx& sc, const sample_key& k, uint64_t dim) {
         return owen_open(sc, k, sobol_dimension(dim), o) ? (float)owen_bits<0u, 24u>(o) * 0x1p-24f : -1.0f;
     }
     return (float)(indexed_bits(k, dim) >> 40) * 0x1p-24f;
+}
+
+/* sample_1d of several dimensions, their scrambles in one loop. */
+template <int COUNT>
+BF_D void sample_each(const sampler_ctx& sc, const sample_key& k, const uint64_t* dims, float* out) {
+    if (sc.kind == BF_SAMPLER_SOBOL_OWEN) {
+        owen_stream o[COUNT];
+        bool ok[COUNT];
+        uint32_t flips[COUNT];
+#pragma unroll
+        for (int j = 0; j < COUNT; ++j) {
+            o[j] = owen_stream{0u, 0u, 0u};
+            ok[j] = owen_open(sc, k, sobol_dimension(dims[j]), o[j]);
+            flips[j] = 0u;
+        }
+#pragma unroll 1
+        for (uint32_t depth = 0; depth < 24u; ++depth)
+#pragma unroll
+            for (int j = 0; j < COUNT; ++j) flips[j] = (flips[j] << 1) | (owen_flip(o[j], depth) >> 31);
+#pragma unroll
+        for (int j = 0; j < COUNT; ++j) out[j] = ok[j] ? (float)(o[j].input ^ flips[j]) * 0x1p-24f : -1.0f;
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < COUNT; ++j) out[j] = (float)(indexed_bits(k, dims[j]) >> 40) * 0x1p-24f;
 }
 
 /* sample_1d(dim) < p, formed from as many leading bits as decide it (eight, but for one lane in
@@ -179,101 +205,74 @@ BF_D float sample_head(const sampler_ctx& sc, const sample_key& k, uint64_t dim)
 }
 
 /* ---- checked arithmetic: TransportDevice.cuh:196-259 --------------------------------------- */
+/* The helpers of the shade stage evaluate every condition and combine the verdicts without branches:
+ * a failed check is rare, a value computed past one is never used, and nested early exits cost the
+ * kernels more scalar mask arithmetic than the skipped operations. */
 BF_D bool checked_product(float l, float r, float& out) {
-    if (!bf_isfinite(l) || l < 0.0f || !bf_isfinite(r) || r < 0.0f) return false;
     const float p = l * r;
-    if (!bf_isfinite(p) || p < 0.0f || (l != 0.0f && r != 0.0f && p == 0.0f)) return false;
     out = p;
-    return true;
+    return bf_isfinite(l) & (l >= 0.0f) & bf_isfinite(r) & (r >= 0.0f) & bf_isfinite(p) & (p >= 0.0f) &
+           ((l == 0.0f) | (r == 0.0f) | (p != 0.0f));
 }
 
 template <int NN, int ND>
 BF_D int checked_product_quotient(const float (&num)[NN], const float (&den)[ND], float& out) {
-    bool has_zero = false;
-#pragma unroll
-    for (int i = 0; i < ND; ++i)
-        if (!bf_isfinite(den[i]) || !(den[i] > 0.0f)) return BF_L_INVALID;
-#pragma unroll
-    for (int i = 0; i < NN; ++i) {
-        if (!bf_isfinite(num[i]) || num[i] < 0.0f) return BF_L_INVALID;
-        has_zero = has_zero || num[i] == 0.0f;
-    }
-    if (has_zero) {
-        out = 0.0f;
-        return BF_L_OK;
-    }
+    bool has_zero = false, valid = true;
     float significand = 1.0f;
     int exponent = 0;
 #pragma unroll
     for (int i = 0; i < NN; ++i) {
+        valid = valid & (bool)bf_isfinite(num[i]) & (num[i] >= 0.0f);
+        has_zero = has_zero | (num[i] == 0.0f);
         int e;
         significand *= bf_frexpf(num[i], &e);
         exponent += e;
     }
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
+        valid = valid & (bool)bf_isfinite(den[i]) & (den[i] > 0.0f);
         int e;
         significand /= bf_frexpf(den[i], &e);
         exponent -= e;
     }
-    if (!bf_isfinite(significand) || !(significand > 0.0f)) return BF_L_NOT_REPRESENTABLE;
     int ne;
-    significand = bf_frexpf(significand, &ne);
-    exponent += ne;
-    const float r = bf_ldexpf(significand, exponent);
-    if (!bf_isfinite(r) || !(r > 0.0f)) return BF_L_NOT_REPRESENTABLE;
-    out = r;
-    return BF_L_OK;
+    const float scaled = bf_frexpf(significand, &ne);
+    const float r = bf_ldexpf(scaled, exponent + ne);
+    const bool representable = bf_isfinite(significand) & (significand > 0.0f) & bf_isfinite(r) & (r > 0.0f);
+    out = has_zero ? 0.0f : r;
+    return !valid ? BF_L_INVALID : (has_zero | representable ? BF_L_OK : BF_L_NOT_REPRESENTABLE);
 }
 
 /* TransportDevice.cuh:552-590 */
 BF_D bool joint_light_pdf(float selection, float conditional, float& out) {
-    if (!bf_isfinite(selection) || !(selection > 0.0f) || selection > 1.0f || !bf_isfinite(conditional) ||
-        conditional < 0.0f)
-        return false;
-    if (conditional == 0.0f) {
-        out = 0.0f;
-        return true;
-    }
+    const bool valid = bf_isfinite(selection) & (selection > 0.0f) & (selection <= 1.0f) & bf_isfinite(conditional) &
+                       (conditional >= 0.0f);
     const float num[2] = {selection, conditional};
     const float den[1] = {1.0f};
-    return checked_product_quotient(num, den, out) == BF_L_OK;
+    return valid & (checked_product_quotient(num, den, out) == BF_L_OK);
 }
 
 /* TransportDevice.cuh:592-628 */
 BF_D bool ratio_at_most_one(float n, float d, bool squared, float& out) {
-    if (!bf_isfinite(n) || !(n > 0.0f) || !bf_isfinite(d) || !(d > 0.0f) || n > d) return false;
     int ne, de;
     const float ns = bf_frexpf(n, &ne);
     const float ds = bf_frexpf(d, &de);
     const float ratio = ns / ds;
-    const float r = squared ? bf_ldexpf(ratio * ratio, 2 * (ne - de)) : bf_ldexpf(ratio, ne - de);
-    if (!bf_isfinite(r) || r < 0.0f || r > 1.0f) return false;
+    const float r = bf_ldexpf(squared ? ratio * ratio : ratio, squared ? 2 * (ne - de) : ne - de);
     out = r;
-    return true;
+    return bf_isfinite(n) & (n > 0.0f) & bf_isfinite(d) & (d > 0.0f) & (n <= d) & bf_isfinite(r) & (r >= 0.0f) & (r <= 1.0f);
 }
 
 /* TransportDevice.cuh:630-689 */
 BF_D bool mis_weight(uint32_t heuristic, float sampled, float competing, float& out) {
-    if (!bf_isfinite(sampled) || !(sampled > 0.0f) || !bf_isfinite(competing) || competing < 0.0f || heuristic > 1u)
-        return false;
-    if (competing == 0.0f) {
-        out = 1.0f;
-        return true;
-    }
+    const bool less = sampled < competing;
     float ratio;
-    if (sampled < competing) {
-        if (!ratio_at_most_one(sampled, competing, heuristic == 1u, ratio) || !(ratio > 0.0f)) return false;
-        const float w = ratio / (1.0f + ratio);
-        if (!bf_isfinite(w) || !(w > 0.0f) || w > 1.0f) return false;
-        out = w;
-        return true;
-    }
-    if (!ratio_at_most_one(competing, sampled, heuristic == 1u, ratio)) return false;
-    const float w = 1.0f / (1.0f + ratio);
-    if (!bf_isfinite(w) || !(w > 0.0f) || w > 1.0f) return false;
-    out = w;
-    return true;
+    const bool ok = ratio_at_most_one(less ? sampled : competing, less ? competing : sampled, heuristic == 1u, ratio);
+    const float w = (less ? ratio : 1.0f) / (1.0f + ratio);
+    const bool alone = competing == 0.0f;
+    out = alone ? 1.0f : w;
+    return bf_isfinite(sampled) & (sampled > 0.0f) & bf_isfinite(competing) & (competing >= 0.0f) & (heuristic <= 1u) &
+           (alone | (ok & (!less | (ratio > 0.0f)) & bf_isfinite(w) & (w > 0.0f) & (w <= 1.0f)));
 }
 
 /* Russian roulette (TransportDevice.cuh:711-782): the survival probability clamp(max(throughput) *
@@ -317,21 +316,18 @@ BF_D bool finite_nonnegative4(float4 t) {
 
 /* TransportDevice.cuh:327-333 */
 BF_D bool unit_vector(v3f d) {
-    if (!fin3(d)) return false;
     const float sq = fmaf(d.x, d.x, fmaf(d.y, d.y, d.z * d.z));
-    return bf_isfinite(sq) && fabsf(sq - 1.0f) <= 128.0f * BF_EPS;
+    return fin3(d) & bf_isfinite(sq) & (fabsf(sq - 1.0f) <= 128.0f * BF_EPS);
 }
 
 /* CudaWavefrontStages.cu:326-349 */
 BF_D bool normalize3(v3f v, v3f& out) {
-    if (!fin3(v)) return false;
     const float m = fmaxf(fabsf(v.x), fmaxf(fabsf(v.y), fabsf(v.z)));
-    if (!bf_isfinite(m) || m == 0.0f) return false;
     const v3f s = mk(v.x / m, v.y / m, v.z / m);
     const float mag = sqrtf(dot3(s, s));
-    if (!bf_isfinite(mag) || !(mag > 0.0f)) return false;
+    const bool finite = fin3(v);
     out = mk(s.x / mag, s.y / mag, s.z / mag);
-    return fin3(out);
+    return finite & bf_isfinite(m) & (m != 0.0f) & bf_isfinite(mag) & (mag > 0.0f) & fin3(out);
 }
 
 BF_D bool valid_surface_event(uint32_t bits) {

@@ -59,14 +59,36 @@
 #ifndef BF_SHADOW_REFILL
 #define BF_SHADOW_REFILL 32u /* the same for an any-hit wave (16, 24 measured slower, 40 equal) */
 #endif
+/* Buckets of the shade order: 0-3 are shaded by the general kernel (0 several closures, 1 rough
+ * diffuse, 2 mirror, 3 refraction), 4-6 by the kernel of their one closure. */
+#define BF_SHADE_BUCKETS 8u
+#define BF_BUCKET_LAMBERT 4u
+#define BF_BUCKET_CONDUCTOR 5u
+#define BF_BUCKET_DIELECTRIC 6u
+
+/* Shade kernels of a mode: any material, Lambertian materials, materials of one closure of a kind
+ * that has a bucket. The last two are also what one item is shaded as. */
+#define BF_SHADE_ANY 0u
+#define BF_SHADE_LAMBERT 1u
+#define BF_SHADE_SINGLE 2u
+#define BF_SHADE_KERNELS 3u
+#define BF_SHADE_CONDUCTOR 3u
+#define BF_SHADE_DIELECTRIC 4u
+#define BF_SHADE_MODES 4u
+/* Register budgets of the shade kernels, in waves per SIMD. What a lane spills is read and written
+ * through the vector memory path, which costs more than the waves it would buy: with a budget of 2 the
+ * single-closure kernels keep nearly everything in registers (the shade stage of a 1920x1080x64 frame
+ * of 1024 instances 65.2 ms, against 75.0 with 3 waves, 83.1 with 4 and 107 with 5; of a 256x256x16
+ * frame with maps 8.9 ms, against 16.8 with 3 and 21.2 with 4). The general kernel indexes its closures in
+ * scratch whatever its budget and gains from the third wave (9.1 to 8.7 ms in an adjoint replay). */
 #ifndef BF_SHADE_WAVES_PER_SIMD
-#define BF_SHADE_WAVES_PER_SIMD 3 /* register budget of the forward shade kernels (waves per SIMD; 1 and 2 measured slower) */
+#define BF_SHADE_WAVES_PER_SIMD 3 /* any material */
+#endif
+#ifndef BF_SHADE_SINGLE_WAVES
+#define BF_SHADE_SINGLE_WAVES 2 /* materials of one closure */
 #endif
 #ifndef BF_SHADE_BLOCK
 #define BF_SHADE_BLOCK 256u /* lanes per shade workgroup (64 measured slower, 128 equal) */
-#endif
-#ifndef BF_ADJOINT_SHADE_WAVES_PER_SIMD
-#define BF_ADJOINT_SHADE_WAVES_PER_SIMD 3 /* the adjoint shade kernel (1 and 2 measured slower) */
 #endif
 
 /* A punctual light with its spot-cone cosines formed once on the host. */
@@ -187,6 +209,7 @@ typedef struct bf_dev_scene {
     const bf_dev_image* images;
     const float* image_texels;
     const bf_surface_maps_desc* maps;
+    const uint8_t* material_buckets;   /* shade-order bucket of each material */
     uint32_t exact_walk;               /* boxes or depths outside the bound engine's range: every launch
                                         * takes the step-exact walk */
 } bf_dev_scene;

@@ -453,6 +453,7 @@ struct bf_hip_scene {
     uint32_t max_blas_depth = 0, tlas_depth = 0;
     uint32_t light_count = 0;
     std::vector<uint32_t> texture_floats; /* width * height * channels per texture slot */
+    uint32_t shade_buckets = 0;           /* bit b: some instance's material is in shade bucket b */
     bool has_maps = false;                /* some material has a normal or bump map */
     bool sampled = false;                 /* holds point-sampled spectra at sampled_wavelengths */
     float sampled_wavelengths[BF_SPECTRUM_LANES] = {};
@@ -895,6 +896,25 @@ int build_scene(const bf_scene_desc* d, bf_hip_scene* s, bool upload) {
     s->texture_floats.clear();
     for (uint32_t t = 0; t < d->texture_count; ++t)
         s->texture_floats.push_back(d->textures[t].width * d->textures[t].height * d->textures[t].channels);
+    /* -- shade buckets: a material of one closure, selected for certain, by its kind -- */
+    std::vector<uint8_t> material_buckets(d->material_count, 0u);
+    for (uint32_t m = 0; m < d->material_count; ++m) {
+        const bf_material_desc& M = d->materials[m];
+        if (M.closure_count != 1u || M.closure_offset >= d->closure_count || M.probabilities[0] != 1.0f || M.cdf[0] != 0.0f ||
+            M.cdf[1] != 1.0f)
+            continue;
+        switch (d->closures[M.closure_offset].kind) {
+        case BF_CLOSURE_LAMBERTIAN: material_buckets[m] = BF_BUCKET_LAMBERT; break;
+        case BF_CLOSURE_ROUGH_CONDUCTOR: material_buckets[m] = BF_BUCKET_CONDUCTOR; break;
+        case BF_CLOSURE_ROUGH_DIELECTRIC: material_buckets[m] = BF_BUCKET_DIELECTRIC; break;
+        case BF_CLOSURE_ROUGH_DIFFUSE: material_buckets[m] = 1u; break;
+        case BF_CLOSURE_SPECULAR_REFLECTION: material_buckets[m] = 2u; break;
+        case BF_CLOSURE_SPECULAR_TRANSMISSION: material_buckets[m] = 3u; break;
+        default: break;
+        }
+    }
+    s->shade_buckets = 0u;
+    for (uint32_t i = 0; i < d->instance_count; ++i) s->shade_buckets |= 1u << material_buckets[d->instances[i].material_index];
     bool textured = false;
     for (uint32_t c = 0; c < d->closure_count; ++c) {
         const bf_closure_desc& C = d->closures[c];
@@ -1002,6 +1022,7 @@ int build_scene(const bf_scene_desc* d, bf_hip_scene* s, bool upload) {
     const size_t o_uv = A.add(d->uvs, d->vertex_count * 2 * sizeof(float));
     const size_t o_idx = A.add(d->indices, d->triangle_count * 3 * sizeof(uint32_t));
     const size_t o_mat = A.add(d->materials, d->material_count * sizeof(bf_material_desc));
+    const size_t o_buck = A.add(material_buckets.data(), material_buckets.size());
     const size_t o_clo = A.add(d->closures, d->closure_count * sizeof(bf_closure_desc));
     const size_t o_spe = A.add(d->spectra, d->spectrum_count * sizeof(bf_spectrum_desc));
     const size_t o_spv = A.add(d->spectrum_values, d->spectrum_value_count * sizeof(float));
@@ -1053,6 +1074,7 @@ int build_scene(const bf_scene_desc* d, bf_hip_scene* s, bool upload) {
     S.tlas_root_ref = tlas_ref[s->tlas_root];
     S.instance_count = d->instance_count;
     S.exact_walk = exact_walk ? 1u : 0u;
+    S.material_buckets = base + o_buck;
     const bf_bvh_node& tr = s->tlas_nodes[s->tlas_root];
     const float trb[6] = {tr.min_x, tr.min_y, tr.min_z, tr.max_x, tr.max_y, tr.max_z};
     std::memcpy(S.tlas_root_box, trb, sizeof trb);
@@ -1124,7 +1146,8 @@ struct bf_hip_workspace {
     uint2* spill = nullptr;                  /* traversal stack spill, BF_STACK_DEPTH x spill_lanes */
     uint32_t spill_lanes = 0;
     uint32_t trace_lanes[3] = {0, 0, 0};
-    uint32_t shade_blocks = 0, adjoint_shade_blocks = 0;
+    uint32_t shade_blocks[BF_SHADE_MODES * BF_SHADE_KERNELS] = {};
+    uint32_t* bucket_ranges = nullptr;
     int device = 0;
     /* a captured group of bounces, replayed while paths remain (keyed by what its arguments hold) */
     hipGraphExec_t graph = nullptr;
@@ -1577,9 +1600,7 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     const uint32_t tiles = bfk_compact_tiles((uint32_t)n);
     hipError_t de = hipGetDevice(&w->device);
     const bool resident = de == hipSuccess && bfk_trace_resident_lanes(w->device, w->trace_lanes);
-    w->shade_blocks = de == hipSuccess ? bfk_shade_resident_blocks(w->device, false) : 0u;
-    w->adjoint_shade_blocks = de == hipSuccess ? bfk_shade_resident_blocks(w->device, true) : 0u;
-    if (!resident || w->shade_blocks == 0 || w->adjoint_shade_blocks == 0) {
+    if (!resident || !bfk_shade_resident_blocks(w->device, w->shade_blocks)) {
         delete w;
         return set_error(BF_DEVICE_ERROR, "cannot query the kernels' occupancy on the current device");
     }
@@ -1596,7 +1617,8 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     const size_t o_bc = A.add(nullptr, (size_t)tiles * 32), o_bo = A.add(nullptr, (size_t)tiles * 32);
     const size_t o_route = A.add(nullptr, n), o_tc = A.add(nullptr, (size_t)tiles * 8), o_to = A.add(nullptr, (size_t)tiles * 8),
                  o_sizes = A.add(nullptr, 64), o_hist = A.add(nullptr, BF_HISTORY_BOUNCES * 16), o_fail = A.add(nullptr, 16),
-                 o_samp = A.add(nullptr, 16), o_trav = A.add(nullptr, 64), o_fetch = A.add(nullptr, 2 * BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE * 4), o_hash = A.add(nullptr, BF_REPORT_MAX_BOUNCES * 16),
+                 o_samp = A.add(nullptr, 16), o_trav = A.add(nullptr, 64), o_fetch = A.add(nullptr, 2 * BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE * 4),
+                 o_ranges = A.add(nullptr, (BF_SHADE_BUCKETS + 1u) * 4), o_hash = A.add(nullptr, BF_REPORT_MAX_BOUNCES * 16),
                  o_jobs = A.add(nullptr, BF_MAX_BATCH_JOBS * sizeof(bf_dev_job)),
                  o_replicas = A.add(nullptr, (size_t)BF_GRADIENT_REPLICAS * BF_GRADIENT_ROW * sizeof(float)),
                  o_spill = A.add(nullptr, (size_t)w->spill_lanes * BF_STACK_DEPTH * sizeof(uint2));
@@ -1646,6 +1668,7 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     w->sample_counts = (uint32_t*)(b + o_samp);
     w->traversal = (unsigned long long*)(b + o_trav);
     w->fetch = (uint32_t*)(b + o_fetch);
+    w->bucket_ranges = (uint32_t*)(b + o_ranges);
     w->hashes = (unsigned long long*)(b + o_hash);
     w->jobs = (bf_dev_job*)(b + o_jobs);
     w->replicas = (float*)(b + o_replicas);
@@ -1699,6 +1722,13 @@ int validate_options(const bf_transport_options* o) {
     return BF_OK;
 }
 
+/* Kernels of one shade stage: its shade kernels, and three for an order. */
+uint64_t shade_dispatches(const bf_transport_params& P) {
+    bool ordered = false;
+    const uint32_t kernels = bfk_shade_plan(&P, &ordered);
+    return (uint64_t)__builtin_popcount(kernels) + (ordered ? 3u : 0u);
+}
+
 /* Issues one bounce of the loop on `stream` (no host synchronisation). The adjoint replay stops
  * after the shade stage: its light samples are resolved from the tape, so no shadow ray exists. */
 int issue_bounce(bf_hip_workspace* w, bf_transport_report& rep, const bf_transport_params& P, bool batch, bool instrument,
@@ -1711,7 +1741,7 @@ int issue_bounce(bf_hip_workspace* w, bf_transport_report& rep, const bf_transpo
     STAGE(BF_STAGE_COMPACTION, 3,
           bfk_compact(w->route, &w->sizes[0], n_max, ray_q, w->tile_counts, w->tile_offsets, w->queues[1], &w->sizes[1], 0u,
                       w->queues[2], &w->sizes[4], 0u, stream));
-    STAGE(BF_STAGE_SHADE, P.shade_order ? 4 : 1,
+    STAGE(BF_STAGE_SHADE, shade_dispatches(P),
           bfk_shade(&P, w->queues[1], &w->sizes[1], n_max, w->route, w->sample_counts, batch, P.shade_mode, stream));
     STAGE(BF_STAGE_COMPACTION, 3,
           bfk_compact(w->route, &w->sizes[1], n_max, w->queues[1], w->tile_counts, w->tile_offsets, w->queues[2],
@@ -1864,7 +1894,6 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
     P.bucket_offsets = w->bucket_offsets;
     /* orders live in queues that are free while the stage runs: the shadow queue is built after
      * shade (and is empty during closest hit); the hit queue is consumed before the shadow stage */
-    if (o->launch & BF_LAUNCH_SHADE_ORDER) P.shade_order = w->queues[2];
     if (o->launch & BF_LAUNCH_TRACE_ORDER) {
         P.closest_order = w->queues[2];
         P.shadow_order = w->queues[1];
@@ -1874,8 +1903,11 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
     P.step_counters = w->traversal;
     for (uint32_t j = 0; j < job_count; ++j)
         if (jobs[j].scene->dev.exact_walk || !(inputs || jobs[j].frame.camera.t_min >= 0.0f)) P.exact_walk = 1u;
-    P.shade_blocks = w->shade_blocks;
-    P.adjoint_shade_blocks = w->adjoint_shade_blocks;
+    std::copy(std::begin(w->shade_blocks), std::end(w->shade_blocks), P.shade_blocks);
+    P.bucket_ranges = w->bucket_ranges;
+    P.shade_order = w->queues[2];
+    P.shade_grouped = (o->launch & BF_LAUNCH_SHADE_ORDER) != 0u ? 1u : 0u;
+    for (uint32_t j = 0; j < job_count; ++j) P.shade_buckets |= jobs[j].scene->shade_buckets;
     const uint32_t block_log2 = (o->launch & BF_LAUNCH_TRACE_BLOCK_MASK) >> 16;
     P.trace_block = block_log2 == 0 ? 128u : 1u << block_log2;
     P.jobs = w->jobs;
@@ -2074,7 +2106,7 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
                 }
                 HIP_TRY(hipGraphLaunch(w->graph, stream));
                 rep.stage_metrics[BF_STAGE_CLOSEST_HIT].kernel_dispatches += group;
-                rep.stage_metrics[BF_STAGE_SHADE].kernel_dispatches += group;
+                rep.stage_metrics[BF_STAGE_SHADE].kernel_dispatches += group * shade_dispatches(P);
                 if (!adjoint) rep.stage_metrics[BF_STAGE_SHADOW].kernel_dispatches += group;
                 rep.stage_metrics[BF_STAGE_COMPACTION].kernel_dispatches += (adjoint ? 6u : 9u) * group;
                 rep.stage_metrics[BF_STAGE_AUXILIARY].kernel_dispatches += group;

@@ -96,8 +96,10 @@ typedef struct bf_transport_params {
     uint32_t trace_lanes[3];    /* resident lanes of closest-hit, shadow and counting traversal launches */
     uint32_t exact_walk;        /* traversal launches take the step-exact walk (see bf_traversal.h) */
     unsigned long long* step_counters; /* where such a launch counts when the caller asked for no counters */
-    uint32_t shade_blocks;      /* resident forward shade workgroups (persistent grid) */
-    uint32_t adjoint_shade_blocks; /* resident adjoint shade workgroups */
+    uint32_t shade_blocks[BF_SHADE_MODES * BF_SHADE_KERNELS]; /* resident workgroups of each shade kernel
+                                                               * (persistent grids), by mode and kernel */
+    uint32_t shade_buckets;     /* bit b: some instance's material is in shade bucket b */
+    uint32_t shade_grouped;     /* group the hit queue by bucket even where one kernel shades it all */
     uint32_t* fetch;            /* traversal work counters of closest-hit, then shadow launches, cleared
                                  * before each: BF_CLAIM_SEGMENTS each, BF_CLAIM_STRIDE words apart */
     uint32_t trace_block;       /* lanes per traversal workgroup: 64, 128 or 256 */
@@ -105,11 +107,12 @@ typedef struct bf_transport_params {
     float film_normalization;
     uint32_t shade_mode;        /* BF_SHADE_* of this launch (host bookkeeping: part of the graph-cache key) */
     float* gradient_replicas;   /* BF_GRADIENT_REPLICAS rows of BF_GRADIENT_ROW floats */
-    uint32_t* shade_order;      /* non-null: shade visits the hit queue grouped by closure kind (a free queue) */
+    uint32_t* shade_order;      /* where the grouped order of the hit queue goes (a free queue) */
     uint32_t* closest_order;    /* non-null: traversal claims rays grouped by direction octant (free queues) */
     uint32_t* shadow_order;
     uint32_t* bucket_counts;    /* per-tile bucket counts / offsets of these groupings */
     uint32_t* bucket_offsets;
+    uint32_t* bucket_ranges;    /* items of bucket b: [ranges[b], ranges[b + 1]) of the order */
 } bf_transport_params;
 
 #ifdef __cplusplus
@@ -149,8 +152,21 @@ hipError_t bfk_bounce_end(uint32_t* sizes, uint32_t* history, uint32_t history_b
 hipError_t bfk_film(const bf_dev_paths* paths, const bf_dev_job* job, float pdf, float normalization, hipStream_t s);
 /* Lanes the device holds at once for closest-hit, shadow and counting traversal; false on error. */
 bool bfk_trace_resident_lanes(int device, uint32_t* lanes);
-/* Workgroups the device holds at once for the shade kernels, 0 on error. */
-uint32_t bfk_shade_resident_blocks(int device, bool adjoint);
+/* The kernels of one shade stage (bit k: BF_SHADE_* k), and whether they take an order of the queue. */
+uint32_t bfk_shade_plan(const bf_transport_params* P, bool* ordered);
+/* Workgroups the device holds at once of each shade kernel, by mode and kernel; false on error. */
+bool bfk_shade_resident_blocks(int device, uint32_t* blocks);
+/* One mode's share of the above, and the launch of one of its kernels over `count_ptr` items, or the
+ * range of the order that is the kernel's when `order` is given (bf_shade.hip, built once per mode). */
+#define BFK_SHADE_MODE_DECLARE(name)                                                                                  \
+    bool bfk_shade_blocks_##name(int device, uint32_t* blocks);                                                       \
+    void bfk_shade_##name(const bf_transport_params* P, uint32_t kernel, const uint32_t* queue,                       \
+                          const uint32_t* count_ptr, uint32_t max_count, const uint32_t* order, uint8_t* route,       \
+                          uint32_t* sample_counts, bool batch, hipStream_t s);
+BFK_SHADE_MODE_DECLARE(plain)
+BFK_SHADE_MODE_DECLARE(textured)
+BFK_SHADE_MODE_DECLARE(adjoint)
+BFK_SHADE_MODE_DECLARE(mapped)
 hipError_t bfk_queue_hash(const uint32_t* queue, const uint32_t* count_ptr, unsigned long long* out, hipStream_t s);
 hipError_t bfk_scene_closest_hit(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
                                  bf_closest_hit_result* results, uint32_t* counters, hipStream_t s);

@@ -344,20 +344,15 @@ __global__ __launch_bounds__(BF_BLOCK) void k_compact_scatter(const uint8_t* rou
 }
 
 /* ---- shade order: hit-queue items grouped by the closure kind of their material ---------------
- * Shading a wave of mixed closure kinds issues every kind's code under a partial mask. The shade
- * stage can instead visit the hit queue through a permutation that groups items by kind (stable
- * within a kind); each item still writes its route at its own queue position, so the compactions
- * that follow see the queue order unchanged. Buckets: 0 multi-closure, 1..4 the closure kind. */
-#define BF_SHADE_BUCKETS 8u
-
+ * Shading a wave of mixed closure kinds issues every kind's code under a partial mask, and a kernel
+ * that can shade every kind needs registers for the widest of them. The shade stage therefore
+ * visits the hit queue through a permutation that groups items by bucket (stable within one); each item still writes its route at its own queue position, so the
+ * compactions that follow see the queue order unchanged. */
 template <bool BATCH>
 BF_D uint32_t shade_bucket(const bf_transport_params& P, const uint32_t* queue, uint32_t i) {
     const uint32_t slot = queue[i];
     const bf_dev_scene& S = job_at<BATCH>(P, slot).scene;
-    const bf_material_desc& M = S.materials[S.instances[P.paths.hit_ids[slot].x].material_index];
-    if (M.closure_count != 1u) return 0u;
-    const uint32_t kind = S.closures[M.closure_offset].kind;
-    return kind < BF_SHADE_BUCKETS ? kind : 0u;
+    return S.material_buckets[S.instances[P.paths.hit_ids[slot].x].material_index];
 }
 
 /* Traversal order: rays grouped by direction octant, so that a wave's rays tend to take the same
@@ -399,7 +394,7 @@ __global__ __launch_bounds__(BF_BLOCK) void k_bucket_count(bf_transport_params P
 
 /* single workgroup: tile offsets = bucket base (items of lower buckets) + earlier tiles' counts */
 __global__ __launch_bounds__(1024) void k_bucket_scan(const uint32_t* count_ptr, const uint32_t* tile_counts,
-                                                      uint32_t* tile_offsets) {
+                                                      uint32_t* tile_offsets, uint32_t* ranges) {
     __shared__ uint32_t partial[BF_SHADE_BUCKETS][1024];
     __shared__ uint32_t base[BF_SHADE_BUCKETS];
     const uint32_t t = threadIdx.x;
@@ -429,8 +424,10 @@ __global__ __launch_bounds__(1024) void k_bucket_scan(const uint32_t* count_ptr,
         uint32_t run = 0;
         for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) {
             base[b] = run;
+            ranges[b] = run;
             run += partial[b][1023];
         }
+        ranges[BF_SHADE_BUCKETS] = run;
     }
     __syncthreads();
     uint32_t run[BF_SHADE_BUCKETS];
@@ -1261,7 +1258,7 @@ static void launch_work_order(const bf_transport_params* P, const uint32_t* queu
     const uint32_t tiles = bfk_compact_tiles(max_count);
     const dim3 grid(tiles < 4096u ? tiles : 4096u);
     hipLaunchKernelGGL((k_bucket_count<BATCH, KEY>), grid, dim3(BF_BLOCK), 0, s, *P, queue, count_ptr, keys, tile_counts);
-    hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, s, count_ptr, tile_counts, tile_offsets);
+    hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, s, count_ptr, tile_counts, tile_offsets, P->bucket_ranges);
     hipLaunchKernelGGL(k_bucket_scatter, grid, dim3(BF_BLOCK), 0, s, keys, count_ptr, tile_offsets, order);
 }
 
@@ -1274,6 +1271,45 @@ void bfk_work_order(const bf_transport_params* P, uint32_t key, const uint32_t* 
     if (key == BF_KEY_SHADE) launch(batch ? launch_work_order<true, BF_KEY_SHADE> : launch_work_order<false, BF_KEY_SHADE>);
     else if (key == BF_KEY_RAY) launch(batch ? launch_work_order<true, BF_KEY_RAY> : launch_work_order<false, BF_KEY_RAY>);
     else launch(batch ? launch_work_order<true, BF_KEY_SHADOW> : launch_work_order<false, BF_KEY_SHADOW>);
+}
+
+bool bfk_shade_resident_blocks(int device, uint32_t* blocks) {
+    return bfk_shade_blocks_plain(device, blocks + BF_SHADE_PLAIN * BF_SHADE_KERNELS) &&
+           bfk_shade_blocks_textured(device, blocks + BF_SHADE_TEXTURED * BF_SHADE_KERNELS) &&
+           bfk_shade_blocks_adjoint(device, blocks + BF_SHADE_ADJOINT * BF_SHADE_KERNELS) &&
+           bfk_shade_blocks_mapped(device, blocks + BF_SHADE_MAPPED * BF_SHADE_KERNELS);
+}
+
+/* The kernels that the frames' materials need, in one order of the hit queue when it holds more than
+ * one kind of item. */
+uint32_t bfk_shade_plan(const bf_transport_params* P, bool* ordered) {
+    const uint32_t mask = P->shade_buckets;
+    const uint32_t single = mask >> BF_BUCKET_LAMBERT;
+    uint32_t kernels = (mask & 0xFu) != 0u ? 1u << BF_SHADE_ANY : 0u;
+    if (single != 0u) kernels |= single == 1u ? 1u << BF_SHADE_LAMBERT : 1u << BF_SHADE_SINGLE;
+    const bool one_kind = (single & (single - 1u)) == 0u && ((mask & 0xFu) == 0u || single == 0u);
+    *ordered = !one_kind || (P->shade_grouped != 0u && (mask & (mask - 1u)) != 0u);
+    return kernels;
+}
+
+hipError_t bfk_shade(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr, uint32_t max_count,
+                     uint8_t* route, uint32_t* sample_counts, bool batch, uint32_t mode, hipStream_t s) {
+    if (max_count == 0) return hipSuccess;
+    bool ordered = false;
+    const uint32_t kernels = bfk_shade_plan(P, &ordered);
+    const uint32_t* order = nullptr;
+    if (ordered) {
+        /* the route bytes of the hit queue are free until shade writes them: they hold the keys */
+        bfk_work_order(P, BF_KEY_SHADE, queue, count_ptr, max_count, route, P->shade_order, batch, s);
+        order = P->shade_order;
+    }
+    const auto launch = mode == BF_SHADE_ADJOINT    ? bfk_shade_adjoint
+                        : mode == BF_SHADE_TEXTURED ? bfk_shade_textured
+                        : mode == BF_SHADE_MAPPED   ? bfk_shade_mapped
+                                                    : bfk_shade_plain;
+    for (uint32_t k = 0; k < BF_SHADE_KERNELS; ++k)
+        if (kernels >> k & 1u) launch(P, k, queue, count_ptr, max_count, order, route, sample_counts, batch, s);
+    return hipGetLastError();
 }
 
 int bfk_max_resident(const void* const* kernels, int count, uint32_t block, int device) {

@@ -74,6 +74,37 @@ BF_D float spectrum_at(const bf_dev_scene& S, uint32_t id, float wavelength) {
     return fmaf(v[i + 1] - v[i], f, v[i]);
 }
 
+/* spectrum_at of the four wavelengths of a path: the descriptor is read and the grid step formed once. */
+BF_D void spectrum_lanes(const bf_dev_scene& S, uint32_t id, const float* wl, float* out) {
+    out[0] = out[1] = out[2] = out[3] = 0.0f;
+    if (id == BF_INVALID_INDEX) return;
+    const bf_spectrum_desc sp = S.spectra[id];
+    const float* v = S.spectrum_values + sp.offset;
+    if (sp.count & BF_SPECTRUM_SAMPLED) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            out[k] = __builtin_nanf("");
+#pragma unroll
+            for (int lane = 3; lane >= 0; --lane)
+                if (v[lane] == wl[k]) out[k] = v[4 + lane];
+        }
+        return;
+    }
+    if (sp.count <= 1u) {
+        out[0] = out[1] = out[2] = out[3] = v[0];
+        return;
+    }
+    const float step = 470.0f / (float)(sp.count - 1u);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float t = (wl[k] - 360.0f) / step;
+        uint32_t i = t <= 0.0f ? 0u : (uint32_t)t;
+        if (i > sp.count - 2u) i = sp.count - 2u;
+        const float f = t - (float)i;
+        out[k] = fmaf(v[i + 1] - v[i], f, v[i]);
+    }
+}
+
 BF_D bool valid_cone(float w, float s) { return bf_isfinite(w) && w >= 0.0f && bf_isfinite(s) && s >= 0.0f; }
 
 /* ---- ray cones (CudaWavefrontStages.cu:2816-2867, 3675-3782) ---------------------------------- */

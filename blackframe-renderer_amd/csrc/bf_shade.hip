@@ -1,6 +1,7 @@
 /*
  * The shade stage of a bounce: surface reconstruction, emission, light and closure sampling, Russian
- * roulette, and the texel gradients of the adjoint replay.
+ * roulette, and the texel gradients of the adjoint replay. Built once per mode (BF_SHADE_MODE, with
+ * BF_SHADE_NAME naming its launchers).
  */
 #include <hip/hip_runtime.h>
 
@@ -100,23 +101,29 @@ BF_D bool texture_value(const bf_dev_scene& S, uint32_t slot, const float* uv, f
 
 /* Closure records at the path's wavelengths; textured weights and GGX widths are looked up at the
  * hit's texture coordinates. False when a texture lookup is not representable. */
-template <bool TEX>
-BF_D bool load_mixture(const bf_dev_scene& S, const bf_material_desc& M, const float* wl, const float* uv, mixture_t& mix) {
-    mix.active_count = M.closure_count;
-    for (uint32_t c = 0; c < M.closure_count; ++c) {
+/* The closure kind of a class's materials. */
+template <uint32_t CLASS>
+BF_D uint32_t class_kind(uint32_t kind) {
+    return CLASS == BF_SHADE_LAMBERT      ? (uint32_t)BF_CLOSURE_LAMBERTIAN
+           : CLASS == BF_SHADE_CONDUCTOR  ? (uint32_t)BF_CLOSURE_ROUGH_CONDUCTOR
+           : CLASS == BF_SHADE_DIELECTRIC ? (uint32_t)BF_CLOSURE_ROUGH_DIELECTRIC
+                                          : kind;
+}
+
+template <bool TEX, uint32_t CLASS, uint32_t N>
+BF_D bool load_mixture(const bf_dev_scene& S, const bf_material_desc& M, const float* wl, const float* uv, mixture_t<N>& mix) {
+    mix.active_count = N == 1u ? 1u : M.closure_count;
+    for (uint32_t c = 0; c < N && c < mix.active_count; ++c) {
         const bf_closure_desc D = S.closures[M.closure_offset + c];
         closure_t& r = mix.closures[c];
-        r.kind = D.kind;
+        r.kind = class_kind<CLASS>(D.kind);
         r.lobes = D.lobes;
 #pragma unroll
         for (int k = 0; k < 10; ++k) r.parameters[k] = D.parameters[k];
-#pragma unroll
-        for (int lane = 0; lane < 4; ++lane) {
-            r.weight[lane] = spectrum_at(S, D.weight_spectrum, wl[lane]);
-            if (D.kind == BF_CLOSURE_ROUGH_CONDUCTOR) {
-                r.parameters[lane] = spectrum_at(S, D.eta_spectrum, wl[lane]);
-                r.parameters[4 + lane] = spectrum_at(S, D.k_spectrum, wl[lane]);
-            }
+        spectrum_lanes(S, D.weight_spectrum, wl, r.weight);
+        if (r.kind == BF_CLOSURE_ROUGH_CONDUCTOR) {
+            spectrum_lanes(S, D.eta_spectrum, wl, r.parameters);
+            spectrum_lanes(S, D.k_spectrum, wl, r.parameters + 4);
         }
         if (TEX && D.weight_texture) {
             float t[3];
@@ -131,14 +138,14 @@ BF_D bool load_mixture(const bf_dev_scene& S, const bf_material_desc& M, const f
             bf_texel_footprint f;
             if (!texture_value(S, D.roughness_texture - 1u, uv, t, f)) return false;
             const float ay = S.textures[D.roughness_texture - 1u].channels == 2u ? t[1] : t[0];
-            const int at = D.kind == BF_CLOSURE_ROUGH_CONDUCTOR ? 8 : 2;
+            const int at = r.kind == BF_CLOSURE_ROUGH_CONDUCTOR ? 8 : 2;
             r.parameters[at] = t[0];
             r.parameters[at + 1] = ay;
         }
-        mix.probabilities[c] = M.probabilities[c];
+        mix.probabilities[c] = N == 1u ? 1.0f : M.probabilities[c];
     }
 #pragma unroll
-    for (uint32_t c = 0; c <= BF_MAX_CLOSURES; ++c) mix.cdf[c] = M.cdf[c];
+    for (uint32_t c = 0; c <= N; ++c) mix.cdf[c] = N == 1u ? (float)c : M.cdf[c];
     return true;
 }
 
@@ -161,9 +168,9 @@ BF_D bool sample_punctual(const bf_dev_scene& S, uint32_t index, const float* wl
     const bf_dev_punctual L = S.punctuals[index];
     float spectrum[4];
     bool black = true;
+    spectrum_lanes(S, L.spectrum, wl, spectrum);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        spectrum[c] = spectrum_at(S, L.spectrum, wl[c]);
         if (!bf_isfinite(spectrum[c]) || spectrum[c] < 0.0f) return false;
         if (spectrum[c] != 0.0f) black = false;
     }
@@ -250,7 +257,7 @@ BF_D bool contract_point_endpoint(v3f p, v3f err, v3f to_light, v3f& out) {
 /* sample_registered_light (:2378-2460) + sample_mesh_area_light (:2044-2201); the per-light area
  * CDF of :2085-2147 is a scene constant evaluated by the host, searched here in O(log n). */
 BF_D bool sample_light(const bf_transport_params& P, const bf_dev_scene& S, const sample_key& k, uint64_t first_dim,
-                       const float* wl, uint32_t visibility, const surface_t& surf, incident_t& inc) {
+                       float area_sample, float triangle_sample, const float* wl, uint32_t visibility, const surface_t& surf, incident_t& inc) {
     inc.present = false;
     uint32_t li;
     float sel;
@@ -264,8 +271,6 @@ BF_D bool sample_light(const bf_transport_params& P, const bf_dev_scene& S, cons
     const bf_dev_light L = S.lights[li - S.punctual_count];
     const bf_dev_instance& I = S.instances[L.instance];
     if ((I.visibility_mask & visibility) == 0u) return true;
-    const float area_sample = sample_1d(P.sampler, k, first_dim + 1);
-    const float triangle_sample = sample_1d(P.sampler, k, first_dim + 2);
     if (!(area_sample >= 0.0f) || !(area_sample < 1.0f) || !(triangle_sample >= 0.0f) || !(triangle_sample < 1.0f))
         return false;
     /* first triangle whose cumulative bound exceeds the sample (bounds strictly increase) */
@@ -299,9 +304,9 @@ BF_D bool sample_light(const bf_transport_params& P, const bf_dev_scene& S, cons
     const bf_material_desc& M = S.materials[I.material_index];
     float radiance[4];
     bool black = true;
+    spectrum_lanes(S, M.emission_spectrum, wl, radiance);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        radiance[c] = spectrum_at(S, M.emission_spectrum, wl[c]);
         if (!bf_isfinite(radiance[c]) || radiance[c] < 0.0f) return false;
         if (radiance[c] != 0.0f) black = false;
     }
@@ -412,13 +417,14 @@ BF_D void texel_add(const bf_transport_params& P, const bf_dev_job& J, texel_pen
     for (uint32_t ch = 0; ch < channels; ++ch) p.sc[ch] += sc[ch];
 }
 
-BF_D void texel_gradients(const bf_transport_params& P, const bf_dev_job& J, const bf_dev_scene& S, const bf_material_desc& M, const mixture_t& mix,
-                          const filter_t& filtered, const float* uv, const float* wl, const float* a, bool light, v3f wo,
+template <uint32_t N_>
+BF_D void texel_gradients(const bf_transport_params& P, const bf_dev_job& J, const bf_dev_scene& S, const bf_material_desc& M,
+                          const mixture_t<N_>& mix, const filter_t<N_>& filtered, const float* uv, const float* wl, const float* a, bool light, v3f wo,
                           v3f wi_light, const float* f_light, const float* N, bool cont, bool cont_discrete, v3f wi_cont,
                           const float* f_cont, const float* R) {
     texel_pending weights{BF_INVALID_INDEX, 0u, {}, {0.0f, 0.0f, 0.0f}};
     texel_pending widths{BF_INVALID_INDEX, 0u, {}, {0.0f, 0.0f, 0.0f}};
-    for (uint32_t i = 0; i < mix.active_count; ++i) {
+    for (uint32_t i = 0; i < N_ && i < mix.active_count; ++i) {
         const bf_closure_desc D = S.closures[M.closure_offset + filtered.source_indices[i]];
         const bool wgrad = D.weight_texture && J.texture_gradients[D.weight_texture - 1u];
         const bool rgrad = D.roughness_texture && J.texture_gradients[D.roughness_texture - 1u];
@@ -499,10 +505,11 @@ BF_D void texel_gradients(const bf_transport_params& P, const bf_dev_job& J, con
  * normal / bump maps), or BF_SHADE_ADJOINT: the
  * adjoint replay resolves the light sample from the tape, never routes to the shadow queue and
  * accumulates texel gradients. */
-template <bool BATCH, uint32_t MODE>
-BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32_t i, uint8_t* route,
+template <bool BATCH, uint32_t MODE, uint32_t CLASS>
+BF_D uint32_t shade_item(const bf_transport_params& P, const uint32_t* queue, uint32_t i, uint8_t* route,
                      uint32_t* sample_counts) {
     constexpr bool ADJ = MODE == BF_SHADE_ADJOINT;
+    constexpr uint32_t N = CLASS == BF_SHADE_ANY ? BF_MAX_CLOSURES : 1u;
     const uint32_t slot = queue[i];
     route[i] = 0;
     const bf_dev_job& J = job_at<BATCH>(P, slot);
@@ -529,86 +536,92 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
     const uint32_t visibility = P.paths.visibility[slot];
 
     surface_t surf;
-    if (!surface_data(S, ids.x, ids.y, hit, ro, rd, surf)) return fail_path(P, J, slot, 10);
+    if (!surface_data(S, ids.x, ids.y, hit, ro, rd, surf)) return 10u;
     if (MODE == BF_SHADE_MAPPED && S.maps &&
         (S.maps[surf.material].normal_texture != BF_INVALID_INDEX || S.maps[surf.material].bump_texture != BF_INVALID_INDEX)) {
         /* the shade stage's surface maps (:4170-4193): the cone advanced to the hit sets the
          * footprint; 46 the cone, 47-49 the maps (invalid, numerical, texel budget) */
         float2 at_hit;
         if (!(J.in_cones || J.frame_cones) || !advance_cone(P.paths.cone[slot], rd, hit.x, at_hit))
-            return fail_path(P, J, slot, 46);
+            return 46u;
         const int st = apply_surface_maps(S, surf.material, at_hit, rd, surf.uv[0], surf.uv[1], surf.ng, surf.dpdu,
                                           surf.dpdv, surf.ns);
-        if (st != BF_MAP_OK) return fail_path(P, J, slot, 46u + (uint32_t)st);
+        if (st != BF_MAP_OK) return 46u + (uint32_t)st;
     }
     v3f wo;
-    if (!normalize3(mk(-rd.x, -rd.y, -rd.z), wo)) return fail_path(P, J, slot, 11);
+    if (!normalize3(mk(-rd.x, -rd.y, -rd.z), wo)) return 11u;
     bool front = false;
-    if (!one_sided_emission_support(surf.ng, wo, front)) return fail_path(P, J, slot, 12);
+    if (!one_sided_emission_support(surf.ng, wo, front)) return 12u;
     const bf_material_desc& M = S.materials[surf.material];
     float emitted[4];
+    spectrum_lanes(S, M.emission_spectrum, wl, emitted);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        emitted[c] = spectrum_at(S, M.emission_spectrum, wl[c]);
-        if (!bf_isfinite(emitted[c]) || emitted[c] < 0.0f) return fail_path(P, J, slot, 13);
+        if (!bf_isfinite(emitted[c]) || emitted[c] < 0.0f) return 13u;
     }
-    mixture_t mix;
-    if (!load_mixture<MODE != BF_SHADE_PLAIN>(S, M, wl, surf.uv, mix)) return fail_path(P, J, slot, 42);
+    mixture_t<N> mix;
+    if (!load_mixture<MODE != BF_SHADE_PLAIN, CLASS>(S, M, wl, surf.uv, mix)) return 42u;
     frame3 frame, unrotated;
     const bool created = M.frame_mode == 0u ? make_local_frame(surf.ns, unrotated) : frame_from_tangent(surf.ns, surf.dpdu, unrotated);
-    if (!created || !rotate_frame(unrotated, M.tangent_rotation, frame)) return fail_path(P, J, slot, 14);
+    if (!created || !rotate_frame(unrotated, M.tangent_rotation, frame)) return 14u;
     if (front && !zero4(emitted)) {
         float weight;
-        if (!emission_weight(P, S, ids.x, prev, surf, weight)) return fail_path(P, J, slot, 15);
+        if (!emission_weight(P, S, ids.x, prev, surf, weight)) return 15u;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if (beta[c] == 0.0f || emitted[c] == 0.0f || weight == 0.0f) continue;
             const float num[3] = {beta[c], emitted[c], weight};
             const float den[1] = {1.0f};
             float contribution;
-            if (checked_product_quotient(num, den, contribution) != BF_L_OK) return fail_path(P, J, slot, 16);
+            if (checked_product_quotient(num, den, contribution) != BF_L_OK) return 16u;
             L[c] += contribution;
-            if (!bf_isfinite(L[c])) return fail_path(P, J, slot, 16);
+            if (!bf_isfinite(L[c])) return 16u;
         }
         P.paths.radiance[slot] = make_float4(L[0], L[1], L[2], L[3]);
     }
     if (zero4(beta)) {
         P.paths.status[slot] = BF_TERM_ZERO_THROUGHPUT;
-        return;
+        return 0u;
     }
     const uint32_t limits[5] = {P.limits[0], P.limits[1], P.limits[2], P.limits[3], P.limits[4]};
     const uint32_t counters[5] = {diffuse, glossy, specular, transmission, 0u};
     if (diffuse > limits[0] || glossy > limits[1] || specular > limits[2] || transmission > limits[3])
-        return fail_path(P, J, slot, 17);
-    filter_t filtered;
+        return 17u;
+    filter_t<N> filtered;
     filter_by_depth(mix, limits, counters, depth, filtered);
-    if (filtered.status != BF_L_OK) return fail_path(P, J, slot, 18);
+    if (filtered.status != BF_L_OK) return 18u;
     if (mix.active_count == 0 && filtered.source_count != 0) {
         /* the depth categories that blocked the path ride above the termination byte */
         P.paths.status[slot] = BF_TERM_DEPTH_LIMIT | (filtered.blocked << 8);
-        return;
+        return 0u;
     }
+    if (N == 1u) mix.active_count = 1u;
     const v3f wo_local = to_local(frame, wo);
     const uint64_t first_dim = 4ull + (uint64_t)depth * 10ull;
-    const float bsdf_component = sample_1d(P.sampler, key, first_dim + 3);
-    const float bsdf_u = sample_1d(P.sampler, key, first_dim + 4);
-    const float bsdf_v = sample_1d(P.sampler, key, first_dim + 5);
+    /* light area and triangle, closure u and v, closure selection: one Lambert or conductor closure has
+     * nothing to select (where that dimension has no sample the next one has none either, and that
+     * fails the path the same way) */
+    constexpr bool SELECTS = CLASS != BF_SHADE_LAMBERT && CLASS != BF_SHADE_CONDUCTOR;
+    const uint64_t dims[5] = {first_dim + 1, first_dim + 2, first_dim + 4, first_dim + 5, first_dim + 3};
+    float samples[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    sample_each<SELECTS ? 5 : 4>(P.sampler, key, dims, samples);
+    const float bsdf_u = samples[2], bsdf_v = samples[3], bsdf_component = samples[4];
     wave_count(&sample_counts[0]);
     mixture_sample_t bs;
     sample_mixture(mix, filtered, wo_local, bsdf_component, bsdf_u, bsdf_v, bs);
     const bool has_continuation = bs.status == BF_L_OK;
-    if (!has_continuation && bs.status != BF_L_OUTSIDE) return fail_path(P, J, slot, 19);
+    if (!has_continuation && bs.status != BF_L_OUTSIDE) return 19u;
     if (has_continuation) {
         const bool delta = valid_surface_event(bs.lobes) && (bs.lobes & BF_LOBE_SPECULAR);
         if (!valid_surface_event(bs.lobes) || (bs.discrete != 0u) != delta || !bf_isfinite(bs.pdf) || !(bs.pdf > 0.0f) ||
             (delta && bs.pdf > 1.0f))
-            return fail_path(P, J, slot, 20);
+            return 20u;
     }
     incident_t inc;
     inc.present = false;
     if (S.light_count != 0u && mixture_nonblack(mix)) {
         wave_count(&sample_counts[1]);
-        if (!sample_light(P, S, key, first_dim, wl, visibility, surf, inc)) return fail_path(P, J, slot, 21);
+        if (!sample_light(P, S, key, first_dim, samples[0], samples[1], wl, visibility, surf, inc)) return 21u;
     }
     bool has_shadow = false;
     float4 shadow_o = make_float4(0.0f, 0.0f, 0.0f, 0.0f), shadow_d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -625,19 +638,19 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
                 if (wo_local.z > 0.0f && wi_local.z > 0.0f)
                     for (int c = 0; c < 4; ++c) bsdf[c] = mix.closures[0].weight[c];
             } else if (mixture_eval(mix, filtered, wo_local, wi_local, bsdf) != BF_L_OK) {
-                return fail_path(P, J, slot, 22);
+                return 22u;
             }
             for (int c = 0; c < 4; ++c) nee_f[c] = singleton_lambert ? bsdf[c] * BF_INV_PI : bsdf[c];
             if (!zero4(bsdf)) {
                 float corr;
-                if (!shading_correction(surf.ng, surf.ns, wo, inc.direction, corr)) return fail_path(P, J, slot, 23);
+                if (!shading_correction(surf.ng, surf.ns, wo, inc.direction, corr)) return 23u;
                 if (corr > 0.0f) {
                     float w = 1.0f; /* punctual lights are discrete: no MIS (:4437-4470) */
                     if (inc.kind == BF_INCIDENT_SURFACE) {
                         float joint, bsdf_pdf;
-                        if (!joint_light_pdf(inc.selection, inc.conditional, joint)) return fail_path(P, J, slot, 24);
-                        if (mixture_pdf(mix, filtered, wo_local, wi_local, bsdf_pdf) != BF_L_OK) return fail_path(P, J, slot, 24);
-                        if (!mis_weight(P.mis, joint, bsdf_pdf, w)) return fail_path(P, J, slot, 24);
+                        if (!joint_light_pdf(inc.selection, inc.conditional, joint)) return 24u;
+                        if (mixture_pdf(mix, filtered, wo_local, wi_local, bsdf_pdf) != BF_L_OK) return 24u;
+                        if (!mis_weight(P.mis, joint, bsdf_pdf, w)) return 24u;
                     }
                     /* the visible-shadow contribution of process_shadow_kernel (:4772-4908),
                      * evaluated now from the same frozen factors */
@@ -653,11 +666,11 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
                             const float num[7] = {beta[c], bsdf[c], coefficient, inc.radiance[c], cosine, corr, w};
                             st = checked_product_quotient(num, den, contribution[c]);
                         }
-                        if (st != BF_L_OK) return fail_path(P, J, slot, 41);
+                        if (st != BF_L_OK) return 41u;
                     }
                     /* prepare_shadow_ray (:4042-4105) */
                     v3f src, endpoint;
-                    if (!offset_point(surf.position, surf.error, surf.ng, inc.direction, src)) return fail_path(P, J, slot, 25);
+                    if (!offset_point(surf.position, surf.error, surf.ng, inc.direction, src)) return 25u;
                     if (inc.kind == BF_INCIDENT_INFINITE) {
                         shadow_o = make_float4(src.x, src.y, src.z, BF_INFINITY_F);
                         shadow_d = make_float4(inc.direction.x, inc.direction.y, inc.direction.z, 0.0f);
@@ -667,9 +680,9 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
                                               ? contract_point_endpoint(inc.position, inc.error, inc.direction, endpoint)
                                               : offset_point(inc.position, inc.error, inc.normal, mul3(inc.direction, -1.0f), endpoint);
                         if (!ends || !scaled_segment(sub3(endpoint, src), seg) || !(dot3(seg.direction, inc.direction) > 0.0f))
-                            return fail_path(P, J, slot, 25);
+                            return 25u;
                         const float tmax = bf_next_toward_zero_f(seg.length);
-                        if (!(tmax > 0.0f)) return fail_path(P, J, slot, 25);
+                        if (!(tmax > 0.0f)) return 25u;
                         shadow_o = make_float4(src.x, src.y, src.z, tmax);
                         shadow_d = make_float4(seg.direction.x, seg.direction.y, seg.direction.z, 0.0f);
                     }
@@ -682,10 +695,10 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
     bool continuation = has_continuation;
     float corr = 0.0f;
     if (continuation) {
-        if (!to_world(frame, bs.incoming, wi)) return fail_path(P, J, slot, 26);
+        if (!to_world(frame, bs.incoming, wi)) return 26u;
         bool geo = false;
         if (!shading_correction(surf.ng, surf.ns, wo, wi, corr) || !geometric_event_support(surf.ng, wo, wi, bs.lobes, geo))
-            return fail_path(P, J, slot, 27);
+            return 27u;
         continuation = corr > 0.0f && geo;
     }
     uint32_t pending_term = BF_TERM_OUTSIDE_SUPPORT;
@@ -694,22 +707,22 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
         /* update_closure_throughput (:3894-3938) */
         float nb[4];
         const float cosine = fabsf(bs.incoming.z);
-        if (!bf_isfinite(cosine) || !(cosine > 0.0f)) return fail_path(P, J, slot, 28);
+        if (!bf_isfinite(cosine) || !(cosine > 0.0f)) return 28u;
         if (mix.active_count == 1 && mix.closures[0].kind == BF_CLOSURE_LAMBERTIAN && corr == 1.0f) {
             for (int c = 0; c < 4; ++c)
-                if (!checked_product(beta[c], mix.closures[0].weight[c], nb[c])) return fail_path(P, J, slot, 28);
+                if (!checked_product(beta[c], mix.closures[0].weight[c], nb[c])) return 28u;
         } else {
             for (int c = 0; c < 4; ++c) {
                 const float num[4] = {beta[c], bs.value[c], cosine, corr};
                 const float den[1] = {bs.pdf};
-                if (checked_product_quotient(num, den, nb[c]) != BF_L_OK) return fail_path(P, J, slot, 28);
+                if (checked_product_quotient(num, den, nb[c]) != BF_L_OK) return 28u;
             }
         }
         const float next_eta = eta_scale * bs.eta_scale;
         if (!bf_isfinite(bs.eta_scale) || !(bs.eta_scale > 0.0f) || !bf_isfinite(next_eta) || !(next_eta > 0.0f))
-            return fail_path(P, J, slot, 29);
+            return 29u;
         v3f origin;
-        if (!offset_point(surf.position, surf.error, surf.ng, wi, origin)) return fail_path(P, J, slot, 30);
+        if (!offset_point(surf.position, surf.error, surf.ng, wi, origin)) return 30u;
         const bool delta_event = (bs.lobes & BF_LOBE_SPECULAR) != 0u;
         delta_flags = ((delta_flags & 2u) ? 2u : 0u) | (delta_event ? 1u : 2u);
         /* advance_depth_event (:3851-3880) */
@@ -725,16 +738,16 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
         if (J.in_cones || J.frame_cones) {
             /* the sampled closure's compact index, then the cone advanced to the hit and scattered */
             uint32_t compact = mix.active_count, matches = 0u;
-            for (uint32_t k = 0; k < mix.active_count; ++k)
+            for (uint32_t k = 0; k < N && k < mix.active_count; ++k)
                 if (filtered.source_indices[k] == bs.selected) {
                     compact = k;
                     ++matches;
                 }
             float2 advanced, next;
-            if (matches != 1u || compact >= mix.active_count) return fail_path(P, J, slot, 43);
-            if (!advance_cone(P.paths.cone[slot], rd, hit.x, advanced)) return fail_path(P, J, slot, 44);
-            if (!propagate_cone(advanced, mix.closures[compact], bs.lobes, wo_local, bs.incoming, next))
-                return fail_path(P, J, slot, 45);
+            if (matches != 1u || compact >= mix.active_count) return 43u;
+            if (!advance_cone(P.paths.cone[slot], rd, hit.x, advanced)) return 44u;
+            if (!propagate_cone(advanced, mix.closures[N == 1u ? 0u : compact], bs.lobes, wo_local, bs.incoming, next))
+                return 45u;
             P.paths.cone[slot] = next;
         }
         P.paths.ray_origin[slot] = make_float4(origin.x, origin.y, origin.z, ro4.w);
@@ -751,12 +764,12 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
             bool survived = false;
             if (replay) {
                 p = *frozen;
-                if (!finite_nonnegative4(beta4) || !bf_isfinite(p) || !(p > 0.0f) || p > 1.0f) return fail_path(P, J, slot, 32);
+                if (!finite_nonnegative4(beta4) || !bf_isfinite(p) || !(p > 0.0f) || p > 1.0f) return 32u;
             } else if (!roulette_probability(beta4, eta_scale, P.rr_min, P.rr_max, p)) {
-                return fail_path(P, J, slot, 32);
+                return 32u;
             }
             if (!sample_below(P.sampler, key, first_dim + 9, p, survived) || (survived && !roulette_survive(beta4, p)))
-                return fail_path(P, J, slot, 32);
+                return 32u;
             if (frozen && !replay && !ADJ) *frozen = p;
             if (!survived) {
                 cont_pending = false;
@@ -776,7 +789,7 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
         if (visible) {
             for (int c = 0; c < 4; ++c) {
                 L[c] += contribution[c];
-                if (!bf_isfinite(L[c]) || L[c] < 0.0f) return fail_path(P, J, slot, 41);
+                if (!bf_isfinite(L[c]) || L[c] < 0.0f) return 41u;
             }
             P.paths.radiance[slot] = make_float4(L[0], L[1], L[2], L[3]);
         }
@@ -790,10 +803,10 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
         }
         if (!cont_pending) {
             P.paths.status[slot] = pending_term;
-            return;
+            return 0u;
         }
         route[i] = 2;
-        return;
+        return 0u;
     }
     if (has_shadow) {
         shadow_d.w = __uint_as_float((cont_pending ? 1u : 0u) | (pending_term << 8) | (vertex << 16));
@@ -801,74 +814,91 @@ BF_D void shade_item(const bf_transport_params& P, const uint32_t* queue, uint32
         P.paths.shadow_direction[slot] = shadow_d;
         P.paths.shadow_contribution[slot] = make_float4(contribution[0], contribution[1], contribution[2], contribution[3]);
         route[i] = 1;
-        return;
+        return 0u;
     }
     if (!cont_pending) {
         P.paths.status[slot] = pending_term;
-        return;
+        return 0u;
     }
     route[i] = 2;
+    return 0u;
 }
 
-template <bool BATCH, uint32_t MODE>
-__global__ __launch_bounds__(BF_SHADE_BLOCK, MODE == BF_SHADE_ADJOINT ? BF_ADJOINT_SHADE_WAVES_PER_SIMD : BF_SHADE_WAVES_PER_SIMD) void k_shade(bf_transport_params P, const uint32_t* queue,
-                                                                             const uint32_t* count_ptr, const uint32_t* order,
-                                                                             uint8_t* route, uint32_t* sample_counts) {
-    const uint32_t n = *count_ptr;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        shade_item<BATCH, MODE>(P, queue, order ? order[i] : i, route, sample_counts);
-}
-
-extern "C" {
-
-/* Resident workgroups of the forward shade variants, or of the adjoint ones (which hold fewer
- * waves per SIMD): the persistent shade grid of each, so that no workgroup waits for a slot. */
-uint32_t bfk_shade_resident_blocks(int device, bool adjoint) {
-    const void* forward[6] = {(const void*)k_shade<false, BF_SHADE_PLAIN>,    (const void*)k_shade<true, BF_SHADE_PLAIN>,
-                              (const void*)k_shade<false, BF_SHADE_TEXTURED>, (const void*)k_shade<true, BF_SHADE_TEXTURED>,
-                              (const void*)k_shade<false, BF_SHADE_MAPPED>,   (const void*)k_shade<true, BF_SHADE_MAPPED>};
-    const void* backward[2] = {(const void*)k_shade<false, BF_SHADE_ADJOINT>, (const void*)k_shade<true, BF_SHADE_ADJOINT>};
-    return adjoint ? (uint32_t)bfk_max_resident(backward, 2, BF_SHADE_BLOCK, device)
-                   : (uint32_t)bfk_max_resident(forward, 6, BF_SHADE_BLOCK, device);
-}
-
-} /* extern "C" */
-
-template <bool BATCH>
-static void launch_shade(const bf_transport_params* P, dim3 grid, const uint32_t* queue, const uint32_t* count_ptr,
-                         const uint32_t* order, uint8_t* route, uint32_t* sample_counts, uint32_t mode, hipStream_t s) {
-    const dim3 block(BF_SHADE_BLOCK);
-    if (mode == BF_SHADE_ADJOINT)
-        hipLaunchKernelGGL((k_shade<BATCH, BF_SHADE_ADJOINT>), grid, block, 0, s, *P, queue, count_ptr, order, route,
-                           sample_counts);
-    else if (mode == BF_SHADE_TEXTURED)
-        hipLaunchKernelGGL((k_shade<BATCH, BF_SHADE_TEXTURED>), grid, block, 0, s, *P, queue, count_ptr, order, route,
-                           sample_counts);
-    else if (mode == BF_SHADE_MAPPED)
-        hipLaunchKernelGGL((k_shade<BATCH, BF_SHADE_MAPPED>), grid, block, 0, s, *P, queue, count_ptr, order, route,
-                           sample_counts);
-    else
-        hipLaunchKernelGGL((k_shade<BATCH, BF_SHADE_PLAIN>), grid, block, 0, s, *P, queue, count_ptr, order, route,
-                           sample_counts);
-}
-
-extern "C" {
-
-hipError_t bfk_shade(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr, uint32_t max_count,
-                     uint8_t* route, uint32_t* sample_counts, bool batch, uint32_t mode, hipStream_t s) {
-    if (max_count == 0) return hipSuccess;
-    const uint32_t* order = nullptr;
-    if (P->shade_order) {
-        /* the route bytes of the hit queue are free until shade writes them: they hold the keys */
-        bfk_work_order(P, BF_KEY_SHADE, queue, count_ptr, max_count, route, P->shade_order, batch, s);
-        order = P->shade_order;
+/* One kernel's items: the whole queue, or its buckets' range of the order. An item of a single closure
+ * keeps it in registers and runs that kind's code alone; the general path indexes up to
+ * BF_MAX_CLOSURES of any kind in scratch (1.2 KB a lane). One kernel for every kind of single closure
+ * leaves no kernel waiting for the longest wave of the one before: 1.3 ms of shading in a 333x187x1
+ * frame, against 2.3 with a kernel per kind and 1.5 with the general kernel alone. The Lambertian
+ * kernel needs neither the order nor the other kinds' registers. */
+template <bool BATCH, uint32_t MODE, uint32_t KERNEL>
+__global__ __launch_bounds__(BF_SHADE_BLOCK, KERNEL == BF_SHADE_ANY ? BF_SHADE_WAVES_PER_SIMD : BF_SHADE_SINGLE_WAVES) void k_shade(
+    bf_transport_params P, const uint32_t* queue, const uint32_t* count_ptr, const uint32_t* order, uint8_t* route,
+    uint32_t* sample_counts) {
+    const uint32_t begin = KERNEL == BF_SHADE_ANY || !order ? 0u : P.bucket_ranges[BF_BUCKET_LAMBERT];
+    const uint32_t end = !order ? *count_ptr : P.bucket_ranges[KERNEL == BF_SHADE_ANY ? BF_BUCKET_LAMBERT : BF_BUCKET_DIELECTRIC + 1u];
+    /* without an order the queue holds one kind */
+    const uint32_t lambert_end = order ? P.bucket_ranges[BF_BUCKET_CONDUCTOR] : 0u;
+    const uint32_t conductor_end =
+        order ? P.bucket_ranges[BF_BUCKET_DIELECTRIC] : (P.shade_buckets >> BF_BUCKET_CONDUCTOR & 1u) != 0u ? end : 0u;
+    for (uint32_t i = begin + blockIdx.x * blockDim.x + threadIdx.x; i < end; i += gridDim.x * blockDim.x) {
+        /* a single closure's items from the end: the longest, the dielectrics, first */
+        const uint32_t at = KERNEL == BF_SHADE_SINGLE ? end - 1u - (i - begin) : i;
+        const uint32_t item = order ? order[at] : at;
+        uint32_t code;
+        if constexpr (KERNEL != BF_SHADE_SINGLE) {
+            code = shade_item<BATCH, MODE, KERNEL>(P, queue, item, route, sample_counts);
+        } else if (at < lambert_end) {
+            code = shade_item<BATCH, MODE, BF_SHADE_LAMBERT>(P, queue, item, route, sample_counts);
+        } else if (at < conductor_end) {
+            code = shade_item<BATCH, MODE, BF_SHADE_CONDUCTOR>(P, queue, item, route, sample_counts);
+        } else {
+            code = shade_item<BATCH, MODE, BF_SHADE_DIELECTRIC>(P, queue, item, route, sample_counts);
+        }
+        if (code != 0u) {
+            const uint32_t slot = queue[item];
+            fail_path(P, job_at<BATCH>(P, slot), slot, code);
+        }
     }
-    const uint32_t needed = blocks_for(max_count, BF_SHADE_BLOCK);
-    const uint32_t resident = mode == BF_SHADE_ADJOINT ? P->adjoint_shade_blocks : P->shade_blocks;
-    const dim3 grid(needed < resident ? needed : resident);
-    if (batch) launch_shade<true>(P, grid, queue, count_ptr, order, route, sample_counts, mode, s);
-    else launch_shade<false>(P, grid, queue, count_ptr, order, route, sample_counts, mode, s);
-    return hipGetLastError();
+}
+
+#define BF_JOIN2(a, b) a##b
+#define BF_JOIN(a, b) BF_JOIN2(a, b)
+
+template <uint32_t KERNEL>
+static void launch_kernel(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr, uint32_t max_count,
+                         const uint32_t* order, uint8_t* route, uint32_t* sample_counts, bool batch, hipStream_t s) {
+    const uint32_t grid = std::min(blocks_for(max_count, BF_SHADE_BLOCK), P->shade_blocks[BF_SHADE_MODE * BF_SHADE_KERNELS + KERNEL]);
+    if (batch)
+        hipLaunchKernelGGL((k_shade<true, BF_SHADE_MODE, KERNEL>), dim3(grid), dim3(BF_SHADE_BLOCK), 0, s, *P, queue, count_ptr,
+                           order, route, sample_counts);
+    else
+        hipLaunchKernelGGL((k_shade<false, BF_SHADE_MODE, KERNEL>), dim3(grid), dim3(BF_SHADE_BLOCK), 0, s, *P, queue, count_ptr,
+                           order, route, sample_counts);
+}
+
+template <uint32_t KERNEL>
+static uint32_t kernel_blocks(int device) {
+    const void* plain = (const void*)k_shade<false, BF_SHADE_MODE, KERNEL>;
+    const void* batch = (const void*)k_shade<true, BF_SHADE_MODE, KERNEL>;
+    return (uint32_t)std::min(bfk_max_resident(&plain, 1, BF_SHADE_BLOCK, device), bfk_max_resident(&batch, 1, BF_SHADE_BLOCK, device));
+}
+
+extern "C" {
+
+bool BF_JOIN(bfk_shade_blocks_, BF_SHADE_NAME)(int device, uint32_t* blocks) {
+    blocks[BF_SHADE_ANY] = kernel_blocks<BF_SHADE_ANY>(device);
+    blocks[BF_SHADE_LAMBERT] = kernel_blocks<BF_SHADE_LAMBERT>(device);
+    blocks[BF_SHADE_SINGLE] = kernel_blocks<BF_SHADE_SINGLE>(device);
+    return blocks[0] != 0u && blocks[1] != 0u && blocks[2] != 0u;
+}
+
+void BF_JOIN(bfk_shade_, BF_SHADE_NAME)(const bf_transport_params* P, uint32_t kernel, const uint32_t* queue,
+                                        const uint32_t* count_ptr, uint32_t max_count, const uint32_t* order, uint8_t* route,
+                                        uint32_t* sample_counts, bool batch, hipStream_t s) {
+    const auto launch = kernel == BF_SHADE_LAMBERT  ? launch_kernel<BF_SHADE_LAMBERT>
+                        : kernel == BF_SHADE_SINGLE ? launch_kernel<BF_SHADE_SINGLE>
+                                                    : launch_kernel<BF_SHADE_ANY>;
+    launch(P, queue, count_ptr, max_count, order, route, sample_counts, batch, s);
 }
 
 } /* extern "C" */

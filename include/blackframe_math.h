@@ -59,8 +59,8 @@ BF_HD double bf_bits_double(uint64_t bits) {
 #if defined(__HIP_DEVICE_COMPILE__)
 /* gfx950 classifies and takes floats apart in one instruction each (the values of the bit forms
  * below for every float; ldexp rounds once, to nearest even, as a correctly rounded one must) */
-BF_HD int bf_isnan(float v) { return __builtin_isnan(v); }
-BF_HD int bf_isfinite(float v) { return __builtin_isfinite(v); }
+BF_HD bool bf_isnan(float v) { return __builtin_isnan(v); }
+BF_HD bool bf_isfinite(float v) { return __builtin_isfinite(v); }
 #else
 BF_HD int bf_isnan(float v) { return (bf_float_bits(v) & 0x7FFFFFFFu) > 0x7F800000u; }
 BF_HD int bf_isfinite(float v) { return (bf_float_bits(v) & 0x7F800000u) != 0x7F800000u; }
