@@ -1126,8 +1126,7 @@ struct bf_hip_workspace {
     bf_dev_paths paths{};
     uint32_t* queues[4] = {nullptr, nullptr, nullptr, nullptr}; /* ray, hit, shadow, continuation */
     uint8_t* route = nullptr;
-    uint32_t* tile_counts = nullptr;
-    uint32_t* tile_offsets = nullptr;
+    uint32_t* compact_counts = nullptr;
     uint32_t* sizes = nullptr;     /* [0] ray [1] hit [2] shadow [3] cont [4..5] scratch [7] bounce */
     uint32_t* history = nullptr;   /* [bounce][ray, hit, shadow, cont] */
     uint32_t* failure = nullptr;   /* [0] count, [2..3] lowest (job << 48 | path << 8 | failure code) */
@@ -1135,8 +1134,7 @@ struct bf_hip_workspace {
     unsigned long long* traversal = nullptr; /* 6 counters */
     uint32_t* fetch = nullptr;               /* traversal work counters */
     float* replicas = nullptr;               /* BF_GRADIENT_REPLICAS x BF_GRADIENT_ROW adjoint scratch */
-    uint32_t* bucket_counts = nullptr;       /* shade-order grouping: per-tile bucket counts / offsets */
-    uint32_t* bucket_offsets = nullptr;
+    uint32_t* bucket_counts = nullptr;       /* shade-order grouping: per-chunk bucket counts */
     unsigned long long* hashes = nullptr;    /* [bounce][ray, shadow] FNV-1a-64 of the queues */
     uint32_t* host_words = nullptr;          /* pinned readback */
     uint32_t* host_history = nullptr;        /* pinned readback of the history */
@@ -1597,7 +1595,6 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     if (!w) return set_error(BF_RESOURCE_EXHAUSTED, "host allocation failed");
     w->capacity = capacity;
     const uint64_t n = capacity;
-    const uint32_t tiles = bfk_compact_tiles((uint32_t)n);
     hipError_t de = hipGetDevice(&w->device);
     const bool resident = de == hipSuccess && bfk_trace_resident_lanes(w->device, w->trace_lanes);
     if (!resident || !bfk_shade_resident_blocks(w->device, w->shade_blocks)) {
@@ -1614,8 +1611,8 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
                  o_cone = A.add(nullptr, n * 8);
     size_t o_q[4];
     for (int k = 0; k < 4; ++k) o_q[k] = A.add(nullptr, n * 4);
-    const size_t o_bc = A.add(nullptr, (size_t)tiles * 32), o_bo = A.add(nullptr, (size_t)tiles * 32);
-    const size_t o_route = A.add(nullptr, n), o_tc = A.add(nullptr, (size_t)tiles * 8), o_to = A.add(nullptr, (size_t)tiles * 8),
+    const size_t o_bc = A.add(nullptr, BF_PART_COUNTS * 4u);
+    const size_t o_route = A.add(nullptr, n), o_cc = A.add(nullptr, BF_COMPACT_WORDS * 4u),
                  o_sizes = A.add(nullptr, 64), o_hist = A.add(nullptr, BF_HISTORY_BOUNCES * 16), o_fail = A.add(nullptr, 16),
                  o_samp = A.add(nullptr, 16), o_trav = A.add(nullptr, 64), o_fetch = A.add(nullptr, 2 * BF_CLAIM_SEGMENTS * BF_CLAIM_STRIDE * 4),
                  o_ranges = A.add(nullptr, (BF_SHADE_BUCKETS + 1u) * 4), o_hash = A.add(nullptr, BF_REPORT_MAX_BOUNCES * 16),
@@ -1658,10 +1655,8 @@ int blackframe_hip_workspace_create(uint64_t capacity, bf_hip_workspace** out) {
     w->paths.cone = (float2*)(b + o_cone);
     for (int k = 0; k < 4; ++k) w->queues[k] = (uint32_t*)(b + o_q[k]);
     w->route = b + o_route;
-    w->tile_counts = (uint32_t*)(b + o_tc);
+    w->compact_counts = (uint32_t*)(b + o_cc);
     w->bucket_counts = (uint32_t*)(b + o_bc);
-    w->bucket_offsets = (uint32_t*)(b + o_bo);
-    w->tile_offsets = (uint32_t*)(b + o_to);
     w->sizes = (uint32_t*)(b + o_sizes);
     w->history = (uint32_t*)(b + o_hist);
     w->failure = (uint32_t*)(b + o_fail);
@@ -1722,11 +1717,11 @@ int validate_options(const bf_transport_options* o) {
     return BF_OK;
 }
 
-/* Kernels of one shade stage: its shade kernels, and three for an order. */
+/* Kernels of one shade stage: its shade kernels, and two for an order. */
 uint64_t shade_dispatches(const bf_transport_params& P) {
     bool ordered = false;
     const uint32_t kernels = bfk_shade_plan(&P, &ordered);
-    return (uint64_t)__builtin_popcount(kernels) + (ordered ? 3u : 0u);
+    return (uint64_t)__builtin_popcount(kernels) + (ordered ? 2u : 0u);
 }
 
 /* Issues one bounce of the loop on `stream` (no host synchronisation). The adjoint replay stops
@@ -1738,13 +1733,13 @@ int issue_bounce(bf_hip_workspace* w, bf_transport_report& rep, const bf_transpo
 #define STAGE(stage, dispatches, call) HIP_TRY(staged(w, rep, instrument, (stage), (dispatches), stream, [&] { return (call); }))
     if (hash_slot) STAGE(BF_STAGE_AUXILIARY, 1, bfk_queue_hash(ray_q, &w->sizes[0], hash_slot, stream));
     STAGE(BF_STAGE_CLOSEST_HIT, 1, bfk_trace_closest(&P, ray_q, &w->sizes[0], n_max, w->route, counters, batch, stream));
-    STAGE(BF_STAGE_COMPACTION, 3,
-          bfk_compact(w->route, &w->sizes[0], n_max, ray_q, w->tile_counts, w->tile_offsets, w->queues[1], &w->sizes[1], 0u,
+    STAGE(BF_STAGE_COMPACTION, 2,
+          bfk_compact(w->route, &w->sizes[0], n_max, ray_q, w->compact_counts, w->queues[1], &w->sizes[1], 0u,
                       w->queues[2], &w->sizes[4], 0u, stream));
     STAGE(BF_STAGE_SHADE, shade_dispatches(P),
           bfk_shade(&P, w->queues[1], &w->sizes[1], n_max, w->route, w->sample_counts, batch, P.shade_mode, stream));
-    STAGE(BF_STAGE_COMPACTION, 3,
-          bfk_compact(w->route, &w->sizes[1], n_max, w->queues[1], w->tile_counts, w->tile_offsets, w->queues[2],
+    STAGE(BF_STAGE_COMPACTION, 2,
+          bfk_compact(w->route, &w->sizes[1], n_max, w->queues[1], w->compact_counts, w->queues[2],
                       &w->sizes[2], 0u, cont_q, &w->sizes[3], 0u, stream));
     if (adjoint) {
         STAGE(BF_STAGE_AUXILIARY, 1, bfk_bounce_end(w->sizes, w->history, BF_HISTORY_BOUNCES, stream));
@@ -1752,8 +1747,8 @@ int issue_bounce(bf_hip_workspace* w, bf_transport_report& rep, const bf_transpo
     }
     if (hash_slot) STAGE(BF_STAGE_AUXILIARY, 1, bfk_queue_hash(w->queues[2], &w->sizes[2], hash_slot + 1, stream));
     STAGE(BF_STAGE_SHADOW, 1, bfk_trace_shadow(&P, w->queues[2], &w->sizes[2], n_max, w->route, counters, batch, stream));
-    STAGE(BF_STAGE_COMPACTION, 3,
-          bfk_compact(w->route, &w->sizes[2], n_max, w->queues[2], w->tile_counts, w->tile_offsets, w->queues[1],
+    STAGE(BF_STAGE_COMPACTION, 2,
+          bfk_compact(w->route, &w->sizes[2], n_max, w->queues[2], w->compact_counts, w->queues[1],
                       &w->sizes[5], 0u, cont_q, &w->sizes[3], 1u, stream));
     STAGE(BF_STAGE_AUXILIARY, 1, bfk_bounce_end(w->sizes, w->history, BF_HISTORY_BOUNCES, stream));
 #undef STAGE
@@ -1891,7 +1886,6 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
     P.fetch = w->fetch;
     P.gradient_replicas = w->replicas;
     P.bucket_counts = w->bucket_counts;
-    P.bucket_offsets = w->bucket_offsets;
     /* orders live in queues that are free while the stage runs: the shadow queue is built after
      * shade (and is empty during closest hit); the hit queue is consumed before the shadow stage */
     if (o->launch & BF_LAUNCH_TRACE_ORDER) {
@@ -2048,8 +2042,8 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
             /* path inputs: only the paths whose inputs validated enter the ray queue (sizes[6] holds
              * the slot count the compaction reads) */
             STAGE(BF_STAGE_AUXILIARY, 1, bfk_set_words(w->sizes + 6, 1, n, stream));
-            STAGE(BF_STAGE_COMPACTION, 3,
-                  bfk_compact(w->route, &w->sizes[6], n, cont_q, w->tile_counts, w->tile_offsets, ray_q, &w->sizes[0], 0u,
+            STAGE(BF_STAGE_COMPACTION, 2,
+                  bfk_compact(w->route, &w->sizes[6], n, cont_q, w->compact_counts, ray_q, &w->sizes[0], 0u,
                               w->queues[2], &w->sizes[4], 0u, stream));
         }
         const bool record = o->record_queues && first_launch;

@@ -110,8 +110,7 @@ typedef struct bf_transport_params {
     uint32_t* shade_order;      /* where the grouped order of the hit queue goes (a free queue) */
     uint32_t* closest_order;    /* non-null: traversal claims rays grouped by direction octant (free queues) */
     uint32_t* shadow_order;
-    uint32_t* bucket_counts;    /* per-tile bucket counts / offsets of these groupings */
-    uint32_t* bucket_offsets;
+    uint32_t* bucket_counts;    /* per-chunk bucket counts of these groupings (BF_PART_COUNTS words) */
     uint32_t* bucket_ranges;    /* items of bucket b: [ranges[b], ranges[b + 1]) of the order */
 } bf_transport_params;
 
@@ -142,11 +141,13 @@ void bfk_work_order(const bf_transport_params* P, uint32_t key, const uint32_t* 
                     uint32_t max_count, uint8_t* keys, uint32_t* order, bool batch, hipStream_t s);
 /* Workgroups of `block` lanes the device holds at once: the most over `count` kernels, 0 on error. */
 int bfk_max_resident(const void* const* kernels, int count, uint32_t block, int device);
-/* 256-item tiles the compaction of max_count items uses (size of the tile count / offset arrays / 2). */
-uint32_t bfk_compact_tiles(uint32_t max_count);
+/* Words of chunk counts that a partition launch may use: 2 a workgroup in a compaction, one per bucket
+ * in a work order. A compaction holds two bases behind them. */
+#define BF_PART_COUNTS 4096u
+#define BF_COMPACT_WORDS (BF_PART_COUNTS + 2u)
 hipError_t bfk_compact(const uint8_t* route, const uint32_t* count_ptr, uint32_t max_count, const uint32_t* src,
-                       uint32_t* tile_counts, uint32_t* tile_offsets, uint32_t* dst1, uint32_t* size1, uint32_t append1,
-                       uint32_t* dst2, uint32_t* size2, uint32_t append2, hipStream_t s);
+                       uint32_t* counts, uint32_t* dst1, uint32_t* size1, uint32_t append1, uint32_t* dst2, uint32_t* size2,
+                       uint32_t append2, hipStream_t s);
 /* sizes[0..3] -> history[4 * sizes[7]], sizes[0] = sizes[3], sizes[1..5] = 0, ++sizes[7] */
 hipError_t bfk_bounce_end(uint32_t* sizes, uint32_t* history, uint32_t history_bounces, hipStream_t s);
 hipError_t bfk_film(const bf_dev_paths* paths, const bf_dev_job* job, float pdf, float normalization, hipStream_t s);

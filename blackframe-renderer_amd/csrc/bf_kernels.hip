@@ -240,107 +240,188 @@ __global__ __launch_bounds__(BF_BLOCK) void k_camera(bf_transport_params P, uint
     P.paths.ray_direction[slot] = make_float4(d.x, d.y, d.z, J.camera.t_min);
 }
 
-/* ---- stable compaction: wave64 ballot/popcount ranks + tile-offset scan -----------------------
- * For route values r = 1, 2: dst_r[base_r + exclusive_prefix(route == r)] = src[i], which is the
- * stable exclusive-scan append of CudaWavefrontQueueCompaction.cu:55-315. The item count is read
- * on the device and the kernels stride over 256-item tiles, so launches can be issued (and
- * captured) before the count is known. */
-__global__ __launch_bounds__(BF_BLOCK) void k_compact_count(const uint8_t* route, const uint32_t* count_ptr,
-                                                            uint32_t* tile_counts) {
-    __shared__ uint32_t wave_counts[2][BF_BLOCK / 64];
-    const uint32_t n = *count_ptr;
-    const uint32_t tiles = (n + BF_BLOCK - 1u) / BF_BLOCK;
-    const uint32_t wave = threadIdx.x >> 6;
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t i = tile * BF_BLOCK + threadIdx.x;
-        const uint8_t r = i < n ? route[i] : 0;
-        const uint64_t m1 = __ballot(r == 1);
-        const uint64_t m2 = __ballot(r == 2);
-        if ((threadIdx.x & 63u) == 0u) {
-            wave_counts[0][wave] = (uint32_t)__popcll(m1);
-            wave_counts[1][wave] = (uint32_t)__popcll(m2);
+/* ---- stable partition of a queue ---------------------------------------------------------------
+ * A launch has one workgroup per chunk of consecutive items. The first kernel counts each chunk's
+ * items per destination; in the second every workgroup adds up the chunks before its own (a few
+ * thousand words that all of them read from L2) and writes its items behind them, so no kernel of one
+ * workgroup stands between the two: the scan of 256-item tiles that did took 5.6 us where everything
+ * else fits in 4, and 9.6 ms of a 1920x1080x64 frame. The item count is read on the device, so
+ * launches can be issued (and captured) before it is known.
+ *
+ * Within a chunk a workgroup takes BF_PART_TILE items at a time, each wave a run of 128 in rounds of
+ * 64 whose loads are in flight together, with one barrier for the tile. Two rounds: 8 leave a small
+ * launch too few workgroups (a 64x64x16 frame 1573 us, 4 1508, 2 1442), 1 gains nothing more there and
+ * loses in large ones. */
+#define BF_PART_ROUNDS 2u
+#define BF_PART_TILE (BF_PART_ROUNDS * BF_BLOCK)
+
+struct chunk_t {
+    uint32_t begin, end;
+    uint32_t used; /* chunks that hold items, at least one */
+};
+
+/* n < 2^31 (a workspace's capacity) and at most 2^12 chunks, so no product leaves 32 bits */
+BF_D chunk_t own_chunk(uint32_t n) {
+    const uint32_t tiles = (n + BF_PART_TILE - 1u) / BF_PART_TILE;
+    const uint32_t per = tiles > gridDim.x ? (tiles + gridDim.x - 1u) / gridDim.x : 1u;
+    const uint32_t items = per * BF_PART_TILE;
+    const uint32_t begin = blockIdx.x * items;
+    chunk_t c;
+    c.begin = begin < n ? begin : n;
+    c.end = begin + items < n ? begin + items : n;
+    c.used = tiles > 1u ? (per > 1u ? (tiles + per - 1u) / per : tiles) : 1u;
+    return c;
+}
+
+/* chunk_counts[N * blockIdx.x + b] = items of the chunk with key b */
+template <uint32_t N, typename KEY>
+BF_D void count_chunk(uint32_t n, uint32_t* chunk_counts, KEY&& key_at) {
+    __shared__ uint32_t wave_counts[N][BF_BLOCK / 64];
+    const chunk_t c = own_chunk(n);
+    if (blockIdx.x >= c.used) return;
+    uint32_t own[N] = {};
+    for (uint32_t base = c.begin; base < c.end; base += BF_PART_TILE) {
+        uint32_t keys[BF_PART_ROUNDS];
+#pragma unroll
+        for (uint32_t r = 0; r < BF_PART_ROUNDS; ++r) {
+            const uint32_t offset = r * BF_BLOCK + threadIdx.x;
+            keys[r] = offset < c.end - base ? key_at(base + offset) : N;
         }
-        __syncthreads();
-        if (threadIdx.x < 2u) {
-            uint32_t total = 0;
-            for (uint32_t w = 0; w < BF_BLOCK / 64; ++w) total += wave_counts[threadIdx.x][w];
-            tile_counts[2 * tile + threadIdx.x] = total;
-        }
-        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < BF_PART_ROUNDS; ++r)
+#pragma unroll
+            for (uint32_t b = 0; b < N; ++b) own[b] += (uint32_t)__popcll(__ballot(keys[r] == b));
+    }
+    if ((threadIdx.x & 63u) == 0u)
+#pragma unroll
+        for (uint32_t b = 0; b < N; ++b) wave_counts[b][threadIdx.x >> 6] = own[b];
+    __syncthreads();
+    if (threadIdx.x < N) {
+        uint32_t total = 0;
+        for (uint32_t w = 0; w < BF_BLOCK / 64; ++w) total += wave_counts[threadIdx.x][w];
+        chunk_counts[N * blockIdx.x + threadIdx.x] = total;
     }
 }
 
-/* single workgroup: exclusive scan of the per-tile counts for both routes, plus the queue bases */
-__global__ __launch_bounds__(1024) void k_compact_scan(const uint32_t* count_ptr, const uint32_t* tile_counts,
-                                                       uint32_t* tile_offsets, uint32_t* size1, uint32_t* size2,
-                                                       uint32_t append1, uint32_t append2) {
-    __shared__ uint32_t partial[2][1024];
-    const uint32_t t = threadIdx.x;
-    const uint32_t tiles = (*count_ptr + BF_BLOCK - 1u) / BF_BLOCK;
-    const uint32_t per = (tiles + 1023u) / 1024u;
-    const uint32_t begin = t * per;
-    const uint32_t end = begin + per < tiles ? begin + per : tiles;
-    uint32_t s1 = 0, s2 = 0;
-    for (uint32_t b = begin; b < end; ++b) {
-        s1 += tile_counts[2 * b];
-        s2 += tile_counts[2 * b + 1];
-    }
-    partial[0][t] = s1;
-    partial[1][t] = s2;
+/* before[b], all[b]: items with key b in the chunks before this one, and in all of them */
+template <uint32_t N>
+BF_D void chunk_prefix(const chunk_t& c, const uint32_t* chunk_counts, uint32_t (&before)[N], uint32_t (&all)[N]) {
+    __shared__ uint32_t partial[2][N][BF_BLOCK / 64];
+    uint32_t lower[N] = {}, every[N] = {};
+    for (uint32_t k = threadIdx.x; k < c.used; k += BF_BLOCK)
+#pragma unroll
+        for (uint32_t b = 0; b < N; ++b) {
+            const uint32_t v = chunk_counts[N * k + b];
+            every[b] += v;
+            lower[b] += k < blockIdx.x ? v : 0u;
+        }
+#pragma unroll
+    for (uint32_t b = 0; b < N; ++b)
+#pragma unroll
+        for (uint32_t step = 32u; step != 0u; step >>= 1) {
+            every[b] += __shfl_xor(every[b], (int)step, 64);
+            lower[b] += __shfl_xor(lower[b], (int)step, 64);
+        }
+    if ((threadIdx.x & 63u) == 0u)
+#pragma unroll
+        for (uint32_t b = 0; b < N; ++b) {
+            partial[0][b][threadIdx.x >> 6] = lower[b];
+            partial[1][b][threadIdx.x >> 6] = every[b];
+        }
     __syncthreads();
-    for (uint32_t off = 1; off < 1024u; off <<= 1) {
-        const uint32_t a = t >= off ? partial[0][t - off] : 0u;
-        const uint32_t c = t >= off ? partial[1][t - off] : 0u;
-        __syncthreads();
-        partial[0][t] += a;
-        partial[1][t] += c;
-        __syncthreads();
-    }
-    const uint32_t base1 = append1 ? *size1 : 0u;
-    const uint32_t base2 = append2 ? *size2 : 0u;
-    uint32_t run1 = base1 + partial[0][t] - s1;
-    uint32_t run2 = base2 + partial[1][t] - s2;
-    for (uint32_t b = begin; b < end; ++b) {
-        tile_offsets[2 * b] = run1;
-        tile_offsets[2 * b + 1] = run2;
-        run1 += tile_counts[2 * b];
-        run2 += tile_counts[2 * b + 1];
-    }
-    __syncthreads();
-    if (t == 1023u) {
-        *size1 = base1 + partial[0][1023];
-        *size2 = base2 + partial[1][1023];
+#pragma unroll
+    for (uint32_t b = 0; b < N; ++b) {
+        before[b] = 0u;
+        all[b] = 0u;
+#pragma unroll
+        for (uint32_t w = 0; w < BF_BLOCK / 64; ++w) {
+            before[b] += partial[0][b][w];
+            all[b] += partial[1][b][w];
+        }
     }
 }
 
-__global__ __launch_bounds__(BF_BLOCK) void k_compact_scatter(const uint8_t* route, const uint32_t* count_ptr,
-                                                              const uint32_t* src, const uint32_t* tile_offsets,
-                                                              uint32_t* dst1, uint32_t* dst2) {
-    __shared__ uint32_t wave_counts[2][BF_BLOCK / 64];
-    const uint32_t n = *count_ptr;
-    const uint32_t tiles = (n + BF_BLOCK - 1u) / BF_BLOCK;
+/* put(i, b, p) for every item i of the chunk with key b < N: p counts from run[b] up, in queue order */
+template <uint32_t N, typename KEY, typename PUT>
+BF_D void scatter_chunk(const chunk_t& c, uint32_t (&run)[N], KEY&& key_at, PUT&& put) {
+    __shared__ uint32_t wave_counts[2][N][BF_BLOCK / 64];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = threadIdx.x >> 6;
     const uint64_t below = lane == 0u ? 0ull : (~0ull >> (64u - lane));
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t i = tile * BF_BLOCK + threadIdx.x;
-        const uint8_t r = i < n ? route[i] : 0;
-        const uint64_t m1 = __ballot(r == 1);
-        const uint64_t m2 = __ballot(r == 2);
-        if (lane == 0u) {
-            wave_counts[0][wave] = (uint32_t)__popcll(m1);
-            wave_counts[1][wave] = (uint32_t)__popcll(m2);
+    uint32_t parity = 0;
+    for (uint32_t base = c.begin; base < c.end; base += BF_PART_TILE, parity ^= 1u) {
+        uint32_t keys[BF_PART_ROUNDS], own[N] = {};
+#pragma unroll
+        for (uint32_t r = 0; r < BF_PART_ROUNDS; ++r) {
+            const uint32_t offset = (wave * BF_PART_ROUNDS + r) * 64u + lane;
+            keys[r] = offset < c.end - base ? key_at(base + offset) : N;
         }
+#pragma unroll
+        for (uint32_t r = 0; r < BF_PART_ROUNDS; ++r)
+#pragma unroll
+            for (uint32_t b = 0; b < N; ++b) own[b] += (uint32_t)__popcll(__ballot(keys[r] == b));
+        if (lane == 0u)
+#pragma unroll
+            for (uint32_t b = 0; b < N; ++b) wave_counts[parity][b][wave] = own[b];
+        /* the other parity's counts are read by waves of the tile before, the same parity's by none:
+         * a wave gets here again only past the barrier of the tile between */
         __syncthreads();
-        if (r != 0) {
-            const uint32_t k = r - 1u;
-            uint32_t rank = (uint32_t)__popcll((k == 0 ? m1 : m2) & below);
-            for (uint32_t w = 0; w < wave; ++w) rank += wave_counts[k][w];
-            const uint32_t position = tile_offsets[2 * tile + k] + rank;
-            (k == 0 ? dst1 : dst2)[position] = src[i];
+        uint32_t at[N];
+#pragma unroll
+        for (uint32_t b = 0; b < N; ++b) {
+            at[b] = run[b];
+#pragma unroll
+            for (uint32_t w = 0; w < BF_BLOCK / 64; ++w) {
+                const uint32_t v = wave_counts[parity][b][w];
+                at[b] += w < wave ? v : 0u;
+                run[b] += v;
+            }
         }
-        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < BF_PART_ROUNDS; ++r) {
+            uint32_t position = 0;
+#pragma unroll
+            for (uint32_t b = 0; b < N; ++b) {
+                const uint64_t m = __ballot(keys[r] == b);
+                if (keys[r] == b) position = at[b] + (uint32_t)__popcll(m & below);
+                at[b] += (uint32_t)__popcll(m);
+            }
+            if (keys[r] < N) put(base + (wave * BF_PART_ROUNDS + r) * 64u + lane, keys[r], position);
+        }
     }
+}
+
+/* Compaction. For route values r = 1, 2: dst_r[base_r + exclusive_prefix(route == r)] = src[i], which is
+ * the stable exclusive-scan append of CudaWavefrontQueueCompaction.cu:55-315; base_r is the size of
+ * the destination where it is appended to. */
+__global__ __launch_bounds__(BF_BLOCK) void k_compact_count(const uint8_t* route, const uint32_t* count_ptr,
+                                                            uint32_t* chunk_counts, uint32_t* bases, const uint32_t* size1,
+                                                            const uint32_t* size2, uint32_t append1, uint32_t append2) {
+    if (blockIdx.x == 0u && threadIdx.x == 0u) { /* the next kernel overwrites the sizes */
+        bases[0] = append1 ? *size1 : 0u;
+        bases[1] = append2 ? *size2 : 0u;
+    }
+    count_chunk<2u>(*count_ptr, chunk_counts, [&](uint32_t i) { return (uint32_t)route[i] - 1u; });
+}
+
+__global__ __launch_bounds__(BF_BLOCK) void k_compact_scatter(const uint8_t* route, const uint32_t* count_ptr,
+                                                              const uint32_t* src, const uint32_t* chunk_counts,
+                                                              const uint32_t* bases, uint32_t* dst1, uint32_t* dst2,
+                                                              uint32_t* size1, uint32_t* size2) {
+    const chunk_t c = own_chunk(*count_ptr);
+    if (blockIdx.x >= c.used) return;
+    uint32_t run[2], all[2];
+    chunk_prefix<2u>(c, chunk_counts, run, all);
+    const uint32_t base1 = bases[0], base2 = bases[1];
+    if (blockIdx.x == 0u && threadIdx.x == 0u) {
+        *size1 = base1 + all[0];
+        *size2 = base2 + all[1];
+    }
+    run[0] += base1;
+    run[1] += base2;
+    scatter_chunk<2u>(
+        c, run, [&](uint32_t i) { return (uint32_t)route[i] - 1u; },
+        [&](uint32_t i, uint32_t b, uint32_t p) { (b == 0u ? dst1 : dst2)[p] = src[i]; });
 }
 
 /* ---- shade order: hit-queue items grouped by the closure kind of their material ---------------
@@ -368,105 +449,32 @@ BF_D uint32_t bucket_key(const bf_transport_params& P, const uint32_t* queue, ui
 
 template <bool BATCH, uint32_t KEY>
 __global__ __launch_bounds__(BF_BLOCK) void k_bucket_count(bf_transport_params P, const uint32_t* queue,
-                                                           const uint32_t* count_ptr, uint8_t* keys, uint32_t* tile_counts) {
-    __shared__ uint32_t wave_counts[BF_SHADE_BUCKETS][BF_BLOCK / 64];
-    const uint32_t n = *count_ptr;
-    const uint32_t tiles = (n + BF_BLOCK - 1u) / BF_BLOCK;
-    const uint32_t wave = threadIdx.x >> 6;
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t i = tile * BF_BLOCK + threadIdx.x;
-        const uint32_t key = i < n ? bucket_key<BATCH, KEY>(P, queue, i) : BF_SHADE_BUCKETS;
-        if (i < n) keys[i] = (uint8_t)key;
-#pragma unroll
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) {
-            const uint64_t m = __ballot(key == b);
-            if ((threadIdx.x & 63u) == 0u) wave_counts[b][wave] = (uint32_t)__popcll(m);
-        }
-        __syncthreads();
-        if (threadIdx.x < BF_SHADE_BUCKETS) {
-            uint32_t total = 0;
-            for (uint32_t w = 0; w < BF_BLOCK / 64; ++w) total += wave_counts[threadIdx.x][w];
-            tile_counts[BF_SHADE_BUCKETS * tile + threadIdx.x] = total;
-        }
-        __syncthreads();
-    }
+                                                           const uint32_t* count_ptr, uint8_t* keys, uint32_t* chunk_counts) {
+    count_chunk<BF_SHADE_BUCKETS>(*count_ptr, chunk_counts, [&](uint32_t i) {
+        const uint32_t key = bucket_key<BATCH, KEY>(P, queue, i);
+        keys[i] = (uint8_t)key;
+        return key;
+    });
 }
 
-/* single workgroup: tile offsets = bucket base (items of lower buckets) + earlier tiles' counts */
-__global__ __launch_bounds__(1024) void k_bucket_scan(const uint32_t* count_ptr, const uint32_t* tile_counts,
-                                                      uint32_t* tile_offsets, uint32_t* ranges) {
-    __shared__ uint32_t partial[BF_SHADE_BUCKETS][1024];
-    __shared__ uint32_t base[BF_SHADE_BUCKETS];
-    const uint32_t t = threadIdx.x;
-    const uint32_t tiles = (*count_ptr + BF_BLOCK - 1u) / BF_BLOCK;
-    const uint32_t per = (tiles + 1023u) / 1024u;
-    const uint32_t begin = t * per;
-    const uint32_t end = begin + per < tiles ? begin + per : tiles;
-    uint32_t own[BF_SHADE_BUCKETS];
-#pragma unroll
-    for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) own[b] = 0u;
-    for (uint32_t tile = begin; tile < end; ++tile)
-#pragma unroll
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) own[b] += tile_counts[BF_SHADE_BUCKETS * tile + b];
-#pragma unroll
-    for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) partial[b][t] = own[b];
-    __syncthreads();
-    for (uint32_t off = 1; off < 1024u; off <<= 1) {
-        uint32_t add[BF_SHADE_BUCKETS];
-#pragma unroll
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) add[b] = t >= off ? partial[b][t - off] : 0u;
-        __syncthreads();
-#pragma unroll
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) partial[b][t] += add[b];
-        __syncthreads();
-    }
-    if (t == 0u) {
-        uint32_t run = 0;
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) {
-            base[b] = run;
-            ranges[b] = run;
-            run += partial[b][1023];
-        }
-        ranges[BF_SHADE_BUCKETS] = run;
-    }
-    __syncthreads();
-    uint32_t run[BF_SHADE_BUCKETS];
-#pragma unroll
-    for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) run[b] = base[b] + partial[b][t] - own[b];
-    for (uint32_t tile = begin; tile < end; ++tile)
-#pragma unroll
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) {
-            tile_offsets[BF_SHADE_BUCKETS * tile + b] = run[b];
-            run[b] += tile_counts[BF_SHADE_BUCKETS * tile + b];
-        }
-}
-
+/* Bucket b starts behind the items of the lower ones: at ranges[b]. */
 __global__ __launch_bounds__(BF_BLOCK) void k_bucket_scatter(const uint8_t* keys, const uint32_t* count_ptr,
-                                                             const uint32_t* tile_offsets, uint32_t* order) {
-    __shared__ uint32_t wave_counts[BF_SHADE_BUCKETS][BF_BLOCK / 64];
-    const uint32_t n = *count_ptr;
-    const uint32_t tiles = (n + BF_BLOCK - 1u) / BF_BLOCK;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
-    const uint64_t below = lane == 0u ? 0ull : (~0ull >> (64u - lane));
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t i = tile * BF_BLOCK + threadIdx.x;
-        const uint32_t key = i < n ? keys[i] : BF_SHADE_BUCKETS;
-        uint64_t mine = 0ull;
+                                                             const uint32_t* chunk_counts, uint32_t* ranges, uint32_t* order) {
+    const chunk_t c = own_chunk(*count_ptr);
+    if (blockIdx.x >= c.used) return;
+    uint32_t run[BF_SHADE_BUCKETS], all[BF_SHADE_BUCKETS];
+    chunk_prefix<BF_SHADE_BUCKETS>(c, chunk_counts, run, all);
+    uint32_t start = 0;
 #pragma unroll
-        for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) {
-            const uint64_t m = __ballot(key == b);
-            if (key == b) mine = m;
-            if (lane == 0u) wave_counts[b][wave] = (uint32_t)__popcll(m);
-        }
-        __syncthreads();
-        if (key < BF_SHADE_BUCKETS) {
-            uint32_t rank = (uint32_t)__popcll(mine & below);
-            for (uint32_t w = 0; w < wave; ++w) rank += wave_counts[key][w];
-            order[tile_offsets[BF_SHADE_BUCKETS * tile + key] + rank] = i;
-        }
-        __syncthreads();
+    for (uint32_t b = 0; b < BF_SHADE_BUCKETS; ++b) {
+        run[b] += start;
+        if (blockIdx.x == 0u && threadIdx.x == 0u) ranges[b] = start;
+        start += all[b];
     }
+    if (blockIdx.x == 0u && threadIdx.x == 0u) ranges[BF_SHADE_BUCKETS] = start;
+    scatter_chunk<BF_SHADE_BUCKETS>(
+        c, run, [&](uint32_t i) { return (uint32_t)keys[i]; },
+        [&](uint32_t i, uint32_t, uint32_t p) { order[p] = i; });
 }
 
 /* End of a bounce: record the queue sizes of the bounce, make the continuation queue the next ray
@@ -1251,15 +1259,18 @@ hipError_t bfk_camera(const bf_transport_params* P, uint32_t count, uint32_t* ra
 
 } /* extern "C" */
 
+/* Workgroups of a partition: one tile each, until the counts that each of them adds up (`keys` words a
+ * workgroup) would outweigh its items. */
+static uint32_t partition_blocks(uint32_t max_count, uint32_t keys) {
+    return std::min(blocks_for(max_count ? max_count : 1u, BF_PART_TILE), BF_PART_COUNTS / keys);
+}
+
 template <bool BATCH, uint32_t KEY>
 static void launch_work_order(const bf_transport_params* P, const uint32_t* queue, const uint32_t* count_ptr,
-                               uint32_t max_count, uint8_t* keys, uint32_t* tile_counts, uint32_t* tile_offsets,
-                               uint32_t* order, hipStream_t s) {
-    const uint32_t tiles = bfk_compact_tiles(max_count);
-    const dim3 grid(tiles < 4096u ? tiles : 4096u);
-    hipLaunchKernelGGL((k_bucket_count<BATCH, KEY>), grid, dim3(BF_BLOCK), 0, s, *P, queue, count_ptr, keys, tile_counts);
-    hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(1024), 0, s, count_ptr, tile_counts, tile_offsets, P->bucket_ranges);
-    hipLaunchKernelGGL(k_bucket_scatter, grid, dim3(BF_BLOCK), 0, s, keys, count_ptr, tile_offsets, order);
+                               uint32_t max_count, uint8_t* keys, uint32_t* order, hipStream_t s) {
+    const dim3 grid(partition_blocks(max_count, BF_SHADE_BUCKETS));
+    hipLaunchKernelGGL((k_bucket_count<BATCH, KEY>), grid, dim3(BF_BLOCK), 0, s, *P, queue, count_ptr, keys, P->bucket_counts);
+    hipLaunchKernelGGL(k_bucket_scatter, grid, dim3(BF_BLOCK), 0, s, keys, count_ptr, P->bucket_counts, P->bucket_ranges, order);
 }
 
 /* max_count items' permutation grouped by `key` into `order`; `keys` holds one byte per item. */
@@ -1267,7 +1278,7 @@ extern "C" {
 
 void bfk_work_order(const bf_transport_params* P, uint32_t key, const uint32_t* queue, const uint32_t* count_ptr,
                     uint32_t max_count, uint8_t* keys, uint32_t* order, bool batch, hipStream_t s) {
-    const auto launch = [&](auto kernel) { kernel(P, queue, count_ptr, max_count, keys, P->bucket_counts, P->bucket_offsets, order, s); };
+    const auto launch = [&](auto kernel) { kernel(P, queue, count_ptr, max_count, keys, order, s); };
     if (key == BF_KEY_SHADE) launch(batch ? launch_work_order<true, BF_KEY_SHADE> : launch_work_order<false, BF_KEY_SHADE>);
     else if (key == BF_KEY_RAY) launch(batch ? launch_work_order<true, BF_KEY_RAY> : launch_work_order<false, BF_KEY_RAY>);
     else launch(batch ? launch_work_order<true, BF_KEY_SHADOW> : launch_work_order<false, BF_KEY_SHADOW>);
@@ -1322,17 +1333,15 @@ int bfk_max_resident(const void* const* kernels, int count, uint32_t block, int 
     return cus * m;
 }
 
-uint32_t bfk_compact_tiles(uint32_t max_count) { return blocks_for(max_count ? max_count : 1u, BF_BLOCK); }
-
 hipError_t bfk_compact(const uint8_t* route, const uint32_t* count_ptr, uint32_t max_count, const uint32_t* src,
-                       uint32_t* tile_counts, uint32_t* tile_offsets, uint32_t* dst1, uint32_t* size1, uint32_t append1,
-                       uint32_t* dst2, uint32_t* size2, uint32_t append2, hipStream_t s) {
-    const uint32_t tiles = bfk_compact_tiles(max_count);
-    const dim3 grid(tiles < 4096u ? tiles : 4096u);
-    hipLaunchKernelGGL(k_compact_count, grid, dim3(BF_BLOCK), 0, s, route, count_ptr, tile_counts);
-    hipLaunchKernelGGL(k_compact_scan, dim3(1), dim3(1024), 0, s, count_ptr, tile_counts, tile_offsets, size1, size2,
-                       append1, append2);
-    hipLaunchKernelGGL(k_compact_scatter, grid, dim3(BF_BLOCK), 0, s, route, count_ptr, src, tile_offsets, dst1, dst2);
+                       uint32_t* counts, uint32_t* dst1, uint32_t* size1, uint32_t append1, uint32_t* dst2, uint32_t* size2,
+                       uint32_t append2, hipStream_t s) {
+    const dim3 grid(partition_blocks(max_count, 2u));
+    uint32_t* bases = counts + BF_PART_COUNTS;
+    hipLaunchKernelGGL(k_compact_count, grid, dim3(BF_BLOCK), 0, s, route, count_ptr, counts, bases, size1, size2, append1,
+                       append2);
+    hipLaunchKernelGGL(k_compact_scatter, grid, dim3(BF_BLOCK), 0, s, route, count_ptr, src, counts, bases, dst1, dst2, size1,
+                       size2);
     return hipGetLastError();
 }
 

@@ -87,3 +87,20 @@ def test_light_counts(bf, oracle, hip, lights, sampler):
 
 def test_sample_indexes_past_a_byte(bf, oracle, hip):
     check(bf, oracle, hip, boxes(bf, ("lambert", "dielectric"), 4, 2, 2), 2, 2, 515, max_depth=4)
+
+
+def test_partitions_of_several_tiles_a_workgroup(bf, hip):
+    """9.4 M paths in one launch, past one tile of 512 items a workgroup in the compactions (from 1 M) and
+    in the shade order (from 256 K), against a launch per sample."""
+    width, height, spp = 1025, 1021, 9
+    scene, camera = boxes(bf, ("lambert", "conductor", "dielectric", "mixture"), 1, width, height)
+    frame = bf.scenes.frame_desc(camera, spp)
+    options = bf.scenes.transport_options(max_depth=3)
+    device_scene = hip.XpuScene(scene)
+    films = []
+    for capacity in (width * height * spp, width * height):
+        ws = hip.XpuWavefrontTransportWorkspace(capacity)
+        films.append(hip.trace_xpu_wavefront_transport(ws, device_scene, frame, options)["film"].host())
+        ws.close()
+    for name in ("film", "film_counts"):
+        assert np.array_equal(films[0][name].view(np.uint32), films[1][name].view(np.uint32)), name
