@@ -677,7 +677,7 @@ def main():
         "paths_per_s": round(path_count * args.steps / elapsed, 1),
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_trace_closest",
+            "kernel": "k_trace<closest hit>",
             "achieved": round(achieved, 2),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -694,7 +694,7 @@ def main():
                               "ms_per_frame": round(stage_ns[k] / args.steps * 1e-6, 3),
                               "achieved": round(b / (stage_ns[k] / args.steps * 1e-9) / 1e9, 2),
                               "frac": round(b / (stage_ns[k] / args.steps * 1e-9) / 1e9 / HBM_PEAK_GBS, 5)}
-                       for name, k, b in (("k_trace_shadow", 3, shadow_bytes + 208 * report.shadow_queries),
+                       for name, k, b in (("k_trace<any hit>", 3, shadow_bytes + 208 * report.shadow_queries),
                                           ("k_shade", 2, 680 * report.shade_lanes))
                        if stage_ns[k] > 0},
         },
