@@ -67,7 +67,7 @@
 #define BF_BUCKET_DIELECTRIC 6u
 
 /* Shade kernels of a mode: any material, Lambertian materials, materials of one closure of a kind
- * that has a bucket. The last two are also what one item is shaded as. */
+ * that has a bucket. One item is shaded as any, Lambertian, conductor or dielectric. */
 #define BF_SHADE_ANY 0u
 #define BF_SHADE_LAMBERT 1u
 #define BF_SHADE_SINGLE 2u
@@ -79,11 +79,11 @@
  * through the vector memory path, which costs more than the waves it would buy: with a budget of 2 the
  * single-closure kernels keep nearly everything in registers (the shade stage of a 1920x1080x64 frame
  * of 1024 instances 65.2 ms, against 75.0 with 3 waves, 83.1 with 4 and 107 with 5; of a 256x256x16
- * frame with maps 8.9 ms, against 16.8 with 3 and 21.2 with 4). The general kernel indexes its closures in
- * scratch whatever its budget and gains from the third wave (9.1 to 8.7 ms in an adjoint replay). */
-#ifndef BF_SHADE_WAVES_PER_SIMD
-#define BF_SHADE_WAVES_PER_SIMD 3 /* any material */
-#endif
+ * frame with maps 8.9 ms, against 16.8 with 3 and 21.2 with 4). The general kernel does too without
+ * texture gradients or texture-weighted mixtures (with maps 8.9 ms against 18.7 with 3 waves; a 640x360x16
+ * frame 5.6 against 6.0); with those its closures, indexed in scratch, keep it waiting whatever its
+ * budget, and the third wave gains (9.1 to 8.8 ms in an adjoint replay, 5.1 to 4.8 in its forward pass). */
+#define BF_SHADE_WAVES_PER_SIMD(mode) ((mode) == 0u || (mode) == 3u ? 2 : 3) /* any material, by mode */
 #ifndef BF_SHADE_SINGLE_WAVES
 #define BF_SHADE_SINGLE_WAVES 2 /* materials of one closure */
 #endif

@@ -99,8 +99,6 @@ BF_D bool texture_value(const bf_dev_scene& S, uint32_t slot, const float* uv, f
     return true;
 }
 
-/* Closure records at the path's wavelengths; textured weights and GGX widths are looked up at the
- * hit's texture coordinates. False when a texture lookup is not representable. */
 /* The closure kind of a class's materials. */
 template <uint32_t CLASS>
 BF_D uint32_t class_kind(uint32_t kind) {
@@ -110,6 +108,8 @@ BF_D uint32_t class_kind(uint32_t kind) {
                                           : kind;
 }
 
+/* Closure records at the path's wavelengths; textured weights and GGX widths are looked up at the
+ * hit's texture coordinates. False when a texture lookup is not representable. */
 template <bool TEX, uint32_t CLASS, uint32_t N>
 BF_D bool load_mixture(const bf_dev_scene& S, const bf_material_desc& M, const float* wl, const float* uv, mixture_t<N>& mix) {
     mix.active_count = N == 1u ? 1u : M.closure_count;
@@ -831,7 +831,7 @@ BF_D uint32_t shade_item(const bf_transport_params& P, const uint32_t* queue, ui
  * frame, against 2.3 with a kernel per kind and 1.5 with the general kernel alone. The Lambertian
  * kernel needs neither the order nor the other kinds' registers. */
 template <bool BATCH, uint32_t MODE, uint32_t KERNEL>
-__global__ __launch_bounds__(BF_SHADE_BLOCK, KERNEL == BF_SHADE_ANY ? BF_SHADE_WAVES_PER_SIMD : BF_SHADE_SINGLE_WAVES) void k_shade(
+__global__ __launch_bounds__(BF_SHADE_BLOCK, KERNEL == BF_SHADE_ANY ? BF_SHADE_WAVES_PER_SIMD(MODE) : BF_SHADE_SINGLE_WAVES) void k_shade(
     bf_transport_params P, const uint32_t* queue, const uint32_t* count_ptr, const uint32_t* order, uint8_t* route,
     uint32_t* sample_counts) {
     const uint32_t begin = KERNEL == BF_SHADE_ANY || !order ? 0u : P.bucket_ranges[BF_BUCKET_LAMBERT];
