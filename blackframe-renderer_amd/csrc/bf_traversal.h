@@ -935,10 +935,11 @@ BF_D void bound_node(WorldRay world, Stack& stack, bound_state& ts) {
     const float lead = nv1 - nv0;
     bool first = both ? lead > 0.0f : h0;
     if (both && !(fabsf(lead) > fmaf(nv0 + nv1, BF_SLAB_REL, 4.0f * BF_SLAB_ABS))) {
-        /* a tie when each axis has equal near planes or lies below both near values */
+        /* a tie when each axis has equal near planes or lies below both near values; NaN reciprocals
+         * tell nothing of the direction's signs, so the near planes are not known here */
         const float below = fmaf(fminf(nv0, nv1), 1.0f - 2.0f * BF_SLAB_REL, -4.0f * BF_SLAB_ABS);
         const float up = 1.0f + BF_SLAB_REL;
-        const bool tie = (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
+        const bool tie = !bf_isnan(ts.inv.x) && (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
                          (n0.y == n1.y || fmaxf(q0.y, q1.y) * up < below) &&
                          (n0.z == n1.z || fmaxf(q0.z, q1.z) * up < below);
         first = true;

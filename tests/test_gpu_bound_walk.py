@@ -124,3 +124,45 @@ def test_deep_stacks_match_the_oracle(bf, abi, oracle, hip):
     xs, want = hip.XpuScene(scene), oracle.scene(scene)
     assert result_bytes(xs.closest_hit(rays)) == result_bytes(want.closest_hit(rays))
     assert result_bytes(xs.occlusion(rays)) == result_bytes(want.occlusion(rays))
+
+
+def stacked_corner(bf, split):
+    """Sibling boxes that share their min corner and differ in extent: triangle A, and B1 in A's plane
+    with B2 above it. A ray from above enters B's box first and finds B1; A's box is then culled where
+    t rounds below it. split: one triangle per instance (siblings in the TLAS) or one geometry."""
+    s = bf.scenes.Scene()
+    material = s.add_material(1, [bf.scenes.lambert(0.5)])
+    triangles = [[[0, 0, 0], [2, 0, 0], [0, 0, 2]], [[0, 0, 0], [6, 0, 0], [0, 0, 2]], [[4, 3, 0], [6, 4, 0], [6, 4, 2]]]
+    for k, group in enumerate([[t] for t in triangles] if split else [triangles]):
+        corners = np.concatenate(group)
+        g = s.add_geometry(11 + k, corners, [[0, 1, 0]] * len(corners), [[0, 0]] * len(corners),
+                           np.arange(len(corners)).reshape(-1, 3))
+        s.add_instance(100 + k, 100 + k, g, material, bf.scenes.affine())
+    s.set_environment(0.25)
+    return s.finalize()
+
+
+@pytest.mark.parametrize("split", [False, True], ids=["blas", "tlas"])
+@pytest.mark.parametrize("direction", [(-0.01, -1.0, 1e-42), (-0.01, -1.0, -1e-42), (-1e-42, -1.0, 0.01),
+                                       (-0.01 * 2.0 ** 127, -(2.0 ** 127), -0.02 * 2.0 ** 127)],
+                         ids=["up", "down", "x", "huge"])
+def test_sibling_order_where_bounds_do_not_hold(bf, abi, oracle, hip, split, direction):
+    """Directions without binary32 reciprocals (a subnormal component, or past 2^126) and negative others."""
+    rng = np.random.default_rng(4)
+    n = 4000
+    rays = (abi.TransportRay * n)()
+    view = np.frombuffer(rays, dtype=np.float32).reshape(n, 12)
+    view[:, 0:3] = rng.uniform([0.0, 4.5, 0.0], [2.0, 9.0, 2.0], size=(n, 3))
+    view[:, 4:7] = np.array(direction) * rng.uniform(0.7, 1.3, size=(n, 1))
+    view[:, 7], view[:, 8] = np.inf, 0.5
+    np.frombuffer(rays, dtype=np.uint32).reshape(n, 12)[:, 9] = 0xFFFFFFFF
+    scene = stacked_corner(bf, split)
+    xs, want = hip.XpuScene(scene), oracle.scene(scene)
+    expected = as_u32(want.closest_hit(rays))
+    # the order is what decides: both triangles of the plane are answers
+    assert len(np.unique(expected[expected[:, 0] == abi.HIT_HIT][:, 13:16], axis=0)) > 1
+    differ = np.nonzero((as_u32(xs.closest_hit(rays)) != expected).any(axis=1))[0]
+    assert differ.size == 0, f"{differ.size} of {n} hits differ, first {differ[:5].tolist()}"
+    options = bf.scenes.transport_options(max_depth=2, rr_first_depth=0)
+    options.failure_policy = abi.FAILURES_COUNT
+    compare(hip, oracle, scene, path_inputs(abi, rays), options)
