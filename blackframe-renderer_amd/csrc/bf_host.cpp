@@ -1152,6 +1152,7 @@ struct bf_hip_workspace {
     bf_transport_params graph_params{};
     uint32_t graph_n = 0, graph_group = 0;
     const uint32_t* graph_ray_q = nullptr;
+    uint64_t graph_dispatches[BF_STAGE_COUNT] = {}; /* what a replay reports, counted at the capture */
     /* bounce groups are captured on this stream (the caller's may be the legacy null stream,
      * which cannot capture) and replayed on the caller's */
     hipStream_t capture_stream = nullptr;
@@ -2070,14 +2071,14 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
                         (void)hipGraphExecDestroy(w->graph);
                         w->graph = nullptr;
                     }
-                    bf_transport_report unused{};
+                    bf_transport_report captured{};
                     if (!w->capture_stream) HIP_TRY(hipStreamCreateWithFlags(&w->capture_stream, hipStreamNonBlocking));
                     HIP_TRY(hipStreamBeginCapture(w->capture_stream, hipStreamCaptureModeThreadLocal));
                     int ist = BF_OK;
                     uint32_t* rq = ray_q;
                     uint32_t* cq = cont_q;
                     for (uint32_t k = 0; k < group && ist == BF_OK; ++k) {
-                        ist = issue_bounce(w, unused, P, batch, false, n, rq, cq, nullptr, nullptr, w->capture_stream);
+                        ist = issue_bounce(w, captured, P, batch, false, n, rq, cq, nullptr, nullptr, w->capture_stream);
                         std::swap(rq, cq);
                     }
                     hipGraph_t g = nullptr;
@@ -2097,13 +2098,12 @@ int trace_jobs(bf_hip_workspace* w, const bf_frame_job* jobs, const bf_adjoint_j
                     w->graph_n = n;
                     w->graph_group = group;
                     w->graph_ray_q = ray_q;
+                    for (uint32_t k = 0; k < BF_STAGE_COUNT; ++k)
+                        w->graph_dispatches[k] = captured.stage_metrics[k].kernel_dispatches;
                 }
                 HIP_TRY(hipGraphLaunch(w->graph, stream));
-                rep.stage_metrics[BF_STAGE_CLOSEST_HIT].kernel_dispatches += group;
-                rep.stage_metrics[BF_STAGE_SHADE].kernel_dispatches += group * shade_dispatches(P);
-                if (!adjoint) rep.stage_metrics[BF_STAGE_SHADOW].kernel_dispatches += group;
-                rep.stage_metrics[BF_STAGE_COMPACTION].kernel_dispatches += (adjoint ? 6u : 9u) * group;
-                rep.stage_metrics[BF_STAGE_AUXILIARY].kernel_dispatches += group;
+                for (uint32_t k = 0; k < BF_STAGE_COUNT; ++k)
+                    rep.stage_metrics[k].kernel_dispatches += w->graph_dispatches[k];
             } else {
                 for (uint32_t k = 0; k < steps; ++k) {
                     const bool rec = record && bounce + k < BF_REPORT_MAX_BOUNCES;

@@ -68,6 +68,29 @@ def test_single_frame_graph_replay_bit_exact(bf, oracle, hip):
         assert np.array_equal(got["film"].host()["film"], expected["film"])
 
 
+def test_replayed_groups_report_the_dispatches_of_issued_ones(bf, hip):
+    """stage_metrics count the kernels of a replayed bounce group as those of a group issued one by one."""
+    import torch
+
+    albedo = torch.full((8, 8, 3), 0.5, device="cuda")
+    roughness = torch.full((1, 1, 1), 0.3, device="cuda")
+    scene, cam, _ = bf.scenes.textured_cornell(24, 24, albedo=(albedo.data_ptr(), 8, 8, 3),
+                                               roughness=(roughness.data_ptr(), 1, 1, 1))
+    xs, frame = hip.XpuScene(scene), bf.scenes.frame_desc(cam, 2)
+    film_gradient = torch.ones(24 * 24 * 3, device="cuda")
+    counts = []
+    for launch in (3, bf.abi.LAUNCH_GRAPH | 3):
+        options = bf.scenes.transport_options(max_depth=8)
+        options.launch = launch
+        ws, tape = hip.XpuWavefrontTransportWorkspace(24 * 24 * 2), hip.Tape(24 * 24 * 2)
+        for _ in range(2):  # the second call replays what the first captured
+            forward = hip.trace_xpu_wavefront_transport(ws, xs, frame, options, tape=tape)["report"]
+            gradients = [torch.zeros_like(albedo), torch.zeros_like(roughness)]
+            adjoint = hip.trace_xpu_wavefront_adjoint(ws, [(xs, frame, tape, film_gradient, gradients)], options)
+            counts.append([[m.kernel_dispatches for m in r.stage_metrics] for r in (forward, adjoint)])
+    assert counts[0][0][4] > 0 and all(c == counts[0] for c in counts), counts
+
+
 @pytest.mark.parametrize("lanes,order", [(64, 0), (256, 0), (128, 0x00100000), (128, 0x00200000), (256, 0x00300000)])
 def test_traversal_workgroup_sizes_bit_exact(bf, oracle, hip, lanes, order):
     """The autotuner's traversal workgroup sizes and the shade / traversal orders
