@@ -169,6 +169,8 @@ BFK_SHADE_MODE_DECLARE(textured)
 BFK_SHADE_MODE_DECLARE(adjoint)
 BFK_SHADE_MODE_DECLARE(mapped)
 hipError_t bfk_queue_hash(const uint32_t* queue, const uint32_t* count_ptr, unsigned long long* out, hipStream_t s);
+/* The cut of a stand-alone ray query: workgroups, and the rays of each. */
+uint32_t bfk_ray_grid(uint32_t count, uint32_t* chunk);
 hipError_t bfk_scene_closest_hit(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count,
                                  bf_closest_hit_result* results, uint32_t* counters, hipStream_t s);
 /* traversal over the reference's device blobs (scene "BLKFSOA4", BVH "BLKFBVH1"); results are

@@ -10,7 +10,7 @@
 
 #define BF_BLOCK 256u
 
-static inline uint32_t blocks_for(uint32_t n, uint32_t b) { return (n + b - 1u) / b; }
+static inline uint32_t blocks_for(uint32_t n, uint32_t b) { return n / b + (n % b != 0u ? 1u : 0u); } /* n + b may not fit */
 
 /* ---- path helpers ----------------------------------------------------------------------------- */
 /* The frame a slot belongs to: the kernel argument in a single-frame launch, the job table entry

@@ -1065,12 +1065,19 @@ bool bfk_trace_resident_lanes(int device, uint32_t* lanes) {
 
 } /* extern "C" */
 
-/* Rays a wave of the bound walk takes: an equal share of one resident generation of waves (6 on
- * each of the device's SIMDs), at most 256 so that the last waves of a large launch even out. */
-static uint32_t ray_chunk(uint32_t count) {
+extern "C" {
+
+/* How a stand-alone query of `count` > 0 rays is cut: `chunk` consecutive rays a wave, one wave a
+ * workgroup; returns the workgroups. An equal share of 6 waves on each of the 1024 SIMDs of an undivided
+ * MI355X, at most 256 rays so that the last waves of a large launch even out. The SIMD count is a tuning
+ * constant (results do not depend on the cut), not the device's own. */
+uint32_t bfk_ray_grid(uint32_t count, uint32_t* chunk) {
     const uint32_t waves = 6u * 4u * 256u;
-    return std::min(blocks_for(count, waves), 256u);
+    *chunk = std::min(blocks_for(count, waves), 256u);
+    return blocks_for(count, *chunk);
 }
+
+} /* extern "C" */
 
 template <bool ANY>
 static hipError_t scene_trace(const bf_dev_scene* S, const bf_transport_ray* rays, uint32_t count, void* results,
@@ -1080,9 +1087,9 @@ static hipError_t scene_trace(const bf_dev_scene* S, const bf_transport_ray* ray
         hipLaunchKernelGGL(k_scene_counting<ANY>, dim3(blocks_for(count, BF_API_BLOCK)), dim3(BF_API_BLOCK), 0, s, *S, rays,
                            count, results, counters);
     } else {
-        const uint32_t chunk = ray_chunk(count);
-        hipLaunchKernelGGL(k_scene_trace<ANY>, dim3(blocks_for(count, chunk)), dim3(BF_API_BLOCK), 0, s, *S, rays, count,
-                           chunk, results);
+        uint32_t chunk = 0;
+        const uint32_t grid = bfk_ray_grid(count, &chunk);
+        hipLaunchKernelGGL(k_scene_trace<ANY>, dim3(grid), dim3(BF_API_BLOCK), 0, s, *S, rays, count, chunk, results);
     }
     return hipGetLastError();
 }

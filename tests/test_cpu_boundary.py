@@ -146,3 +146,14 @@ def test_extension_negotiation(abi, hip):
     assert backend.get_device_descriptor(None, 1 << 20, C.byref(desc)) == 5
     desc.struct_size = 4
     assert backend.get_device_descriptor(None, 0, C.byref(desc)) == 1
+
+
+@pytest.mark.parametrize("count", [1, 63, 6143, 6144, 6145, 1572864, 1572865, 2 ** 31, 2 ** 32 - 6144, 2 ** 32 - 6143, 2 ** 32 - 1])
+def test_ray_queries_of_any_count_are_cut_without_a_remainder(hip, count):
+    """Every ray in one workgroup's chunk, no workgroup without rays, up to the largest count the ABI takes."""
+    grid = C.CDLL(str(hip.LIB_PATH)).bfk_ray_grid
+    grid.argtypes, grid.restype = [C.c_uint32, C.POINTER(C.c_uint32)], C.c_uint32
+    chunk = C.c_uint32(0)
+    blocks = grid(count, C.byref(chunk))
+    assert 1 <= chunk.value <= 256
+    assert (blocks - 1) * chunk.value < count <= blocks * chunk.value
