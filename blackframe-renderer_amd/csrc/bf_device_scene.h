@@ -39,8 +39,18 @@
 #ifndef BF_TRACE_WAVES_PER_SIMD
 #define BF_TRACE_WAVES_PER_SIMD 6 /* register budget of the closest-hit traversal (waves per SIMD) */
 #endif
+/* The step-exact counting walk, whose binary64 reciprocals want registers: the closest-hit kernel spills 6
+ * at 4 waves per SIMD, 58 at 5 and 159 at 6. A counted 1920x1080x4 frame of 1024 instances takes 39.4, 46.2
+ * and 65.7 ms with them (3 waves: 42.5). A quarter for its leaf phase: 38.4 ms, half 39.4. Refill at 24
+ * idle lanes: 39.4 ms, 40: 40.1. */
 #ifndef BF_COUNT_WAVES_PER_SIMD
-#define BF_COUNT_WAVES_PER_SIMD 6 /* the step-exact counting walk */
+#define BF_COUNT_WAVES_PER_SIMD 4
+#endif
+#ifndef BF_COUNT_REFILL
+#define BF_COUNT_REFILL 24u
+#endif
+#ifndef BF_COUNT_LEAF_PHASE
+#define BF_COUNT_LEAF_PHASE 4u
 #endif
 #ifndef BF_LEAF_PHASE
 /* Traversal waves step interior nodes and leaves in separate iterations: leaves once they are this

@@ -490,32 +490,20 @@ BF_D void stack_push(trav_stack<S, LANES, Spill>& s, uint2 entry) {
 }
 
 template <uint32_t S, uint32_t LANES, typename Spill>
-BF_D uint2 stack_pop(trav_stack<S, LANES, Spill>& s) {
-    if (S < BF_STACK_DEPTH && s.sp == 0u) {
+BF_D void stack_refill(trav_stack<S, LANES, Spill>& s) {
+    if (S < BF_STACK_DEPTH && s.sp == 0u && s.gsp != 0u) {
         s.gsp -= S / 2;
 #pragma unroll
         for (uint32_t k = 0; k < S / 2; ++k) s.lds[k * LANES] = s.spill.get(s.gsp + k);
         s.sp = S / 2;
     }
-    --s.sp;
-    return s.lds[s.sp * LANES];
 }
 
-/*
- * Traverses TLAS then BLASes depth-first in the reference's order. Returns a traversal status
- * (BF_HIT_MISS = no error). The stack must be empty on entry and is empty on a normal return.
- * `world(o, d)` re-reads the world-space ray when a BLAS is left, so that no copy of it stays
- * live through the loop. The winning candidate keeps (t, ids, leaf); its barycentrics are
- * re-derived by closest_hit_barycentrics from the same deterministic triangle test.
- */
-/* The world-space ray of a traversal, re-read through its functor when a BLAS is left. A functor
- * type may provide its own overload (found by argument-dependent lookup) that keeps the
- * reciprocals instead of recomputing them. */
-template <typename WorldRay>
-BF_D void world_space(const WorldRay& world, trav_space& s) {
-    v3f o, d;
-    world(o, d);
-    make_space(o, d, s);
+template <uint32_t S, uint32_t LANES, typename Spill>
+BF_D uint2 stack_pop(trav_stack<S, LANES, Spill>& s) {
+    stack_refill(s);
+    --s.sp;
+    return s.lds[s.sp * LANES];
 }
 
 /* Loop state of one ray's traversal between steps (the stack lives in trav_stack). */
@@ -529,7 +517,7 @@ struct trav_state {
 
 /* Starts a ray: empties the stack and pushes the TLAS root when the ray meets its box. On a normal
  * return an empty stack means the ray is already done. */
-template <bool COUNT, uint32_t S, uint32_t LANES, typename Spill>
+template <uint32_t S, uint32_t LANES, typename Spill>
 BF_D uint32_t traverse_begin(const bf_dev_scene& S_, const trav_ray& ray, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
                              trav_hit& best, bool& occluded, trav_counters& ctr) {
     best.present = false;
@@ -553,96 +541,112 @@ BF_D uint32_t traverse_begin(const bf_dev_scene& S_, const trav_ray& ray, trav_s
                              h, nv);
     if (st != BF_HIT_MISS) return st;
     if (!h) {
-        if (COUNT) ctr.nodes++;
+        ctr.nodes++;
         return BF_HIT_MISS;
     }
     stack_push(stack, nv.entry);
     return BF_HIT_MISS;
 }
 
-/* One step: pops one stack entry and processes it (a node's two child boxes, an instance entry,
- * or a triangle). Returns a traversal status (BF_HIT_MISS = no error); the ray is done when the
- * stack is empty. `world(o, d)` re-reads the world-space ray when a BLAS is left, so that no copy
- * of it stays live between steps. */
-template <bool ANY, bool COUNT, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
-BF_D uint32_t traverse_step(const bf_dev_scene& S_, WorldRay world, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
-                            trav_hit& best, bool& occluded, trav_counters& ctr) {
+/* True when the next entry is a leaf (a triangle or an instance) rather than an interior node; the
+ * stack holds entries and has been refilled. */
+template <uint32_t S, uint32_t LANES, typename Spill>
+BF_D bool leaf_on_top(const trav_stack<S, LANES, Spill>& stack) {
+    return (stack.lds[(stack.sp - 1u) * LANES].x & BF_WIDE_LEAF) != 0u;
+}
+
+/* A step is traverse_pop, then traverse_leaf or traverse_node of what it popped; the ray is done when
+ * the stack is empty. Pops one entry; false when the reference would skip it. `leave(space)` forms the
+ * world space again when a BLAS is left, so that no copy of it stays live between steps. */
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill, typename Leave>
+BF_D bool traverse_pop(const bf_dev_scene& S_, Leave leave, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
+                       const trav_hit& best, trav_counters& ctr, uint32_t& ref) {
     if (ts.in_blas && stack_depth(stack) <= ts.blas_base) {
         ts.in_blas = 0u;
-        world_space(world, ts.space); /* back in world space (recomputing is exact) */
+        leave(ts.space);
     }
     const uint2 entry = stack_pop(stack);
-    const uint32_t ref = entry.x & ~BF_NEAR_EXACT;
-    if (COUNT) ctr.nodes++;
+    ref = entry.x & ~BF_NEAR_EXACT;
+    ctr.nodes++;
     const float tcur = ANY ? ts.t_max : best.t;
     /* the reference's pop test: the entry's binary64 near value against the current t_max */
-    uint32_t visit = near_decision(entry, tcur);
-    if (visit == 2u) {
-        const uint32_t index = ref & BF_REF_MASK;
-        const float* box = (ref & BF_WIDE_LEAF) ? (ts.in_blas ? S_.blas_leaf_boxes : S_.tlas_leaf_boxes)
-                                                : (ts.in_blas ? S_.blas_node_boxes : S_.tlas_node_boxes);
-        visit = near_exact(box + 6 * (size_t)index, ts.space, ts.t_min) <= (double)tcur ? 1u : 0u;
-    }
-    if (visit == 0u) return BF_HIT_MISS;
-    if (ref & BF_WIDE_LEAF) {
-        const uint32_t leaf = ref & BF_REF_MASK;
-        if (!ts.in_blas) {
-            const bf_dev_tlas_leaf L = S_.tlas_leaves[leaf];
-            if ((ts.mask & L.visibility_mask) == 0u) return BF_HIT_MISS;
-            const v3f lo = xform_point(L.world_to_local, ts.space.o);
-            const v3f ld = xform_vector(L.world_to_local, ts.space.d);
-            if (!fin3(lo) || !fin3(ld) || (ld.x == 0.0f && ld.y == 0.0f && ld.z == 0.0f)) return BF_HIT_NUMERICAL_FAILURE;
-            if (COUNT) ctr.instances++;
-            const bf_dev_blas B = S_.blases[L.blas_index];
-            trav_space local;
-            make_space(lo, ld, local);
-            bool h;
-            child_near nv;
-            const uint32_t st = slab(B.root_box[0], B.root_box[1], B.root_box[2], B.root_box[3], B.root_box[4],
-                                     B.root_box[5], local, ts.t_min, tcur, B.root_ref, h, nv);
-            if (st != BF_HIT_MISS) return st;
-            if (!h) {
-                if (COUNT) ctr.nodes++;
-                return BF_HIT_MISS;
-            }
-            /* the BLAS root opens the BLAS part of the stack (a fresh stack in the reference) */
-            if (stack_depth(stack) + 1u > stack.cap) return BF_HIT_STACK_OVERFLOW;
-            ts.inst_id = L.instance_id;
-            ts.scene_inst = L.scene_instance;
-            ts.in_blas = 1u;
-            ts.blas_base = stack_depth(stack);
-            ts.space = local;
-            stack_push(stack, nv.entry);
-            return BF_HIT_MISS;
-        }
-        const float4 q0 = S_.leaf_triangles[3 * (size_t)leaf + 0];
-        const float4 q1 = S_.leaf_triangles[3 * (size_t)leaf + 1];
-        const float4 q2 = S_.leaf_triangles[3 * (size_t)leaf + 2];
-        const uint32_t prim = __float_as_uint(q0.w);
-        if (COUNT) ctr.triangles++;
-        tri_result tr;
-        tr.hit = false;
-        trav_shear sh;
-        make_shear(ts.space.d, sh);
-        const uint32_t st = watertight<false>(mk(q0.x, q0.y, q0.z), mk(q1.x, q1.y, q1.z), mk(q2.x, q2.y, q2.z), ts.space.o,
-                                              ts.space.d, sh, ts.t_min, tcur, tr);
+    const uint32_t visit = near_decision(entry, tcur);
+    if (visit != 2u) return visit != 0u;
+    const uint32_t index = ref & BF_REF_MASK;
+    const float* box = (ref & BF_WIDE_LEAF) ? (ts.in_blas ? S_.blas_leaf_boxes : S_.tlas_leaf_boxes)
+                                            : (ts.in_blas ? S_.blas_node_boxes : S_.tlas_node_boxes);
+    return near_exact(box + 6 * (size_t)index, ts.space, ts.t_min) <= (double)tcur;
+}
+
+/* A popped instance entry or triangle. Returns a traversal status (BF_HIT_MISS = no error). */
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill>
+BF_D uint32_t traverse_leaf(const bf_dev_scene& S_, uint32_t ref, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
+                            trav_hit& best, bool& occluded, trav_counters& ctr) {
+    const float tcur = ANY ? ts.t_max : best.t;
+    const uint32_t leaf = ref & BF_REF_MASK;
+    if (!ts.in_blas) {
+        const bf_dev_tlas_leaf L = S_.tlas_leaves[leaf];
+        if ((ts.mask & L.visibility_mask) == 0u) return BF_HIT_MISS;
+        const v3f lo = xform_point(L.world_to_local, ts.space.o);
+        const v3f ld = xform_vector(L.world_to_local, ts.space.d);
+        if (!fin3(lo) || !fin3(ld) || (ld.x == 0.0f && ld.y == 0.0f && ld.z == 0.0f)) return BF_HIT_NUMERICAL_FAILURE;
+        ctr.instances++;
+        const bf_dev_blas B = S_.blases[L.blas_index];
+        trav_space local;
+        make_space(lo, ld, local);
+        bool h;
+        child_near nv;
+        const uint32_t st = slab(B.root_box[0], B.root_box[1], B.root_box[2], B.root_box[3], B.root_box[4],
+                                 B.root_box[5], local, ts.t_min, tcur, B.root_ref, h, nv);
         if (st != BF_HIT_MISS) return st;
-        if (!tr.hit) return BF_HIT_MISS;
-        if (ANY) {
-            occluded = true;
-            stack.sp = 0;
-            stack.gsp = 0;
+        if (!h) {
+            ctr.nodes++;
             return BF_HIT_MISS;
         }
-        if (!precedes(tr.t, ts.inst_id, prim, best)) return BF_HIT_MISS;
-        best.present = true;
-        best.t = tr.t;
-        best.instance_id = ts.inst_id;
-        best.primitive = prim;
-        best.scene_instance = ts.scene_inst;
-        best.leaf = leaf;
+        /* the BLAS root opens the BLAS part of the stack (a fresh stack in the reference) */
+        if (stack_depth(stack) + 1u > stack.cap) return BF_HIT_STACK_OVERFLOW;
+        ts.inst_id = L.instance_id;
+        ts.scene_inst = L.scene_instance;
+        ts.in_blas = 1u;
+        ts.blas_base = stack_depth(stack);
+        ts.space = local;
+        stack_push(stack, nv.entry);
         return BF_HIT_MISS;
     }
+    const float4 q0 = S_.leaf_triangles[3 * (size_t)leaf + 0];
+    const float4 q1 = S_.leaf_triangles[3 * (size_t)leaf + 1];
+    const float4 q2 = S_.leaf_triangles[3 * (size_t)leaf + 2];
+    const uint32_t prim = __float_as_uint(q0.w);
+    ctr.triangles++;
+    tri_result tr;
+    tr.hit = false;
+    trav_shear sh;
+    make_shear(ts.space.d, sh);
+    const uint32_t st = watertight<false>(mk(q0.x, q0.y, q0.z), mk(q1.x, q1.y, q1.z), mk(q2.x, q2.y, q2.z), ts.space.o,
+                                          ts.space.d, sh, ts.t_min, tcur, tr);
+    if (st != BF_HIT_MISS) return st;
+    if (!tr.hit) return BF_HIT_MISS;
+    if (ANY) {
+        occluded = true;
+        stack.sp = 0;
+        stack.gsp = 0;
+        return BF_HIT_MISS;
+    }
+    if (!precedes(tr.t, ts.inst_id, prim, best)) return BF_HIT_MISS;
+    best.present = true;
+    best.t = tr.t;
+    best.instance_id = ts.inst_id;
+    best.primitive = prim;
+    best.scene_instance = ts.scene_inst;
+    best.leaf = leaf;
+    return BF_HIT_MISS;
+}
+
+/* The two child boxes of a popped interior node. */
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill>
+BF_D uint32_t traverse_node(const bf_dev_scene& S_, uint32_t ref, trav_stack<S, LANES, Spill>& stack, trav_state& ts,
+                            const trav_hit& best) {
+    const float tcur = ANY ? ts.t_max : best.t;
     const bf_wide_node* nodes = ts.in_blas ? S_.blas_nodes : S_.tlas_nodes;
     const bf_wide_node N = nodes[ref];
     bool h0, h1;
@@ -688,12 +692,17 @@ BF_D uint32_t traverse_step(const bf_dev_scene& S_, WorldRay world, trav_stack<S
  * The winning candidate keeps (t, ids, leaf); its barycentrics are re-derived by
  * closest_hit_barycentrics from the same deterministic triangle test.
  */
-template <bool ANY, bool COUNT, uint32_t S, uint32_t LANES, typename Spill, typename WorldRay>
-BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, WorldRay world, trav_stack<S, LANES, Spill>& stack, trav_hit& best,
+template <bool ANY, uint32_t S, uint32_t LANES, typename Spill, typename Leave>
+BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, Leave leave, trav_stack<S, LANES, Spill>& stack, trav_hit& best,
                        bool& occluded, trav_counters& ctr) {
     trav_state ts;
-    uint32_t st = traverse_begin<COUNT>(S_, ray, stack, ts, best, occluded, ctr);
-    while (st == BF_HIT_MISS && stack_depth(stack) != 0u) st = traverse_step<ANY, COUNT>(S_, world, stack, ts, best, occluded, ctr);
+    uint32_t st = traverse_begin(S_, ray, stack, ts, best, occluded, ctr);
+    while (st == BF_HIT_MISS && stack_depth(stack) != 0u) {
+        uint32_t ref;
+        if (!traverse_pop<ANY>(S_, leave, stack, ts, best, ctr, ref)) continue;
+        st = (ref & BF_WIDE_LEAF) ? traverse_leaf<ANY>(S_, ref, stack, ts, best, occluded, ctr)
+                                  : traverse_node<ANY>(S_, ref, stack, ts, best);
+    }
     return st;
 }
 
