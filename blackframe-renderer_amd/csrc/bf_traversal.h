@@ -730,7 +730,8 @@ BF_D uint32_t traverse(const bf_dev_scene& S_, const trav_ray& ray, Leave leave,
  * RN(1 / d) = +-inf: its near and far quotients are -inf and +inf inside the slab, (+inf, +inf) or
  * (-inf, -inf) outside, NaN on a plane, which fmaxf / fminf ignore. A space whose numbers leave
  * the range of this analysis (subnormal or huge direction components, origins past 2^126) gets NaN
- * reciprocals: every box is then entered and every order decided in binary64.
+ * reciprocals that keep the direction's signs: every box is then entered, near planes are still told
+ * from far ones, and every order of siblings whose near planes differ is decided in binary64.
  *
  * The launchers use this engine where the boxes' coordinates stay within 2^126, no stack can
  * overflow the reference's 64 entries (both checked when the scene is built) and t_min >= 0;
@@ -791,16 +792,22 @@ struct ring_stack {
     }
 };
 
-/* Binary32 reciprocals of a direction, or NaN where the bounds do not hold. */
+/* Binary32 reciprocals of a direction, or NaN with the direction's signs where the bounds do not hold. */
 BF_D v3f bound_reciprocals(v3f o, v3f d) {
     const float m = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
     const float c = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
     const bool tiny = (fabsf(d.x) < 0x1p-126f && d.x != 0.0f) || (fabsf(d.y) < 0x1p-126f && d.y != 0.0f) ||
                       (fabsf(d.z) < 0x1p-126f && d.z != 0.0f);
     v3f inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    if (tiny || !(m <= 0x1p126f) || !(c <= 0x1p126f)) inv.x = inv.y = inv.z = __builtin_nanf("");
+    if (tiny || !(m <= 0x1p126f) || !(c <= 0x1p126f)) {
+        const float nan = __builtin_nanf("");
+        inv = mk(copysignf(nan, d.x), copysignf(nan, d.y), copysignf(nan, d.z));
+    }
     return inv;
 }
+
+/* True when an axis's near plane is its upper one: by the sign bit, which NaN reciprocals have too. */
+BF_D bool descending(float inv) { return __float_as_int(inv) < 0; }
 
 /* The binary64 verdict on a box against [t_min, t]: the reference's push and pop tests together. */
 BF_D bool box_visited_exact(v3f lo, v3f hi, v3f o, v3f d, float t_min, float t) {
@@ -922,7 +929,7 @@ BF_D void bound_node(WorldRay world, Stack& stack, bound_state& ts) {
     const float4* p = reinterpret_cast<const float4*>(ts.nodes + ts.cur);
     const float4 a = p[0], b = p[1], c = p[2];
     const uint2 child = *reinterpret_cast<const uint2*>(p + 3);
-    const bool sx = ts.inv.x < 0.0f, sy = ts.inv.y < 0.0f, sz = ts.inv.z < 0.0f;
+    const bool sx = descending(ts.inv.x), sy = descending(ts.inv.y), sz = descending(ts.inv.z);
     /* a: lo_x lo_y, b: lo_z hi_x, c: hi_y hi_z, each for both children */
     const v3f n0 = mk(sx ? b.z : a.x, sy ? c.x : a.z, sz ? c.z : b.x);
     const v3f n1 = mk(sx ? b.w : a.y, sy ? c.y : a.w, sz ? c.w : b.y);
@@ -944,11 +951,10 @@ BF_D void bound_node(WorldRay world, Stack& stack, bound_state& ts) {
     const float lead = nv1 - nv0;
     bool first = both ? lead > 0.0f : h0;
     if (both && !(fabsf(lead) > fmaf(nv0 + nv1, BF_SLAB_REL, 4.0f * BF_SLAB_ABS))) {
-        /* a tie when each axis has equal near planes or lies below both near values; NaN reciprocals
-         * tell nothing of the direction's signs, so the near planes are not known here */
+        /* a tie when each axis has equal near planes or lies below both near values */
         const float below = fmaf(fminf(nv0, nv1), 1.0f - 2.0f * BF_SLAB_REL, -4.0f * BF_SLAB_ABS);
         const float up = 1.0f + BF_SLAB_REL;
-        const bool tie = !bf_isnan(ts.inv.x) && (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
+        const bool tie = (n0.x == n1.x || fmaxf(q0.x, q1.x) * up < below) &&
                          (n0.y == n1.y || fmaxf(q0.y, q1.y) * up < below) &&
                          (n0.z == n1.z || fmaxf(q0.z, q1.z) * up < below);
         first = true;
@@ -958,11 +964,7 @@ BF_D void bound_node(WorldRay world, Stack& stack, bound_state& ts) {
             if (ts.tleaf == BF_INVALID_INDEX) world(d, mask);
             trav_space s;
             make_space(ts.o, d, s);
-            /* the near planes by the direction's own signs (the reciprocals may be NaN) */
-            const bool ex = (d.x < 0.0f) != sx, ey = (d.y < 0.0f) != sy, ez = (d.z < 0.0f) != sz;
-            const v3f m0 = mk(ex ? f0.x : n0.x, ey ? f0.y : n0.y, ez ? f0.z : n0.z);
-            const v3f m1 = mk(ex ? f1.x : n1.x, ey ? f1.y : n1.y, ez ? f1.z : n1.z);
-            first = (float)child_near_exact(m0, s, ts.t_min) <= (float)child_near_exact(m1, s, ts.t_min);
+            first = (float)child_near_exact(n0, s, ts.t_min) <= (float)child_near_exact(n1, s, ts.t_min);
         }
     }
     if (both) push_ref(stack, first ? child.y : child.x, first ? lo1 : lo0);
