@@ -533,7 +533,9 @@ __global__ __launch_bounds__(BF_API_BLOCK) void k_scene_counting(bf_dev_scene S,
         out.status = st != BF_HIT_MISS ? st : (occluded ? BF_OCCLUDED : BF_VISIBLE);
         ((bf_occlusion_result*)results)[i] = out;
     } else {
-        closest_record(S, ray, st, best, ((bf_closest_hit_result*)results)[i]);
+        bf_closest_hit_result out;
+        closest_record(S, ray, st, best, out);
+        ((bf_closest_hit_result*)results)[i] = out;
     }
     if (counters) {
         counters[3 * (size_t)i] = ctr.nodes;
