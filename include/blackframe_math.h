@@ -57,8 +57,9 @@ BF_HD double bf_bits_double(uint64_t bits) {
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)
-/* gfx950 classifies and takes floats apart in one instruction each (the values of the bit forms
- * below for every float; ldexp rounds once, to nearest even, as a correctly rounded one must) */
+/* gfx950 classifies and takes floats apart in one instruction each: the values of the bit forms below
+ * for every float, a NaN's payload aside; ldexp rounds once, to nearest even, as a correctly rounded
+ * one must */
 BF_HD bool bf_isnan(float v) { return __builtin_isnan(v); }
 BF_HD bool bf_isfinite(float v) { return __builtin_isfinite(v); }
 #else
