@@ -22,7 +22,7 @@
  * structure, BF_STACK_DEPTH entries in all. */
 #define BF_STRUCTURE_STACK 64u
 #define BF_STACK_DEPTH 128u  /* traversal stack entries per lane (TLAS + BLAS) */
-#define BF_API_STACK 64u     /* LDS entries per lane of the stand-alone traversal launchers (no spill) */
+#define BF_API_STACK 64u     /* LDS entries per lane of the counting stand-alone queries (no spill) */
 #define BF_API_BLOCK 64u     /* lanes per workgroup of the stand-alone traversal launchers */
 /* A traversal stack entry is (reference, near word). Reference bits: 31 BF_WIDE_LEAF, 30
  * BF_NEAR_EXACT (the near word is the binary64 near value rounded up to binary32; otherwise it
@@ -35,7 +35,6 @@
 #ifndef BF_SHADOW_STACK
 #define BF_SHADOW_STACK 16u /* the same for any-hit walks, whose entries are half the size */
 #endif
-#define BF_TRACE_BLOCK 128u  /* lanes per traversal workgroup */
 #ifndef BF_TRACE_WAVES_PER_SIMD
 #define BF_TRACE_WAVES_PER_SIMD 6 /* register budget of the closest-hit traversal (waves per SIMD) */
 #endif

@@ -12,9 +12,9 @@
 #include "bf_traversal.h"
 
 /* ---- closest-hit stage: gather + traversal + classify + miss ---------------------------------- */
-/* The traversal kernels are persistent: a grid sized to the device's resident capacity, each wave
- * taking 64 consecutive queue items at a time with a static stride, so that the per-lane stack
- * spill area is bounded by the grid and empty tail workgroups cost nothing. */
+/* The traversal kernels are persistent: a grid sized to the device's resident capacity, whose waves claim
+ * queue items until none is left (shared_claim), so that the per-lane stack spill area is bounded by the
+ * grid and empty tail workgroups cost nothing. */
 
 /* One lane's ray of a counting launch between traversal steps. */
 struct lane_ray {

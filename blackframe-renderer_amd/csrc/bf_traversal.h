@@ -1,7 +1,10 @@
 /*
- * BVH2 closest-hit and any-hit traversal over 64-byte wide nodes with a per-lane LDS stack.
+ * BVH2 closest-hit and any-hit traversal over 64-byte wide nodes with a per-lane LDS stack: two walks with
+ * the same results, and the triangle tests and stacks that they share.
  *
- * Decisions are bit-identical to the reference traversal (CudaSceneClosestHit.cu:407-1186):
+ * The step-exact walk (traverse_begin / _pop / _leaf / _node) takes every step of the reference's
+ * (CudaSceneClosestHit.cu:407-1186), for launches that count steps and for scenes and cameras outside
+ * the other walk's range:
  *  - the slab test is the binary64 quotient widened by one ulp (:407-455);
  *  - children are pushed far-then-near with the first (lower canonical index) child winning ties
  *    (:466-512); the first child of an internal node always has the lower pre-order index;
@@ -14,6 +17,9 @@
  * structure; here TLAS and BLAS share one stack of BF_STACK_DEPTH entries, each part held to the
  * reference's 64, so a lane reports stack overflow exactly where the reference's would. Slab quotients are formed from a per-ray
  * binary64 reciprocal with one correction step, which yields the correctly rounded quotient.
+ *
+ * The bound walk (bound_begin / _pop / _leaf / _node), which every other launch takes, is described
+ * where it begins, under "traversal on binary32 bounds".
  */
 #ifndef BF_TRAVERSAL_H
 #define BF_TRAVERSAL_H
@@ -435,12 +441,6 @@ BF_D bool precedes(float t, uint32_t inst, uint32_t prim, const trav_hit& c) {
     return !c.present || t < c.t || (t == c.t && (inst < c.instance_id || (inst == c.instance_id && prim < c.primitive)));
 }
 
-/*
- * Per-lane traversal stack of (node reference, near bits) pairs. The top S entries live in LDS,
- * laid out [entry][lane] so that a wave's pushes and pops touch consecutive banks; when a push
- * finds them full, the lower half moves to the lane's column of a global spill area and comes
- * back when the LDS part runs empty. With S = BF_STACK_DEPTH nothing ever spills.
- */
 /* A lane's column of a global spill area. */
 struct column_spill {
     uint2* area;
@@ -464,6 +464,12 @@ struct scratch_spill {
     BF_D void get(uint32_t k, uint32_t& e) const { e = ref[k]; }
 };
 
+/*
+ * The step-exact walk's stack of (node reference, near bits) pairs. The top S entries live in LDS,
+ * laid out [entry][lane] so that a wave's pushes and pops touch consecutive banks; when a push
+ * finds them full, the lower half moves to the lane's spill area and comes back when the LDS part
+ * runs empty (stack_refill). A lane whose cap is S never spills.
+ */
 template <uint32_t S, uint32_t LANES, typename Spill = column_spill>
 struct trav_stack {
     uint2* lds;             /* entry k at lds[k * LANES] (LANES = lanes of the workgroup) */
