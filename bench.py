@@ -9,11 +9,14 @@ per-object Lambert / GGX conductor / GGX dielectric materials, 64 emissive trian
 constant environment, 1920x1080 at 64 spp, 4 wavelengths per path, max depth 16, power MIS.
 
 Printed: one JSON line. `value` is Mrays/s = (closest-hit + shadow queries) / frame time.
-`roofline` prices the dominant kernel (closest-hit traversal) by its algorithmic bytes: per ray
+`roofline.achieved` prices the dominant kernel (closest-hit traversal) by its algorithmic bytes: per ray
 48 B ray + 80 B result + 64 B per BVH node visited + 48 B per triangle tested + 48 B per instance
-entered, counted by the traversal counters of an untimed warmup frame, divided by the kernel's
-summed HIP-event duration over the timed frames (events recorded on the launch stream by the
-library's stage instrumentation). `cpu_baseline` times the CPU wavefront restatement (the oracle,
+entered by the reference's walk, counted by the step-exact kernel in an untimed warmup frame, divided by
+the kernel's summed HIP-event duration over the timed frames (events recorded on the launch stream by the
+library's stage instrumentation). The timed kernel takes another walk, with the same results, and finds
+most of its nodes in L2: this rate compares renderers and is no share of the memory's. `roofline.hbm_gbs`
+is what the kernel moves to and from memory (profiled bytes over the time measured here), and `bound` what
+holds it back. `cpu_baseline` times the CPU wavefront restatement (the oracle,
 threaded with contiguous partitions) on a bounded band of the same frame on this host.
 """
 import argparse
@@ -676,12 +679,15 @@ def main():
                    "first_failure": [report.first_failure_slot, report.first_failure_code] if report.failed_paths else None},
         "paths_per_s": round(path_count * args.steps / elapsed, 1),
         "roofline": {
-            "bound": "hbm",
+            "bound": "vector issue",
             "kernel": "k_trace<closest hit>",
             "achieved": round(achieved, 2),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 5),
+            "basis": "bytes of the reference's walk over this kernel's time",
+            "hbm_gbs": round(traffic / closest_avg_s / 1e9, 2) if traffic else None,
+            "hbm_frac": round(traffic / closest_avg_s / 1e9 / HBM_PEAK_GBS, 5) if traffic else None,
             "traffic": traffic,
             "traffic_source": TRAFFIC_SUMMARY.name if traffic else None,
             "algorithmic_bytes_per_launch": round(closest_bytes / closest_launches),
