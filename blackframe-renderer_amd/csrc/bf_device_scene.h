@@ -89,9 +89,11 @@
  * single-closure kernels keep nearly everything in registers (the shade stage of a 1920x1080x64 frame
  * of 1024 instances 65.2 ms, against 75.0 with 3 waves, 83.1 with 4 and 107 with 5; of a 256x256x16
  * frame with maps 8.9 ms, against 16.8 with 3 and 21.2 with 4). The general kernel does too without
- * texture gradients or texture-weighted mixtures (with maps 8.9 ms against 18.7 with 3 waves; a 640x360x16
- * frame 5.6 against 6.0); with those its closures, indexed in scratch, keep it waiting whatever its
- * budget, and the third wave gains (9.1 to 8.8 ms in an adjoint replay, 5.1 to 4.8 in its forward pass). */
+ * texture gradients or texture-weighted mixtures: 640x360x16 frames of seven boxes take 3.73 ms with
+ * mirrors, 4.18 with rough diffuse and 8.82 with two-closure materials, against 3.99, 4.85 and 9.56 with 3
+ * waves; with a normal map, 320x180x16, 4.00, 3.97 and 8.10 against 6.57, 6.41 and 12.25. With those its
+ * closures, indexed in scratch, keep it waiting whatever its budget, and the third wave gains (9.1 to 8.8
+ * ms in an adjoint replay, 5.1 to 4.8 in its forward pass). */
 #define BF_SHADE_WAVES_PER_SIMD(mode) ((mode) == 0u || (mode) == 3u ? 2 : 3) /* any material, by mode */
 #ifndef BF_SHADE_SINGLE_WAVES
 #define BF_SHADE_SINGLE_WAVES 2 /* materials of one closure */
